@@ -10,6 +10,8 @@
 #include "jas_leaf.hpp"
 
 #include <cfloat>
+#include <limits>
+#include <type_traits>
 
 namespace jas {
 
@@ -431,8 +433,10 @@ __global__ void __launch_bounds__(256) gsm_write_kernel(const float *__restrict_
 }
 
 // ---------------- generic reductions over a leaf (mat_express_t.hpp:511-628) ----------------
-// Per-row and per-column forms use one thread per output and accumulate sequentially in
-// the output type, exactly the order jasmine's loops use (hsum :548-564, vsum :530-546).
+// Every form accumulates one line sequentially in the output type, exactly the order
+// jasmine's loops use (hsum :548-564, vsum :530-546): a line is a dependent chain of `len`
+// additions, and what is left to the kernel is to keep enough of
+// the matrix in flight behind the chains.
 template <typename T>
 __device__ __forceinline__ T leaf_get(const LeafDev &L, int i, int j)
 {
@@ -440,34 +444,240 @@ __device__ __forceinline__ T leaf_get(const LeafDev &L, int i, int j)
 }
 
 template <typename T>
+__device__ __forceinline__ T reduce_step(T acc, T v, int op)
+{
+    return op == 1 ? (v > acc ? v : acc) : acc + v;
+}
+template <typename T>
+__device__ __forceinline__ T reduce_first(int op)
+{
+    return op == 1 ? -std::numeric_limits<T>::max() : (T)0;
+}
+
+// any leaf (modulo broadcasts, transposed column-major views, mixed types): one thread per line
+template <typename T>
 __global__ void reduce_line_kernel(LeafDev L, int rows, int cols, int op, int axis, T *out)
 {
     int o = blockIdx.x * blockDim.x + threadIdx.x;
     int n_out = axis == 0 ? rows : cols;
     if (o >= n_out) return;
     int len = axis == 0 ? cols : rows;
-    T acc = op == 1 ? -std::numeric_limits<T>::max() : (T)0;
-    for (int k = 0; k < len; ++k) {
-        T v = axis == 0 ? leaf_get<T>(L, o, k) : leaf_get<T>(L, k, o);
-        if (op == 1) acc = v > acc ? v : acc;
-        else acc += v;
-    }
+    T acc = reduce_first<T>(op);
+    for (int k = 0; k < len; ++k) acc = reduce_step(acc, axis == 0 ? leaf_get<T>(L, o, k) : leaf_get<T>(L, k, o), op);
     if (op == 2) acc = acc / (T)len;  // vmean / hmean: ele / int (mat_express_t.hpp:566-578)
     out[o] = acc;
 }
 
-// whole-matrix: per-row sequential partials, then a sequential pass over the partials
-template <typename T>
-__global__ void reduce_all_kernel(const T *rowpart, int rows, int cols, int op, T *out)
+// stored element -> accumulator type
+__device__ __forceinline__ float reduce_value(float v) { return v; }
+__device__ __forceinline__ double reduce_value(double v) { return v; }
+__device__ __forceinline__ float reduce_value(uint16_t v) { return bf16_to_f32(v); }
+
+// The chain of one line over n staged chunks at row[0], row[stride], ...: two sets of 32
+// elements, one read from LDS while the other is added, so the read latency hides behind the
+// additions (about 8 cycles each, the dependent-add latency: 8192 elements in 28 us).
+template <bool MAX, int E, typename S, typename T, typename chunk_t>
+__device__ __forceinline__ T reduce_chain(const chunk_t *row, int stride, int n, T acc)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    T acc = op == 1 ? -std::numeric_limits<T>::max() : (T)0;
-    for (int r = 0; r < rows; ++r) {
-        if (op == 1) acc = rowpart[r] > acc ? rowpart[r] : acc;
-        else acc += rowpart[r];
+    constexpr int P = 32 / E;
+    chunk_t a[P], b[P];
+    auto read = [&](chunk_t (&v)[P], int c) {
+#pragma unroll
+        for (int k = 0; k < P; ++k) v[k] = row[(c + k) * stride];
+    };
+    auto step = [&](const chunk_t &v) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            S x;
+            if constexpr (E == 1) x = v;
+            else x = v[e];
+            acc = reduce_step(acc, (T)reduce_value(x), MAX ? 1 : 0);
+        }
+    };
+    int c = 0;
+    if (n >= 2 * P) {
+        read(a, 0);
+        for (; c + 2 * P <= n; c += 2 * P) {
+            read(b, c + P);
+#pragma unroll
+            for (int k = 0; k < P; ++k) step(a[k]);
+            read(a, c + 3 * P <= n ? c + 2 * P : 0);  // (past the last whole set: unused)
+#pragma unroll
+            for (int k = 0; k < P; ++k) step(b[k]);
+        }
     }
-    if (op == 2) acc = acc / (T)((long)rows * cols);  // mean (mat_express_t.hpp:580-585)
-    out[0] = acc;
+    for (; c < n; ++c) step(row[c * stride]);
+    return acc;
+}
+
+// Contiguous lines: element k of line i at x[i * ls + k].  One wave per G lines: all 64
+// lanes load the lines' next 16 KB (1 KB contiguous per instruction) into registers while
+// lanes 0..G-1 add up the previous 16 KB, one line each, from LDS.  In-flight bytes per wave
+// do not depend on G and the issue cost of the chains falls with it (launch_rows).  Loads of 4 bytes (VEC
+// false) serve lines that are not 16-byte aligned.  8192 x 8192 fp32 row sums on MI355X: 70
+// us (3.8 TB/s; one thread per line took 2.0 ms).
+template <typename S, typename T, int G, bool VEC>
+__global__ void __launch_bounds__(64)
+reduce_rows_kernel(const S *__restrict__ x, long ls, int lines, int len, int op, T div, T *__restrict__ out)
+{
+    constexpr int E = VEC ? 16 / (int)sizeof(S) : 1;  // elements per load
+    constexpr int U = VEC ? 16 : 64;                  // loads per lane and stage
+    constexpr int CPL = 64 * U / G;                   // loads per line and stage
+    typedef typename std::conditional<VEC, S __attribute__((ext_vector_type(16 / sizeof(S)))), S>::type chunk_t;
+    // one chunk of padding per line: lanes reading the same column of their lines hit
+    // different banks
+    __shared__ chunk_t st[G * (CPL + 1)];
+    const int lane = threadIdx.x, i0 = blockIdx.x * G;
+    const S *xb = x + (long)i0 * ls;
+    const int nl = min(G, lines - i0);
+    chunk_t r[U];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // past the last line or its end: a clamped element, which no chain reads (a
+            // predicate would put a branch around every load)
+            const int q = u * 64 + lane, li = min(q / CPL, nl - 1), c = min(c0 + (q % CPL) * E, len - E);
+            r[u] = *(const chunk_t *)(xb + (long)li * ls + c);
+        }
+    };
+    T acc = reduce_first<T>(op);
+    load(0);
+    for (int c0 = 0; c0 < len; c0 += CPL * E) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int q = u * 64 + lane;
+            st[q + q / CPL] = r[u];
+        }
+        __syncthreads();
+        if (c0 + CPL * E < len) load(c0 + CPL * E);
+        if (lane < nl) {
+            const int n = min(CPL, (len - c0) / E);  // len % E == 0
+            const chunk_t *row = st + lane * (CPL + 1);
+            acc = op == 1 ? reduce_chain<true, E, S, T>(row, 1, n, acc) : reduce_chain<false, E, S, T>(row, 1, n, acc);
+        }
+    }
+    if (lane < nl) out[i0 + lane] = op == 2 ? acc / div : acc;
+}
+
+// Lines across memory rows: element k of line i at x[k * es + i], adjacent lines adjacent.
+// One wave per CW lines (128, 64 or 32 bytes of every memory row): the lanes load the next
+// 32 KB (VEC: 16 bytes per lane) while lanes 0..CW-1 add up the previous stage from LDS.
+// 8192 x 8192 fp32 column means on MI355X: 78 us (3.4 TB/s; one thread per line took 2.0 ms).
+template <typename S, typename T, int CW, bool VEC>
+__global__ void __launch_bounds__(64)
+reduce_cols_kernel(const S *__restrict__ x, long es, int lines, int len, int op, T div, T *__restrict__ out)
+{
+    constexpr int E = VEC ? 16 / (int)sizeof(S) : 1;
+    constexpr int U = VEC ? 32 : 64;
+    constexpr int CPR = CW / E, RS = 64 * U / CPR;  // loads per memory row, rows per stage
+    typedef typename std::conditional<VEC, S __attribute__((ext_vector_type(16 / sizeof(S)))), S>::type chunk_t;
+    __shared__ __attribute__((aligned(16))) S st[RS * CW];
+    const int lane = threadIdx.x, i0 = blockIdx.x * CW;
+    const int nl = min(CW, lines - i0);
+    const int ci = min((lane % CPR) * E, nl - E), rr = lane / CPR;  // CPR divides 64
+    const S *xb = x + i0 + ci;
+    chunk_t r[U];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(k0 + u * (64 / CPR) + rr, len - 1);  // clamped: no chain reads it
+            r[u] = *(const chunk_t *)(xb + (long)k * es);
+        }
+    };
+    T acc = reduce_first<T>(op);
+    load(0);
+    for (int k0 = 0; k0 < len; k0 += RS) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u) *(chunk_t *)(st + (u * 64 + lane) * E) = r[u];
+        __syncthreads();
+        if (k0 + RS < len) load(k0 + RS);
+        if (lane < nl) {
+            const int n = min(RS, len - k0);
+            acc = op == 1 ? reduce_chain<true, 1, S, T>(st + lane, CW, n, acc) : reduce_chain<false, 1, S, T>(st + lane, CW, n, acc);
+        }
+    }
+    if (lane < nl) out[i0 + lane] = op == 2 ? acc / div : acc;
+}
+
+// lines at x + i * ls + k (contiguous lines)
+template <typename S, typename T>
+static void launch_rows(const S *x, long ls, int lines, int len, int op, T div, T *out, hipStream_t s)
+{
+    const bool vec = (uintptr_t)x % 16 == 0 && (ls * sizeof(S)) % 16 == 0 && (len * sizeof(S)) % 16 == 0;
+#define JAS_RR(GV)                                                                                                   \
+    {                                                                                                                \
+        if (vec)                                                                                                     \
+            hipLaunchKernelGGL((reduce_rows_kernel<S, T, GV, true>), dim3(ceil_div(lines, GV)), dim3(64), 0, s, x, ls, \
+                               lines, len, op, div, out);                                                            \
+        else                                                                                                         \
+            hipLaunchKernelGGL((reduce_rows_kernel<S, T, GV, false>), dim3(ceil_div(lines, GV)), dim3(64), 0, s, x, ls, \
+                               lines, len, op, div, out);                                                            \
+    }
+    // 8192 lines of 8192: 70 us per call with 16 lines per wave, 84 with 8, 120 with 4; 2048 of
+    // 2048: 84 / 78 / 84 us for four calls; fewer lines than that need the waves
+    if (lines >= 4096) JAS_RR(16)
+    else if (lines >= 1024) JAS_RR(8)
+    else if (lines >= 256) JAS_RR(4)
+    else JAS_RR(1)
+#undef JAS_RR
+}
+
+// lines at x + i + k * es (adjacent lines)
+template <typename S, typename T>
+static void launch_cols(const S *x, long es, int lines, int len, int op, T div, T *out, hipStream_t s)
+{
+    const bool vec = (uintptr_t)x % 16 == 0 && (es * sizeof(S)) % 16 == 0 && (lines * sizeof(S)) % 16 == 0;
+#define JAS_RC(BYTES)                                                                                                \
+    {                                                                                                                \
+        constexpr int CWV = BYTES / (int)sizeof(S);                                                                  \
+        if (vec)                                                                                                     \
+            hipLaunchKernelGGL((reduce_cols_kernel<S, T, CWV, true>), dim3(ceil_div(lines, CWV)), dim3(64), 0, s, x, es, \
+                               lines, len, op, div, out);                                                            \
+        else                                                                                                         \
+            hipLaunchKernelGGL((reduce_cols_kernel<S, T, CWV, false>), dim3(ceil_div(lines, CWV)), dim3(64), 0, s, x, es, \
+                               lines, len, op, div, out);                                                            \
+    }
+    // the widest piece of a memory row that still gives every CU a wave
+    if ((long)lines * sizeof(S) >= 256 * 128) JAS_RC(128)
+    else if ((long)lines * sizeof(S) >= 256 * 64) JAS_RC(64)
+    else JAS_RC(32)
+#undef JAS_RC
+}
+
+// The staged kernels for a leaf of element type S; false when its addressing does not fit
+// (modulo wraps, or neither dimension contiguous) or the lines are too short to stage (under
+// 64 elements a wave's stage would be mostly masked): the one-thread-per-line kernel's cases.
+template <typename S, typename T>
+static bool reduce_staged(const LeafDev &L, int rows, int cols, int axis, int op, T div, T *out, hipStream_t s)
+{
+    if (L.kind != LK_STRIDED) return false;
+    const int lines = axis == 0 ? rows : cols, len = axis == 0 ? cols : rows;
+    const long ls = axis == 0 ? L.rs : L.cs, es = axis == 0 ? L.cs : L.rs;  // line and element strides
+    if (len < 64) return false;
+    if (es == 1) launch_rows<S, T>((const S *)L.p, ls, lines, len, op, div, out, s);
+    else if (ls == 1) launch_cols<S, T>((const S *)L.p, es, lines, len, op, div, out, s);
+    else return false;
+    return true;
+}
+
+template <typename T>
+static jas_status reduce_lines(const LeafDev &L, int rows, int cols, int axis, int op, T *out, hipStream_t s)
+{
+    const T div = (T)(axis == 0 ? cols : rows);
+    bool done = false;
+    if constexpr (std::is_same_v<T, float>) {
+        if (L.dtype == JAS_F32) done = reduce_staged<float, float>(L, rows, cols, axis, op, div, out, s);
+        else if (L.dtype == JAS_BF16) done = reduce_staged<uint16_t, float>(L, rows, cols, axis, op, div, out, s);
+    } else {
+        if (L.dtype == JAS_F64) done = reduce_staged<double, double>(L, rows, cols, axis, op, div, out, s);
+    }
+    if (!done)
+        hipLaunchKernelGGL(reduce_line_kernel<T>, dim3(ceil_div(axis == 0 ? rows : cols, 128)), dim3(128), 0, s, L, rows,
+                           cols, op, axis, out);
+    JAS_LAUNCH_CHECK();
+    return JAS_OK;
 }
 
 template <typename T>
@@ -480,18 +690,14 @@ static jas_status reduce_t(const jas_leaf *in, int op, int axis, void *d_out, hi
         L.rs = cols;
         L.cs = 1;
     }
-    if (axis == 0 || axis == 1) {
-        int n_out = axis == 0 ? rows : cols;
-        hipLaunchKernelGGL(reduce_line_kernel<T>, dim3(ceil_div(n_out, 128)), dim3(128), 0, s, L, rows, cols, op,
-                           axis, (T *)d_out);
-        JAS_LAUNCH_CHECK();
-        return JAS_OK;
-    }
+    if (axis == 0 || axis == 1) return reduce_lines<T>(L, rows, cols, axis, op, (T *)d_out, s);
+    // whole matrix: per-row sequential partials, then the partials as one line
     T *part = (T *)workspace(sizeof(T) * (size_t)rows, s);
     JAS_CHECK(part, JAS_ERR_OOM, "jas_reduce: workspace allocation failed");
-    hipLaunchKernelGGL(reduce_line_kernel<T>, dim3(ceil_div(rows, 128)), dim3(128), 0, s, L, rows, cols,
-                       op == 2 ? 0 : op, 0, part);
-    hipLaunchKernelGGL(reduce_all_kernel<T>, dim3(1), dim3(64), 0, s, part, rows, cols, op, (T *)d_out);
+    const jas_status st = reduce_lines<T>(L, rows, cols, 0, op == 2 ? 0 : op, part, s);
+    if (st != JAS_OK) return st;
+    // mean: the sum over rows * cols (mat_express_t.hpp:580-585)
+    launch_rows<T, T>(part, rows, 1, rows, op, (T)((long)rows * cols), (T *)d_out, s);
     JAS_LAUNCH_CHECK();
     return JAS_OK;
 }

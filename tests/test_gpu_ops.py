@@ -239,6 +239,44 @@ def test_reductions_bitexact(jas):
         close(out.numpy()[0], g["sum_max_mean"][k], atol=1e-5, rtol=1e-5)
 
 
+# stage edges of the row form (16 KB over 16 / 8 / 4 / 1 lines per wave, from 4096 / 1024 /
+# 256 lines) and of the column form (128 / 64 / 32 bytes of a row per wave), odd widths
+# (4-byte loads), views with offsets and transposed ones, and short lines (under 64 elements)
+@pytest.mark.parametrize("rows,cols,dt,roff,coff,t", [
+    (4100, 260, "f4", 0, 0, 0), (4097, 255, "f4", 0, 0, 0), (1029, 516, "f4", 0, 0, 0), (257, 1028, "f4", 0, 0, 0),
+    (1030, 1027, "f4", 0, 0, 0), (70, 4100, "f4", 0, 0, 0), (3, 9001, "f4", 0, 0, 0), (1030, 8200, "f4", 0, 0, 0),
+    (300, 4100, "f4", 0, 4, 0), (300, 4101, "f4", 2, 3, 0), (515, 130, "f4", 0, 0, 1), (515, 132, "f4", 4, 0, 1),
+    (2050, 130, "f8", 0, 0, 0), (131, 2051, "f8", 1, 1, 0), (4104, 72, "f8", 0, 0, 1), (300, 2064, "bf", 0, 0, 0),
+    (300, 515, "bf", 0, 1, 0), (200, 40, "f4", 0, 0, 0), (40, 200, "f4", 0, 0, 0), (1, 70, "f4", 0, 0, 0), (70, 1, "f4", 0, 0, 0)])
+def test_reductions_staged_bitexact(jas, rows, cols, dt, roff, coff, t):
+    import ctypes as C
+    x = normal((rows, cols), 7, rows + cols).astype(np.float64 if dt == "f8" else np.float32)
+    x[rows // 2, cols // 3] = -np.inf  # max of a line with an infinity; sums stay finite elsewhere
+    if dt == "bf":
+        u = x.view(np.uint32) >> 16
+        dx, x = jas.to_device(u.astype(np.uint16)), (u << 16).view(np.float32)
+    else:
+        dx = jas.to_device(x)
+    # the logical view: the underlying (a, b) = (i + roff, j + coff), or (j + coff, i + roff) transposed
+    v = x[coff:, roff:].T if t else x[roff:, coff:]
+    lf = jas.leaf(dx, roff=roff, coff=coff, transposed=t, vrows=v.shape[0], vcols=v.shape[1])
+    acc = x.dtype
+    # a running sum / maximum in the accumulator type has jasmine's order: its last entry is the line's result
+    sums = [np.add.accumulate(v, axis=1 - a, dtype=acc).take(-1, 1 - a) for a in (0, 1)]
+    # a maximum starts from the type's lowest finite value (hmax, mat_express_t.hpp:619)
+    maxs = [np.maximum(v.max(axis=1 - a), np.finfo(acc).min) for a in (0, 1)]
+    total = np.add.accumulate(sums[0], dtype=acc)[-1]
+    for op in (0, 1, 2):
+        for axis in (0, 1, 2):
+            n = (v.shape[0], v.shape[1], 1)[axis]
+            want = maxs[axis] if op == 1 and axis < 2 else v.max() if op == 1 else sums[axis] if axis < 2 else total
+            if op == 2:
+                want = want / acc.type(v.size if axis == 2 else v.shape[1 - axis])
+            out = jas.DeviceArray(n, acc)
+            jas.check(jas.lib.jas_reduce(C.byref(lf), op, axis, out.p, 1 if dt == "f8" else 0, None))
+            assert np.array_equal(out.numpy(), np.asarray(want, acc).reshape(n)), (op, axis)
+
+
 @pytest.mark.parametrize("n_vec,length", [(3, 7), (5, 64), (4, 300), (2, 1000), (3, 2048), (2, 4099), (2, 8192),
                                           (1, 16384), (2, 20000)])
 def test_row_ops(jas, n_vec, length):
