@@ -190,7 +190,8 @@ typedef enum {
  * bias_mode: 0 none, 1 bias[m] (weight_net_t bias broadcast over tokens, mat_net_t.hpp:41),
  *            2 bias[n].
  * Replaces mat_dot_t (mat_express_t.hpp:696-784) and weight_net_t::forward
- * (mat_net_t.hpp:38-49).  fp32 MFMA (v_mfma_f32_16x16x4_f32), fp32 accumulate.
+ * (mat_net_t.hpp:38-49).  Products of three-way bf16 splits of both operands on the bf16
+ * matrix cores, fp32 accumulate: fp32 accuracy (csrc/gemm_split.hip).
  * `batch` independent problems at element offsets *_bstride (0 = shared operand). */
 jas_status jas_gemm(int M, int N, int K,
                     const float *d_A, long as0, long as1,

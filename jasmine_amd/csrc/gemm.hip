@@ -4,14 +4,11 @@
 // with sequential-k accumulation, reached from weight_net_t::forward (mat_net_t.hpp:38-49)
 // for every projection and from mat_head_gen_t::forward (mat_mha_t.hpp:53,71).
 //
-// Two kernels:
-//  * gemm_tile_kernel: 128x128x16 LDS-tiled MFMA GEMM (v_mfma_f32_16x16x4_f32) for
-//    prefill-sized problems; any operand strides (transposed views included).
-//  * skinny_kernel: N <= 16 tokens (decode).  The weight matrix is streamed from HBM
-//    straight into MFMA A-operand registers (no LDS), one 16-row tile per wave set, the
-//    K range split across the waves of a workgroup and reduced through LDS, with the
-//    layer's elementwise tail fused into the epilogue (bias, GELU, residual add, SwiGLU,
-//    RoPE + KV-cache append).
+// Here: skinny_kernel for N <= 16 tokens (decode) -- the weight matrix is streamed from HBM
+// straight into MFMA A-operand registers (no LDS), one 16-row tile per wave set, the K range
+// split across the waves of a workgroup and reduced through LDS, with the layer's elementwise
+// tail fused into the epilogue (bias, GELU, residual add, SwiGLU, RoPE + KV-cache append) --
+// the packed weight layouts, and the fp64 GEMM.  Larger products are in gemm_split.hip.
 //
 // MFMA 16x16x4 f32 operand layout (lane l of 64): A[i = l%16][kslot = l/16],
 // B[kslot = l/16][j = l%16], D rows 4*(l/16)+r (r = 0..3), column l%16.  Each lane loads
@@ -29,44 +26,51 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c)
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// ---------------------------------------------------------------- tiled GEMM
-constexpr int TBM = 128, TBN = 128, TBK = 16;  // output tile edge, K slab width
+static bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-// K-contiguous, outer-contiguous, generic strides, packed weights (weight_pack_offset)
-// and the packed layout with bf16 elements (widened on load)
-enum LoadMode : int { LM_KC = 0, LM_OC = 1, LM_GEN = 2, LM_PK = 3, LM_PKB = 4 };
+jas_status gemm_prefill_fused(int M, int N, int K, const void *A, bool a_bf16, const float *X, float *C, long ldc,
+                              const float *bias, const PrefillFused &fz, hipStream_t s)
+{
+    // SwiGLU: M virtual rows = 2 x the output features (gate / up tiles interleaved)
+    JAS_CHECK(fz.mode != FZ_SWIGLU || (M % 32 == 0 && fz.A2 && !bias), JAS_ERR_INVALID, "prefill GEMM: bad SwiGLU shape");
+    JAS_CHECK(fz.mode != FZ_QKV || (fz.d % 16 == 0 && fz.dh % 16 == 0 && M == 3 * fz.d && fz.pos && (!fz.rope || fz.rope_tab)),
+              JAS_ERR_INVALID, "prefill GEMM: bad QKV shape");
+    JAS_CHECK(al16(A) && al16(X) && al16(C) && K % 16 == 0 && ldc % 4 == 0, JAS_ERR_INVALID, "prefill GEMM: bad operands");
+    SplitArgs p{(const float *)A, X, C, bias, K, 1, 1, K, 1, ldc, 0, 0, 0, 0, M, N, K, bias ? 1 : 0, JAS_ACT_NONE, 0};
+    p.fz = fz;
+    return gemm_split(p, true, a_bf16, 1, s);
+}
 
+// ---------------------------------------------------------------- prefill GEMM into a bf16 KV cache
+// C[n][m] of packed weights A [M][K] and token-major X [N][K] on the fp32 matrix cores: the
+// QKV product of a model whose KV cache holds bf16.  A cached key or value is its fp32 sum
+// rounded to 8 bits, so a sum that differs in its last bit now and then rounds to the other
+// neighbour, 2^-8 away, and the logits move by about 1e-4 -- enough to decide a greedy pick
+// differently.  This product therefore keeps the order of its sums (k ascending by 16, within
+// that k = 4 g + t for t = 0..3) and with it every cache entry, whatever computes the others.
+constexpr int TBK = 16;  // K slab width
 
-// Loads an [OUTER (128 or 64) outer x KW (16 or 32) k] tile of X(o, k) = X[o*so + k*sk]
-// into registers (256 threads), then LDS rows [o][k] (K-contiguous, padded stride KW + 4).
-// The packed layouts are read in 16-wide K blocks only.
-template <int MODE, int OUTER = 128, int KW = 16>
+// [OUTER x 16 k] tile of one operand: registers (256 threads), then LDS rows [o][k] (padded
+// stride).  SM_KC: row-major X(o, k), K % 4 == 0; SM_PK / SM_PKB: the packed weight layouts.
+template <int MODE, int OUTER>
 struct TileLoader {
-    static_assert(KW == 16 || (MODE != LM_PK && MODE != LM_PKB), "packed operands use 16-wide K slabs");
-    static constexpr int LD = KW + 4;              // LDS row stride (floats)
-    static constexpr int NV = OUTER * KW / 1024;   // float4 loads per thread (vector modes)
-    static constexpr int NS = OUTER * KW / 256;    // scalar loads per thread (generic mode)
-    float r[NS];
-    __device__ __forceinline__ void load(const float *__restrict__ X, long so, long sk, int o0, int k0, int O, int K,
-                                         int tid)
+    static constexpr int LD = TBK + 4;               // LDS row stride (floats)
+    static constexpr int NV = OUTER * TBK / 1024;    // float4 loads per thread
+    floatx4 r[NV];
+    __device__ __forceinline__ void load(const float *__restrict__ X, long so, int o0, int k0, int O, int K, int tid)
     {
-        if (MODE == LM_KC) {
 #pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                int idx = tid + q * 256, o = idx / (KW / 4), kq = (idx % (KW / 4)) * 4;
-                int go = o0 + o, gk = k0 + kq;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (go < O && gk < K) v = *(const float4 *)(X + (long)go * so + gk);
-                r[4 * q] = v.x; r[4 * q + 1] = v.y; r[4 * q + 2] = v.z; r[4 * q + 3] = v.w;
-            }
-        } else if (MODE == LM_PK || MODE == LM_PKB) {  // 8 row tiles x one 16-wide K block: 8 contiguous blocks
-#pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                int idx = tid + q * 256, i = idx >> 6, ln = idx & 63;
-                long rt = o0 / 16 + i;
-                floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < NV; ++q) {
+            const int idx = tid + q * 256;
+            floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
+            if (MODE == SM_KC) {
+                const int go = o0 + idx / (TBK / 4), gk = k0 + (idx % (TBK / 4)) * 4;
+                if (go < O && gk < K) v = *(const floatx4 *)(X + (long)go * so + gk);
+            } else {
+                const int ln = idx & 63;
+                const long rt = o0 / 16 + (idx >> 6);
                 if (rt * 16 < O) {
-                    if (MODE == LM_PKB) {  // half (k0/16)%2 of the pair tile: 4 of the lane's 8 elements
+                    if (MODE == SM_PKB) {  // half (k0 / 16) % 2 of the pair tile: 4 of the lane's 8 elements
                         const int kb = k0 >> 4;
                         const long off = weight_tile_offset_b(rt, kb >> 1, k32_of(K), (O + 15) >> 4) + ln * 8 + 4 * (kb & 1);
                         v = widen_bf16x4(*(const u32x2 *)((const uint16_t *)(const void *)X + off));
@@ -74,96 +78,45 @@ struct TileLoader {
                         v = *(const floatx4 *)(X + weight_tile_offset(rt, k0 >> 4, K >> 4, (O + 15) >> 4) + ln * 4);
                     }
                 }
-                r[4 * q] = v[0]; r[4 * q + 1] = v[1]; r[4 * q + 2] = v[2]; r[4 * q + 3] = v[3];
             }
-        } else if (MODE == LM_OC) {
-#pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                int idx = tid + q * 256, k = idx / (OUTER / 4), oq = (idx % (OUTER / 4)) * 4;
-                int go = o0 + oq, gk = k0 + k;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (go < O && gk < K) v = *(const float4 *)(X + (long)gk * sk + go);
-                r[4 * q] = v.x; r[4 * q + 1] = v.y; r[4 * q + 2] = v.z; r[4 * q + 3] = v.w;
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < NS; ++q) {
-                int idx = tid + q * 256, o = idx / KW, k = idx % KW;
-                int go = o0 + o, gk = k0 + k;
-                r[q] = (go < O && gk < K) ? X[(long)go * so + (long)gk * sk] : 0.f;
-            }
+            r[q] = v;
         }
     }
     __device__ __forceinline__ void store(float *lds, int tid) const
     {
-        if (MODE == LM_KC) {
 #pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                int idx = tid + q * 256, o = idx / (KW / 4), kq = (idx % (KW / 4)) * 4;
-                *(float4 *)(lds + o * LD + kq) = make_float4(r[4 * q], r[4 * q + 1], r[4 * q + 2], r[4 * q + 3]);
-            }
-        } else if (MODE == LM_PK || MODE == LM_PKB) {
-#pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                int idx = tid + q * 256, i = idx >> 6, ln = idx & 63;
-                *(float4 *)(lds + (i * 16 + (ln & 15)) * LD + 4 * (ln >> 4)) =
-                    make_float4(r[4 * q], r[4 * q + 1], r[4 * q + 2], r[4 * q + 3]);
-            }
-        } else if (MODE == LM_OC) {
-#pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                int idx = tid + q * 256, k = idx / (OUTER / 4), oq = (idx % (OUTER / 4)) * 4;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) lds[(oq + e) * LD + k] = r[4 * q + e];
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < NS; ++q) {
-                int idx = tid + q * 256, o = idx / KW, k = idx % KW;
-                lds[o * LD + k] = r[q];
-            }
+        for (int q = 0; q < NV; ++q) {
+            const int idx = tid + q * 256;
+            float *d = MODE == SM_KC ? lds + (idx / (TBK / 4)) * LD + (idx % (TBK / 4)) * 4
+                                     : lds + ((idx >> 6) * 16 + (idx & 15)) * LD + 4 * ((idx & 63) >> 4);
+            *(floatx4 *)d = r[q];
         }
     }
 };
 
-struct TileArgs {
-    const float *A, *B;
-    float *C;
-    const float *bias;
-    long as0, as1, bs0, bs1, cs0, cs1;
-    long abs_, bbs, cbs, biasbs;
-    int M, N, K;
-    int bias_mode, act, accumulate;
-};
-
-// T x T output tile (T = 128, or 64 for problems too small to fill the chip with 128-wide
-// tiles); 4 waves in a 2 x 2 grid, each T/2 x T/2 (NB x NB blocks of 16 x 16)
-template <int AM, int BMODE, bool C4, int T = TBM, int KW = TBK>
-__global__ void __launch_bounds__(256) gemm_tile_kernel(const TileArgs p)
+// T x T output tile; 4 waves in a 2 x 2 grid, each T/2 x T/2 (NB x NB blocks of 16 x 16)
+template <int AM, int T>
+__global__ void __launch_bounds__(256)
+gemm_fp32_kernel(int M, int N, int K, const float *__restrict__ A, const float *__restrict__ X, float *__restrict__ C,
+                 long ldc, const float *__restrict__ bias)
 {
-    constexpr int NB = T / 32, LD = KW + 4;
+    constexpr int NB = T / 32, LD = TBK + 4;
     // two LDS buffers: slab k is read from one while slab k+1 is written to the other
     __shared__ float As[2][T * LD];
     __shared__ float Bs[2][T * LD];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wm = w >> 1, wn = w & 1, r16 = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
-    const long bz = blockIdx.z;
-    const float *A = p.A + bz * p.abs_;
-    const float *B = p.B + bz * p.bbs;
-    float *C = p.C + bz * p.cbs;
-    const float *bias = p.bias ? p.bias + bz * p.biasbs : nullptr;
 
-    TileLoader<AM, T, KW> la;
-    TileLoader<BMODE, T, KW> lb;
-    // A(m, k) = A[m*as0 + k*as1]: outer = m.  B(k, n) = B[k*bs0 + n*bs1]: outer = n.
-    la.load(A, p.as0, p.as1, m0, 0, p.M, p.K, tid);
-    lb.load(B, p.bs1, p.bs0, n0, 0, p.N, p.K, tid);
+    TileLoader<AM, T> la;
+    TileLoader<SM_KC, T> lb;
+    la.load(A, K, m0, 0, M, K, tid);
+    lb.load(X, K, n0, 0, N, K, tid);
     la.store(As[0], tid);
     lb.store(Bs[0], tid);
-    if (KW < p.K) {  // slab 1 in flight
-        la.load(A, p.as0, p.as1, m0, KW, p.M, p.K, tid);
-        lb.load(B, p.bs1, p.bs0, n0, KW, p.N, p.K, tid);
+    if (TBK < K) {  // slab 1 in flight
+        la.load(A, K, m0, TBK, M, K, tid);
+        lb.load(X, K, n0, TBK, N, K, tid);
     }
     __syncthreads();
 
@@ -174,584 +127,63 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(const TileArgs p)
         for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     int buf = 0;
-    for (int k0 = 0; k0 < p.K; k0 += KW) {
+    for (int k0 = 0; k0 < K; k0 += TBK) {
         // stage slab k+1 (in registers) into the other buffer, then start slab k+2's loads;
         // the other buffer was last read in the previous step, before its closing barrier
-        if (k0 + KW < p.K) {
+        if (k0 + TBK < K) {
             la.store(As[buf ^ 1], tid);
             lb.store(Bs[buf ^ 1], tid);
-            if (k0 + 2 * KW < p.K) {
-                la.load(A, p.as0, p.as1, m0, k0 + 2 * KW, p.M, p.K, tid);
-                lb.load(B, p.bs1, p.bs0, n0, k0 + 2 * KW, p.N, p.K, tid);
+            if (k0 + 2 * TBK < K) {
+                la.load(A, K, m0, k0 + 2 * TBK, M, K, tid);
+                lb.load(X, K, n0, k0 + 2 * TBK, N, K, tid);
             }
         }
         const float *as = As[buf], *bs = Bs[buf];
+        floatx4 a[NB], b[NB];
 #pragma unroll
-        for (int kh = 0; kh < KW / 16; ++kh) {  // 16-wide K blocks of the slab
-            float4 a[NB], b[NB];
+        for (int i = 0; i < NB; ++i) a[i] = *(const floatx4 *)(as + (wm * (T / 2) + i * 16 + r16) * LD + 4 * g);
 #pragma unroll
-            for (int i = 0; i < NB; ++i)
-                a[i] = *(const float4 *)(as + (wm * (T / 2) + i * 16 + r16) * LD + 16 * kh + 4 * g);
+        for (int j = 0; j < NB; ++j) b[j] = *(const floatx4 *)(bs + (wn * (T / 2) + j * 16 + r16) * LD + 4 * g);
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
             for (int j = 0; j < NB; ++j)
-                b[j] = *(const float4 *)(bs + (wn * (T / 2) + j * 16 + r16) * LD + 16 * kh + 4 * g);
 #pragma unroll
-            for (int i = 0; i < NB; ++i)
-#pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    acc[i][j] = mfma4(a[i].x, b[j].x, acc[i][j]);
-                    acc[i][j] = mfma4(a[i].y, b[j].y, acc[i][j]);
-                    acc[i][j] = mfma4(a[i].z, b[j].z, acc[i][j]);
-                    acc[i][j] = mfma4(a[i].w, b[j].w, acc[i][j]);
-                }
-        }
+                for (int t = 0; t < 4; ++t) acc[i][j] = mfma4(a[i][t], b[j][t], acc[i][j]);
         __syncthreads();
         buf ^= 1;
     }
 
-    // epilogue: lane holds rows m = 4g + r of each 16x16 block, column n = r16
+    // lane holds rows m = 4g + r of each 16 x 16 block, column n = r16 (M % 16 == 0)
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-            const int mb = m0 + wm * (T / 2) + i * 16 + 4 * g, n = n0 + wn * (T / 2) + j * 16 + r16;
-            if (n >= p.N) continue;
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                int m = mb + r;
-                float x = acc[i][j][r];
-                if (bias && m < p.M) x = x + (p.bias_mode == 1 ? bias[m] : bias[n]);
-                v[r] = apply_act(x, p.act);
-            }
-            float *cp = C + (long)mb * p.cs0 + (long)n * p.cs1;
-            if (C4 && mb + 3 < p.M) {  // cs0 == 1: four consecutive rows are contiguous
-                float4 o = make_float4(v[0], v[1], v[2], v[3]);
-                if (p.accumulate) {
-                    float4 c = *(float4 *)cp;
-                    o.x += c.x; o.y += c.y; o.z += c.z; o.w += c.w;
-                }
-                *(float4 *)cp = o;
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (mb + r < p.M) {
-                        float *q = cp + (long)r * p.cs0;
-                        *q = p.accumulate ? *q + v[r] : v[r];
-                    }
-            }
+            const int m = m0 + wm * (T / 2) + i * 16 + 4 * g, n = n0 + wn * (T / 2) + j * 16 + r16;
+            if (n >= N || m >= M) continue;
+            floatx4 v = acc[i][j];
+            if (bias) v += *(const floatx4 *)(bias + m);
+            *(floatx4 *)(C + m + (long)n * ldc) = v;
         }
 }
 
-// 64-wide tiles of plain operands take K slabs of 32 (128-byte row segments, half the
-// barriers per flop); 128-wide tiles keep 16 (32-wide slabs need 72 KB of LDS there and
-// lose occupancy), as do packed weights
-template <int AM, int BMODE>
-static void launch_tile_c(const TileArgs &p, bool c4, bool small, int batch, hipStream_t s)
+jas_status gemm_prefill_fp32(int M, int N, int K, const void *A, bool a_bf16, const float *X, float *C, long ldc,
+                             const float *bias, hipStream_t s)
 {
-    constexpr int KW = (AM == LM_PK || AM == LM_PKB) ? 16 : 32;
-    if (small) {
-        const dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), batch);
-        if (c4) hipLaunchKernelGGL((gemm_tile_kernel<AM, BMODE, true, 64, KW>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((gemm_tile_kernel<AM, BMODE, false, 64, KW>), grid, dim3(256), 0, s, p);
-    } else {
-        const dim3 grid(ceil_div(p.N, TBN), ceil_div(p.M, TBM), batch);
-        if (c4) hipLaunchKernelGGL((gemm_tile_kernel<AM, BMODE, true, TBM, TBK>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((gemm_tile_kernel<AM, BMODE, false, TBM, TBK>), grid, dim3(256), 0, s, p);
-    }
-}
-
-template <int AM>
-static void launch_tile_b(const TileArgs &p, int bm, bool c4, bool small, int batch, hipStream_t s)
-{
-    if (bm == LM_KC) launch_tile_c<AM, LM_KC>(p, c4, small, batch, s);
-    else if (bm == LM_OC) launch_tile_c<AM, LM_OC>(p, c4, small, batch, s);
-    else launch_tile_c<AM, LM_GEN>(p, c4, small, batch, s);
-}
-
-static bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
-
-// choose a vector load mode for operand X(o, k) = X[o*so + k*sk] over a batch
-static int pick_mode(const float *X, long so, long sk, int O, int K, long bstride)
-{
-    bool base = al16(X) && (bstride % 4 == 0);
-    if (sk == 1 && K % 4 == 0 && so % 4 == 0 && base) return LM_KC;
-    if (so == 1 && O % 4 == 0 && sk % 4 == 0 && base) return LM_OC;
-    return LM_GEN;
-}
-
-// ---------------------------------------------------------------- direct-to-LDS GEMM
-// The main fp32 GEMM for operands that are contiguous in one dimension.  K slabs of
-// 16 * KB are moved from global memory straight into LDS (global_load_lds_dwordx4: each
-// wave instruction writes 64 lanes x 16 B contiguously at a wave-uniform LDS base), so no
-// register staging and no LDS store instructions sit in the loop.  ST stage buffers keep
-// ST - 1 slabs in flight; one barrier per slab.
-//
-// LDS layouts, chosen so that every fragment read is one conflict-free ds_read_b128:
-//  * K-contiguous operand X(o, k) (and the packed weight layout): per 16 x 16 block, the 64
-//    lanes' float4s in MFMA operand order -- lane r + 16 g holds X(16 b + r, 4 g .. 4 g + 3).
-//    Sub-step t of the four 16x16x4 MFMAs per block takes element t, so k-slot g of
-//    sub-step t is k = 4 g + t, a permutation of K applied to both operands alike.
-//  * Outer-contiguous operand: rows [k][o] as in memory.  Lane (g, r) reads the float4
-//    X(o0 + 4 r .. 4 r + 3, k = 4 g + t): its four elements feed four different 16-wide
-//    blocks (block e takes outer index 4 r + e), so one read serves four MFMAs, and the
-//    output of those blocks comes out as four consecutive columns per lane.
-// The compiler cannot see the LDS writes of the DMA (they are issued as asm, so its
-// wait-count pass does not serialise the LDS reads behind every load in flight); the loop
-// waits on vmcnt itself before each barrier.
-enum DmaMode : int { DM_KC = 0, DM_OC = 1, DM_PK = 2 };
-
-struct DmaArgs {
-    const float *A, *B;
-    float *C;
-    const float *bias;
-    long as0, as1, bs0, bs1, cs0, cs1;
-    long abs_, bbs, cbs, biasbs;
-    int M, N, K;
-    int bias_mode, act, accumulate;
-    int c_vec;  // 1: row-major C with float4 stores over n; 2: column-major C, float4 over m
-    // fused prefill epilogues (packed weights, token-major output, c_vec == 2)
-    DmaFused fz;
-    // residual source added after the bias (residual_net_t's f(x) + x): R(m, n) = resid[m*rs0 + n*rs1]
-    const float *resid = nullptr;
-    long rs0 = 0, rs1 = 0;
-};
-
-// M0 is a reserved register to the compiler; nothing else in these kernels uses it (no
-// relative register indexing, no other LDS DMA), which the AMD assembly of the build shows.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_dma16(const float *src, float *lds_dst)
-{
-    const unsigned la = (unsigned)(size_t)(__attribute__((address_space(3))) float *)lds_dst;
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(la), "v"(src) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// Global address of lane `lane`'s 16 bytes for DMA instruction `ins` of the slab at k0, and
-// whether the slab element group lies inside K (only the tail slab can leave K).
-// X(o, k) = X[o * so + k * sk]; Olim = rows (outer extent); RG = packed row tiles.
-template <int MODE, int O, int KWT>
-__device__ __forceinline__ const float *dma_src(const float *X, const float *X2, long so, long sk, int o0, int Olim,
-                                                int K, int k0, int ins, int lane, int &kfirst)
-{
-    if (MODE == DM_OC) {
-        const int f = 256 * ins + 4 * lane, k = k0 + f / O;
-        int o = o0 + f % O;
-        o = o <= Olim - 4 ? o : Olim - 4;  // clamped groups only feed discarded outputs
-        kfirst = k;
-        return X + (long)(k < K ? k : K - 1) * sk + o;
-    }
-    constexpr int RB = O / 16;
-    const int kb = ins / RB, rb = ins % RB;
-    if (MODE == DM_PK) {
-        const long RG = (Olim + 15) >> 4;
-        long rt = min((long)(o0 >> 4) + rb, RG - 1);
-        const int kblk = (k0 >> 4) + kb;
-        kfirst = 16 * kblk;
-        const float *Xm = X;
-        long RGm = RG;
-        if (X2) {  // SwiGLU: virtual row tile 2f is gate tile f, 2f + 1 up tile f
-            Xm = rt & 1 ? X2 : X;
-            rt >>= 1;
-            RGm = RG >> 1;
-        }
-        return Xm + weight_tile_offset(rt, kblk < (K >> 4) ? kblk : (K >> 4) - 1, K >> 4, RGm) + lane * 4;
-    }
-    int o = o0 + 16 * rb + (lane & 15);
-    o = o < Olim ? o : Olim - 1;
-    kfirst = k0 + 16 * kb + 4 * (lane >> 4);
-    return X + (long)o * so + (kfirst < K ? kfirst : 0);
-}
-
-template <int MODE, int O, int KWT, int NW>
-__device__ __forceinline__ void dma_slab(const float *X, const float *X2, long so, long sk, int o0, int Olim, int K,
-                                         int k0, float *lds, int w, int lane)
-{
-    constexpr int NI = O * KWT / 256;  // 1 KB instructions per slab
-    static_assert(NI % NW == 0, "slab instructions spread evenly over the waves");
-#pragma unroll
-    for (int q = 0; q < NI / NW; ++q) {
-        const int ins = w * (NI / NW) + q;  // wave-uniform
-        int kf;
-        lds_dma16(dma_src<MODE, O, KWT>(X, X2, so, sk, o0, Olim, K, k0, ins, lane, kf), lds + 256 * ins);
-    }
-}
-
-// The last, partial slab (K % (16 KB) != 0): ordinary loads with zeros past K, stored in the
-// same layout.
-template <int MODE, int O, int KWT, int NW>
-__device__ __forceinline__ void tail_slab(const float *X, const float *X2, long so, long sk, int o0, int Olim, int K,
-                                          int k0, float *lds, int w, int lane)
-{
-    constexpr int NI = O * KWT / 256;
-#pragma unroll
-    for (int q = 0; q < NI / NW; ++q) {
-        const int ins = w * (NI / NW) + q;
-        int kf;
-        const float *src = dma_src<MODE, O, KWT>(X, X2, so, sk, o0, Olim, K, k0, ins, lane, kf);
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (MODE == DM_KC) {  // per element: K need not be a multiple of 4
-            float e[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) e[u] = kf + u < K ? src[u] : 0.f;
-            v = make_float4(e[0], e[1], e[2], e[3]);
-        } else if (kf < K) {
-            v = *(const float4 *)src;
-        }
-        *(float4 *)(lds + 256 * ins + 4 * lane) = v;
-    }
-}
-
-// Fragment values of sub-step t of 16-block kb for the NB blocks of this wave
-// (outer offset woff within the tile).
-template <int MODE, int NB, int O>
-__device__ __forceinline__ void dma_frag(const float *s, int kb, int t, int woff, int lane, float (&v)[NB],
-                                         float4 (&blk)[NB])
-{
-    const int r16 = lane & 15, g = lane >> 4;
-    if (MODE != DM_OC) {
-        if (t == 0) {
-#pragma unroll
-            for (int i = 0; i < NB; ++i) blk[i] = *(const float4 *)(s + (kb * (O / 16) + woff / 16 + i) * 256 + lane * 4);
-        }
-#pragma unroll
-        for (int i = 0; i < NB; ++i) v[i] = blk[i][t];
-    } else {
-        constexpr int G = NB < 4 ? NB : 4;
-        const float *row = s + (16 * kb + 4 * g + t) * O + woff;
-#pragma unroll
-        for (int q = 0; q < NB / G; ++q) {
-            if constexpr (G == 4) {
-                const float4 x = *(const float4 *)(row + 64 * q + 4 * r16);
-                v[4 * q] = x.x; v[4 * q + 1] = x.y; v[4 * q + 2] = x.z; v[4 * q + 3] = x.w;
-            } else if constexpr (G == 2) {
-                const float2 x = *(const float2 *)(row + 32 * q + 2 * r16);
-                v[2 * q] = x.x; v[2 * q + 1] = x.y;
-            } else {
-                v[q] = row[16 * q + r16];
-            }
-        }
-    }
-}
-
-// outer index (within the wave tile) of MFMA row/column ii of block i
-template <int MODE, int NB>
-__device__ __forceinline__ int dma_outer(int i, int ii)
-{
-    constexpr int G = NB < 4 ? NB : 4;
-    return MODE != DM_OC ? 16 * i + ii : 16 * G * (i / G) + G * ii + (i % G);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm_barrier()
-{
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// TM x TN tile, NW waves in a WGM x (NW / WGM) grid, ST stages of 16 * KB wide K slabs.
-// Workgroup ids are remapped so that each of the 8 XCDs (ids go round-robin over them)
-// works on a contiguous range of tiles, walked 4 tile rows at a time: the A rows and B
-// columns its workgroups share stay in that XCD's L2.
-template <int AM, int BM, int TM, int TN, int NW, int WGM, int ST, int KB>
-__global__ void __launch_bounds__(NW * 64) gemm_dma_kernel(const DmaArgs p)
-{
-    constexpr int WGN = NW / WGM, WTM = TM / WGM, WTN = TN / WGN, NBI = WTM / 16, NBJ = WTN / 16;
-    constexpr int KWT = 16 * KB, SA = TM * KWT, SB = TN * KWT;
-    constexpr int PER = (SA / 256 + SB / 256) / NW;  // DMA instructions per thread and slab
-    static_assert(PER * (ST - 2) <= 63, "vmcnt range");
-    static_assert(AM != DM_OC || NBI % 4 == 0 || NBI < 4, "outer-contiguous groups");
-    __shared__ __attribute__((aligned(1024))) float lds[ST * (SA + SB)];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = w / WGN, wn = w % WGN, r16 = lane & 15, g = lane >> 4;
-
-    int bx = blockIdx.x, by = blockIdx.y;
-    {
-        constexpr int XG = 4;
-        const int gx = gridDim.x, nt = gx * gridDim.y, per = nt / 8;
-        const int id = blockIdx.y * gx + blockIdx.x;
-        // a permutation of the ids: the first 8 * per go XCD-contiguous, the rest stay
-        const int lid = id < 8 * per ? (id % 8) * per + id / 8 : id;
-        const int grp = lid / (XG * gx), gy0 = grp * XG, rows = min(XG, (int)gridDim.y - gy0);
-        const int in = lid - grp * XG * gx;
-        by = gy0 + in % rows;
-        bx = in / rows;
-    }
-    const int m0 = by * TM, n0 = bx * TN;
-    const long bz = blockIdx.z;
-    const float *A = p.A + bz * p.abs_;
-    const float *B = p.B + bz * p.bbs;
-    const int K = p.K, nk = K / KWT;
-    const bool tail = nk * KWT < K;
-
-    auto issue = [&](int kt) {
-        float *sa = lds + (kt % ST) * (SA + SB), *sb = sa + SA;
-        dma_slab<AM, TM, KWT, NW>(A, p.fz.A2, p.as0, p.as1, m0, p.M, K, kt * KWT, sa, w, lane);
-        dma_slab<BM, TN, KWT, NW>(B, nullptr, p.bs1, p.bs0, n0, p.N, K, kt * KWT, sb, w, lane);
-    };
-    floatx4 acc[NBI][NBJ];
-#pragma unroll
-    for (int i = 0; i < NBI; ++i)
-#pragma unroll
-        for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const float *sa) {
-        const float *sb = sa + SA;
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-            float4 ablk[NBI], bblk[NBJ];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                float av[NBI], bv[NBJ];
-                dma_frag<AM, NBI, TM>(sa, kb, t, wm * WTM, lane, av, ablk);
-                dma_frag<BM, NBJ, TN>(sb, kb, t, wn * WTN, lane, bv, bblk);
-#pragma unroll
-                for (int i = 0; i < NBI; ++i)
-#pragma unroll
-                    for (int j = 0; j < NBJ; ++j) acc[i][j] = mfma4(av[i], bv[j], acc[i][j]);
-            }
-        }
-    };
-
-#pragma unroll
-    for (int s = 0; s < ST - 1; ++s)
-        if (s < nk) issue(s);
-    for (int kt = 0; kt < nk; ++kt) {
-        // slab kt has landed (this thread's loads: the later slabs may still be in flight);
-        // the barrier makes every wave's part visible and retires the reads of the buffer
-        // the next issue overwrites (last read in iteration kt - 1)
-        const int ahead = min(ST - 2, nk - 1 - kt);
-        if (ahead >= 2) wait_vm_barrier<2 * PER>();
-        else if (ahead == 1) wait_vm_barrier<PER>();
-        else wait_vm_barrier<0>();
-        if (kt + ST - 1 < nk) issue(kt + ST - 1);
-        compute(lds + (kt % ST) * (SA + SB));
-    }
-    if (tail) {
-        // stage nk % ST was last read in iteration nk - ST, which every wave finished before
-        // the barrier of iteration nk - 1
-        float *sa = lds + (nk % ST) * (SA + SB), *sb = sa + SA;
-        tail_slab<AM, TM, KWT, NW>(A, p.fz.A2, p.as0, p.as1, m0, p.M, K, nk * KWT, sa, w, lane);
-        tail_slab<BM, TN, KWT, NW>(B, nullptr, p.bs1, p.bs0, n0, p.N, K, nk * KWT, sb, w, lane);
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        compute(sa);
-    }
-
-    // epilogue: block (i, j), lane (g, r16), register r holds MFMA row 4 g + r, column r16
-    float *C = p.C + bz * p.cbs;
-    const float *bias = p.bias ? p.bias + bz * p.biasbs : nullptr;
-    auto finish = [&](float x, int m, int n, float *cp) {
-        if (bias) x = x + (p.bias_mode == 1 ? bias[m] : bias[n]);
-        x = apply_act(x, p.act);
-        if (p.resid) x = x + p.resid[(long)m * p.rs0 + (long)n * p.rs1];
-        return p.accumulate ? *cp + x : x;
-    };
-    const int mw = m0 + wm * WTM, nw = n0 + wn * WTN;
-    if (BM == DM_OC && NBJ >= 4 && p.c_vec == 1) {  // row-major C: four consecutive n per lane
-#pragma unroll
-        for (int i = 0; i < NBI; ++i)
-#pragma unroll
-            for (int q = 0; q < NBJ / 4; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = mw + dma_outer<AM, NBI>(i, 4 * g + r), n = nw + 64 * q + 4 * r16;
-                    if (m >= p.M || n >= p.N) continue;
-                    float *cp = C + (long)m * p.cs0 + n;
-                    float4 o;
-                    o.x = finish(acc[i][4 * q][r], m, n, cp);
-                    o.y = finish(acc[i][4 * q + 1][r], m, n + 1, cp + 1);
-                    o.z = finish(acc[i][4 * q + 2][r], m, n + 2, cp + 2);
-                    o.w = finish(acc[i][4 * q + 3][r], m, n + 3, cp + 3);
-                    *(float4 *)cp = o;
-                }
-    } else if (AM != DM_OC && p.c_vec == 2 && p.fz.mode == FZ_SWIGLU) {
-        // virtual rows: block 2k holds gate features, block 2k + 1 the up features of the same
-        // 16 outputs, so both products of an output sit in one lane: out = silu(gate) * up
-#pragma unroll
-        for (int i = 0; i < NBI; i += 2)
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j) {
-                const int mv = mw + 16 * i + 4 * g, n = nw + dma_outer<BM, NBJ>(j, r16);
-                const int f = (mv >> 5) * 16 + (mv & 15);  // output feature of this lane's first row
-                if (n >= p.N || 2 * f >= p.M) continue;
-                float4 o;
-                o.x = silu_f(acc[i][j][0]) * acc[i + 1][j][0];
-                o.y = silu_f(acc[i][j][1]) * acc[i + 1][j][1];
-                o.z = silu_f(acc[i][j][2]) * acc[i + 1][j][2];
-                o.w = silu_f(acc[i][j][3]) * acc[i + 1][j][3];
-                *(float4 *)(C + f + (long)n * p.cs1) = o;
-            }
-    } else if (AM != DM_OC && p.c_vec == 2 && p.fz.mode == FZ_QKV) {
-        // rows [0, d) q, [d, 2d) k, [2d, 3d) v of token n: bias, rotary on q and k (pairs
-        // (2i, 2i+1) of a head are registers (0, 1) and (2, 3) of one lane), the row, and k / v
-        // into the KV cache at the token's position
-        const DmaFused &z = p.fz;
-#pragma unroll
-        for (int i = 0; i < NBI; ++i)
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j) {
-                const int m = mw + 16 * i + 4 * g, n = nw + dma_outer<BM, NBJ>(j, r16);
-                if (n >= p.N || m >= p.M) continue;
-                float v[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = bias ? acc[i][j][r] + bias[m + r] : acc[i][j][r];
-                const int sec = m / z.d, e = m % z.dh, hh = (m % z.d) / z.dh;
-                const int t = z.pos[n];
-                if (z.rope && sec < 2) {
-#pragma unroll
-                    for (int pr = 0; pr < 2; ++pr) {
-                        const double2 cs = z.rope_tab[(long)t * (z.dh / 2) + (e >> 1) + pr];
-                        const double x0 = v[2 * pr], x1 = v[2 * pr + 1];
-                        v[2 * pr] = (float)(x0 * cs.x - x1 * cs.y);
-                        v[2 * pr + 1] = (float)(x0 * cs.y + x1 * cs.x);
-                    }
-                }
-                *(float4 *)(C + m + (long)n * p.cs1) = make_float4(v[0], v[1], v[2], v[3]);
-                if (sec >= 1) {
-                    const int bseq = n / z.P;
-                    const long dst = (((long)bseq * z.H + hh) * z.ctx + t) * z.dh + e;
-                    void *cache = sec == 1 ? z.kc : z.vc;
-                    if (z.kv_bf16)
-                        *(u32x2 *)((uint16_t *)cache + dst) =
-                            u32x2{(uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
-                                  (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16)};
-                    else
-                        *(float4 *)((float *)cache + dst) = make_float4(v[0], v[1], v[2], v[3]);
-                }
-            }
-    } else if (AM != DM_OC && p.c_vec == 2) {  // column-major C: four consecutive m per lane
-#pragma unroll
-        for (int i = 0; i < NBI; ++i)
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j) {
-                const int m = mw + 16 * i + 4 * g, n = nw + dma_outer<BM, NBJ>(j, r16);
-                if (n >= p.N || m >= p.M) continue;
-                float *cp = C + m + (long)n * p.cs1;
-                if (m + 3 < p.M) {
-                    float4 o;
-                    o.x = finish(acc[i][j][0], m, n, cp);
-                    o.y = finish(acc[i][j][1], m + 1, n, cp + 1);
-                    o.z = finish(acc[i][j][2], m + 2, n, cp + 2);
-                    o.w = finish(acc[i][j][3], m + 3, n, cp + 3);
-                    *(float4 *)cp = o;
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (m + r < p.M) cp[r] = finish(acc[i][j][r], m + r, n, cp + r);
-                }
-            }
-    } else {
-#pragma unroll
-        for (int i = 0; i < NBI; ++i)
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = mw + dma_outer<AM, NBI>(i, 4 * g + r), n = nw + dma_outer<BM, NBJ>(j, r16);
-                    if (m >= p.M || n >= p.N) continue;
-                    float *cp = C + (long)m * p.cs0 + (long)n * p.cs1;
-                    *cp = finish(acc[i][j][r], m, n, cp);
-                }
-    }
-}
-
-// Geometry: 256 x 256 tiles (8 waves, 3 stages) when they give every CU a workgroup, else
-// 128 x 128 (4 waves, 4 stages) when those give every CU at least four, else 64 x 64 (4
-// waves, 4 stages of 32-wide slabs) when those give every CU one, else 32 x 32 (one 16 x 16
-// block per wave: four times the workgroups; jasmine's Transformer-base encoder-decoder, 512
-// x 512 products, encode 0.49 -> 0.34 ms; neutral at 1024^3).  64 x 64 tiles win wherever the 128-wide ones would
-// leave a partly filled last round (GPT-2-small prefill QKV 2304 x 4096 x 768: 90 against
-// 75 TFLOP/s; FC 3072 x 4096 x 768: 92 against 84).  MI355X fp32: 4096^3 at 130-137
-// TFLOP/s, 2048^3 at 113, 1024^3 at 82-89.
-// JAS_GEMM_GEOMETRY=256|128|64|32 forces one geometry (a tuning knob; default: the rule above).
-static int forced_geometry()
-{
-    static const int g = [] {
-        const char *e = getenv("JAS_GEMM_GEOMETRY");
-        return e ? atoi(e) : 0;
-    }();
-    return g;
-}
-
-template <int AM, int BM>
-static void launch_dma(const DmaArgs &p, int batch, hipStream_t s)
-{
-    auto tiles = [&](int t) { return (long)ceil_div(p.M, t) * ceil_div(p.N, t) * batch; };
-    const int fg = forced_geometry();
-    if (fg == 256 || (fg == 0 && tiles(256) >= 256)) {
-        const dim3 grid(ceil_div(p.N, 256), ceil_div(p.M, 256), batch);
-        hipLaunchKernelGGL((gemm_dma_kernel<AM, BM, 256, 256, 8, 2, 3, 1>), grid, dim3(512), 0, s, p);
-    } else if (fg == 128 || (fg == 0 && tiles(128) >= 1024)) {
-        const dim3 grid(ceil_div(p.N, 128), ceil_div(p.M, 128), batch);
-        hipLaunchKernelGGL((gemm_dma_kernel<AM, BM, 128, 128, 4, 2, 4, 1>), grid, dim3(256), 0, s, p);
-    } else if (AM != DM_PK && p.fz.mode == FZ_NONE && (fg == 32 || (fg == 0 && tiles(64) < 256))) {
-        // plain operands only: packed weights and the fused prefill epilogues (SwiGLU pairs
-        // two 16-row blocks in one wave) assume wave tiles of at least 32 rows
-        if constexpr (AM != DM_PK) {
-            const dim3 grid(ceil_div(p.N, 32), ceil_div(p.M, 32), batch);
-            hipLaunchKernelGGL((gemm_dma_kernel<AM, BM, 32, 32, 4, 2, 4, 2>), grid, dim3(256), 0, s, p);
-        }
-    } else {
-        const dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), batch);
-        hipLaunchKernelGGL((gemm_dma_kernel<AM, BM, 64, 64, 4, 2, 4, 2>), grid, dim3(256), 0, s, p);
-    }
-}
-
-// DMA load mode of operand X(o, k) = X[o * so + k * sk] (batch stride bst), or -1
-static int dma_mode(const float *X, long so, long sk, int O, long bst)
-{
-    if (((uintptr_t)X & 15) || bst % 4) return -1;
-    if (sk == 1 && so % 4 == 0) return DM_KC;
-    if (so == 1 && sk % 4 == 0 && O % 4 == 0) return DM_OC;
-    return -1;
-}
-
-static bool gemm_dma(int M, int N, int K, const void *A, long as0, long as1, const float *B, long bs0, long bs1,
-                     float *C, long cs0, long cs1, const float *bias, int bias_mode, int act, int accumulate, int batch,
-                     long abs_, long bbs, long cbs, long biasbs, hipStream_t s, bool a_packed, bool a_bf16,
-                     const DmaFused *fz = nullptr, const float *resid = nullptr, long rs0 = 0, long rs1 = 0)
-{
-    if (a_bf16 || K <= 0) return false;
-    int am = a_packed ? DM_PK : dma_mode((const float *)A, as0, as1, M, abs_);
-    if (a_packed && (((uintptr_t)A & 15) || K % 16 || batch != 1)) return false;
-    const int bm = dma_mode(B, bs1, bs0, N, bbs);
-    if (am < 0 || bm < 0) return false;
-    DmaArgs p;
-    p.A = (const float *)A; p.B = B; p.C = C; p.bias = bias_mode ? bias : nullptr;
-    p.as0 = as0; p.as1 = as1; p.bs0 = bs0; p.bs1 = bs1; p.cs0 = cs0; p.cs1 = cs1;
-    p.abs_ = abs_; p.bbs = bbs; p.cbs = cbs; p.biasbs = biasbs;
-    p.M = M; p.N = N; p.K = K;
-    p.bias_mode = bias_mode; p.act = act; p.accumulate = accumulate;
-    p.resid = resid; p.rs0 = rs0; p.rs1 = rs1;
-    if (resid && (batch != 1 || fz)) return false;
-    const bool ca = ((uintptr_t)C & 15) == 0 && cbs % 4 == 0;
-    p.c_vec = 0;
-    if (ca && cs1 == 1 && cs0 % 4 == 0 && N % 4 == 0) p.c_vec = 1;
-    else if (ca && cs0 == 1 && cs1 % 4 == 0) p.c_vec = 2;
-    if (fz) {
-        if (!a_packed || p.c_vec != 2 || batch != 1 || accumulate || act != JAS_ACT_NONE) return false;
-        p.fz = *fz;
-    }
-#define JAS_DMA_B(AMV)                                                                                 \
-    if (bm == DM_KC) launch_dma<AMV, DM_KC>(p, batch, s);                                             \
-    else launch_dma<AMV, DM_OC>(p, batch, s);
-    if (am == DM_PK) { JAS_DMA_B(DM_PK) }
-    else if (am == DM_KC) { JAS_DMA_B(DM_KC) }
-    else { JAS_DMA_B(DM_OC) }
-#undef JAS_DMA_B
-    return true;
-}
-
-bool gemm_prefill_fused(int M, int N, int K, const void *A, const float *X, float *C, long ldc, const float *bias,
-                        const DmaFused &fz, hipStream_t s)
-{
-    // SwiGLU: M virtual rows = 2 x the output features (gate / up tiles interleaved)
-    if (fz.mode == FZ_SWIGLU && (M % 32 || !fz.A2 || bias)) return false;
-    if (fz.mode == FZ_QKV && (fz.d % 16 || fz.dh % 16 || M != 3 * fz.d || !fz.pos || (fz.rope && !fz.rope_tab)))
-        return false;
-    const bool ok = gemm_dma(M, N, K, A, K, 1, X, 1, K, C, 1, ldc, bias, bias ? 1 : 0, JAS_ACT_NONE, 0, 1, 0, 0, 0, 0,
-                             s, true, false, &fz);
-    return ok && hipGetLastError() == hipSuccess;
+    JAS_CHECK(M % 16 == 0 && K % 16 == 0 && ldc % 4 == 0 && al16(A) && al16(X) && al16(C) && (!bias || al16(bias)),
+              JAS_ERR_INVALID, "prefill GEMM: bad operands");
+    // 64-wide tiles when 128-wide ones give at most three workgroups per CU
+    const bool small = (long)ceil_div(N, 128) * ceil_div(M, 128) <= 3 * 256;
+#define JAS_PF(AM, T)                                                                                              \
+    hipLaunchKernelGGL((gemm_fp32_kernel<AM, T>), dim3(ceil_div(N, T), ceil_div(M, T)), dim3(256), 0, s, M, N, K, \
+                       (const float *)A, X, C, ldc, bias)
+    if (a_bf16 && small) JAS_PF(SM_PKB, 64);
+    else if (a_bf16) JAS_PF(SM_PKB, 128);
+    else if (small) JAS_PF(SM_PK, 64);
+    else JAS_PF(SM_PK, 128);
+#undef JAS_PF
+    JAS_LAUNCH_CHECK();
+    return JAS_OK;
 }
 
 jas_status gemm_general(int M, int N, int K, const void *A, long as0, long as1, const float *B, long bs0, long bs1,
@@ -760,33 +192,10 @@ jas_status gemm_general(int M, int N, int K, const void *A, long as0, long as1, 
                         bool a_bf16)
 {
     JAS_CHECK(!a_bf16 || a_packed, JAS_ERR_INVALID, "gemm: bf16 A only in the packed layout");
-    JAS_CHECK(!a_packed || (K % 16 == 0 && batch == 1), JAS_ERR_INVALID, "gemm: packed A needs K % 16 == 0");
-    if (gemm_dma(M, N, K, A, as0, as1, B, bs0, bs1, C, cs0, cs1, bias, bias_mode, act, accumulate, batch, abs_, bbs,
-                 cbs, biasbs, s, a_packed, a_bf16)) {
-        JAS_LAUNCH_CHECK();
-        return JAS_OK;
-    }
-    TileArgs p;
-    p.A = (const float *)A; p.B = B; p.C = C; p.bias = bias_mode ? bias : nullptr;
-    p.as0 = as0; p.as1 = as1; p.bs0 = bs0; p.bs1 = bs1; p.cs0 = cs0; p.cs1 = cs1;
-    p.abs_ = abs_; p.bbs = bbs; p.cbs = cbs; p.biasbs = biasbs;
-    p.M = M; p.N = N; p.K = K;
-    p.bias_mode = bias_mode; p.act = act; p.accumulate = accumulate;
-    JAS_CHECK(!a_packed || (K % 16 == 0 && batch == 1), JAS_ERR_INVALID, "gemm: packed A needs K % 16 == 0");
-    int am = a_packed ? (a_bf16 ? LM_PKB : LM_PK) : pick_mode((const float *)A, as0, as1, M, K, abs_);
-    int bm = pick_mode(B, bs1, bs0, N, K, bbs);
-    bool c4 = cs0 == 1 && al16(C) && (cs1 % 4 == 0) && (cbs % 4 == 0);
-    // 64-wide tiles when 128-wide ones give at most three workgroups per CU: too few to fill
-    // the chip, or so few rounds that the last, partly empty one weighs (GPT-2-small prefill
-    // GEMMs of 576 and 768 such workgroups: 8.34 -> 8.05 ms per prefill)
-    const bool small = (long)ceil_div(N, TBN) * ceil_div(M, TBM) * batch <= 3 * 256;
-    if (am == LM_PKB) launch_tile_b<LM_PKB>(p, bm, c4, small, batch, s);
-    else if (am == LM_PK) launch_tile_b<LM_PK>(p, bm, c4, small, batch, s);
-    else if (am == LM_KC) launch_tile_b<LM_KC>(p, bm, c4, small, batch, s);
-    else if (am == LM_OC) launch_tile_b<LM_OC>(p, bm, c4, small, batch, s);
-    else launch_tile_b<LM_GEN>(p, bm, c4, small, batch, s);
-    JAS_LAUNCH_CHECK();
-    return JAS_OK;
+    JAS_CHECK(!a_packed || (K % 16 == 0 && batch == 1 && al16(A)), JAS_ERR_INVALID, "gemm: packed A needs K % 16 == 0");
+    const SplitArgs p{(const float *)A, B,    C,   bias_mode ? bias : nullptr, as0, as1, bs0, bs1, cs0,       cs1, abs_,
+                      bbs,              cbs,  biasbs, M,                       N,   K,   bias_mode, act, accumulate};
+    return gemm_split(p, a_packed, a_bf16, batch, s);
 }
 
 // first maximum (ties to the lowest index) over the four 16-lane rows of a wave: lanes l,
@@ -1425,16 +834,6 @@ extern "C" jas_status jas_gemm(int M, int N, int K, const float *A, long as0, lo
                         bbs, cbs, biasbs, s, false);
 }
 
-// C(m, n) += R(m, n) after a product that did not take the residual in its epilogue
-__global__ void add_residual_kernel(float *C, long cs0, long cs1, const float *R, long rs0, long rs1, int M, int N)
-{
-    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (long)M * N) return;
-    const int m = (int)(g / N), n = (int)(g % N);
-    float *c = C + (long)m * cs0 + (long)n * cs1;
-    *c = *c + R[(long)m * rs0 + (long)n * rs1];
-}
-
 extern "C" jas_status jas_gemm_residual(int M, int N, int K, const float *A, long as0, long as1, const float *B,
                                         long bs0, long bs1, float *C, long cs0, long cs1, const float *bias,
                                         int bias_mode, int act, const float *R, long rs0, long rs1,
@@ -1446,19 +845,7 @@ extern "C" jas_status jas_gemm_residual(int M, int N, int K, const float *A, lon
               "jas_gemm_residual: bad bias");
     JAS_CHECK(act >= JAS_ACT_NONE && act <= JAS_ACT_SIGMOID, JAS_ERR_INVALID, "jas_gemm_residual: bad activation");
     if (M == 0 || N == 0) return JAS_OK;
-    hipStream_t s = stream_or_default(stream);
-    if (gemm_dma(M, N, K, A, as0, as1, B, bs0, bs1, C, cs0, cs1, bias, bias_mode, act, 0, 1, 0, 0, 0, 0, s, false,
-                 false, nullptr, R, rs0, rs1)) {
-        JAS_LAUNCH_CHECK();
-        return JAS_OK;
-    }
-    // other operand layouts: the product, then the residual added in the same order
-    const jas_status st = jas_gemm(M, N, K, A, as0, as1, B, bs0, bs1, C, cs0, cs1, bias, bias_mode, act, 0, 1, 0, 0,
-                                   0, 0, stream);
-    if (st != JAS_OK) return st;
-    const long n = (long)M * N;
-    hipLaunchKernelGGL(add_residual_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, C, cs0, cs1, R, rs0,
-                       rs1, M, N);
-    JAS_LAUNCH_CHECK();
-    return JAS_OK;
+    SplitArgs p{A, B, C, bias_mode ? bias : nullptr, as0, as1, bs0, bs1, cs0, cs1, 0, 0, 0, 0, M, N, K, bias_mode, act, 0};
+    p.resid = R, p.rs0 = rs0, p.rs1 = rs1;
+    return gemm_split(p, false, false, 1, stream_or_default(stream));
 }

@@ -139,9 +139,9 @@ jas_status skinny_gemm(const void *W, const void *W2, const float *X, long ldx, 
                        const SkinnyEpiArgs &epi, hipStream_t s, bool packed = false,
                        const SkinnyTuning *tune = nullptr, bool wbf16 = false);
 
-// Fused epilogues of the prefill GEMMs on packed fp32 weights (token-major output).
+// Fused epilogues of the prefill GEMMs on packed weights (token-major output).
 enum FusedMode : int { FZ_NONE = 0, FZ_QKV = 1, FZ_SWIGLU = 2 };
-struct DmaFused {
+struct PrefillFused {
     int mode = FZ_NONE;
     const float *A2 = nullptr;  // FZ_SWIGLU: the up weights (A: the gate weights)
     // FZ_QKV: rows [0, d) q, [d, 2d) k, [2d, 3d) v; rotary on q and k from rope_tab
@@ -150,15 +150,37 @@ struct DmaFused {
     const int32_t *pos = nullptr;
     const double2 *rope_tab = nullptr;
     int rope = 0;
-    void *kc = nullptr, *vc = nullptr;
-    int kv_bf16 = 0;
+    float *kc = nullptr, *vc = nullptr;
     int d = 0, dh = 0, H = 0, P = 0, ctx = 0;
 };
-// C[n][m] for packed weights A [M][K] and token-major X [N][K], with a fused epilogue;
-// false when the product does not qualify (the caller then runs the unfused sequence).
-// FZ_SWIGLU: M = 2 x the output features, C [N][M / 2] = silu(gate) * up.
-bool gemm_prefill_fused(int M, int N, int K, const void *A, const float *X, float *C, long ldc, const float *bias,
-                        const DmaFused &fz, hipStream_t s);
+// C[n][m] for packed weights A [M][K] (a_bf16: the bf16 layout) and token-major X [N][K], with
+// a fused epilogue.  FZ_SWIGLU: M = 2 x the output features, C [N][M / 2] = silu(gate) * up.
+jas_status gemm_prefill_fused(int M, int N, int K, const void *A, bool a_bf16, const float *X, float *C, long ldc,
+                              const float *bias, const PrefillFused &fz, hipStream_t s);
+
+// C[n][m] = A . X (+ bias[m]) for packed weights on the fp32 matrix cores (the QKV product of
+// a model whose KV cache is bf16)
+jas_status gemm_prefill_fp32(int M, int N, int K, const void *A, bool a_bf16, const float *X, float *C, long ldc,
+                             const float *bias, hipStream_t s);
+
+// Staging mode of a GEMM operand X(o, k): K-contiguous, outer-contiguous, any strides, packed
+// weights (weight_pack_offset), packed bf16 weights (weight_pack_offset_b).
+enum SplitMode : int { SM_KC = 0, SM_OC = 1, SM_GEN = 2, SM_PK = 3, SM_PKB = 4 };
+struct SplitArgs {
+    const float *A, *B;
+    float *C;
+    const float *bias;
+    long as0, as1, bs0, bs1, cs0, cs1;
+    long abs_, bbs, cbs, biasbs;
+    int M, N, K;
+    int bias_mode, act, accumulate;
+    PrefillFused fz;  // fused prefill epilogues (packed weights, token-major output)
+    // residual source added after the bias (residual_net_t's f(x) + x): R(m, n) = resid[m*rs0 + n*rs1]
+    const float *resid = nullptr;
+    long rs0 = 0, rs1 = 0;
+};
+// C = act(A B + bias) (+ resid) (+ C); gemm_split.hip
+jas_status gemm_split(SplitArgs p, bool a_packed, bool a_bf16, int batch, hipStream_t s);
 
 // General strided GEMM (see jas_gemm in jasmine_hip.h).
 jas_status gemm_general(int M, int N, int K, const void *A, long as0, long as1, const float *B, long bs0, long bs1,

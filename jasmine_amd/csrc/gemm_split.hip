@@ -1,0 +1,786 @@
+// The GEMM behind mat_dot_t / weight_net_t::forward and the runner's prefill: fp32 products
+// on the bf16 matrix cores.
+//
+// Reference: mat_dot_t::operator() (mat_express_t.hpp:730-736), a scalar triple loop with
+// sequential-k accumulation, reached from weight_net_t::forward (mat_net_t.hpp:38-49).
+//
+// v_mfma_f32_16x16x32_bf16 does 16 times the work of v_mfma_f32_16x16x4_f32 per cycle.  An
+// fp32 number is exactly the sum of three bf16 numbers, x = h + m + l (each the rest rounded
+// to nearest even: 8 significant bits of 24 each, |m| <= 2^-9 |x|, |l| <= 2^-18 |x|), and a
+// product of two bf16 numbers is exact in fp32.  So
+//   a b = hh + (hm + mh) + (mm + hl + lh) + (ml + lm + ll),
+// and the six products of the first three groups leave out at most 2^-26 |a b| -- a quarter
+// of the rounding of one fp32 multiplication.  All six accumulate in fp32, the small ones
+// first; six MFMAs take 96 cycles where the fp32 ones take 256.  Weights stored as bf16 are
+// their own h, and three products are exact.
+//
+// The split happens once per element and workgroup, between the global load and LDS: slabs
+// of 32 k are loaded to registers a slab ahead, split, and written to LDS as three planes
+// of bf16 in MFMA operand order, so that every fragment read is one ds_read_b128.  (Small
+// products skip LDS: gemm_split_k_kernel.)
+//
+// Lane l of a wave (r16 = l % 16, g = l / 16) holds slots j = 0..7 of row r16 in both
+// operands: k = 4 g + j for j < 4 and 16 + 4 g + j - 4 above -- a permutation of the slab's k
+// applied to A and B alike, and the one the packed weight layouts already have.
+//
+// Numbers outside the split's range.  Infinities, NaN and magnitudes that round to infinity
+// in bf16 make the six-product sum non-finite.  Magnitudes below 2^-110 lose the bits of m and
+// l under bf16's smallest step: at most 2^-134 per element, so an error of at most
+// K 2^-134 (max|A| + max|B|) in a sum -- more than 2^-24 of it only if the sum is below
+// K 2^-110 (max|A| + max|B|).  Sums that are non-finite or that small (and not zero) are
+// computed again in fp32 arithmetic (SplitRange).
+#include "gemm.hpp"
+
+#include <type_traits>
+#include <utility>
+
+namespace jas {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // rows need not be aligned
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// The three planes of eight fp32 values (slots 0..7 of a lane).  Each residual is one
+// v_dot2_f32_bf16 of the packed pair with (-1, 0) or (0, -1): x - h, exact, without unpacking
+// h (7 instructions per pair; widening and subtracting took 11).  The two constants stay in
+// registers: given -1.0 as an inline constant the instruction takes it as an fp32 pattern.
+// Exact for every x with 2^-110 <= |x| that does not round to infinity in bf16 (checked over
+// random bit patterns of every exponent).
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4 &h, u32x4 &m, u32x4 &l)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    unsigned c0 = 0x0000bf80u, c1 = 0xbf800000u;  // bf16 (-1, 0) and (0, -1)
+    asm("" : "+s"(c0));
+    asm("" : "+s"(c1));
+    const bf16x2 m0 = __builtin_bit_cast(bf16x2, c0), m1 = __builtin_bit_cast(bf16x2, c1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const bf16x2 a = {(__bf16)x[2 * j], (__bf16)x[2 * j + 1]};
+        const float r0 = __builtin_amdgcn_fdot2_f32_bf16(a, m0, x[2 * j], false);
+        const float r1 = __builtin_amdgcn_fdot2_f32_bf16(a, m1, x[2 * j + 1], false);
+        const bf16x2 b = {(__bf16)r0, (__bf16)r1};
+        const float q0 = __builtin_amdgcn_fdot2_f32_bf16(b, m0, r0, false);
+        const float q1 = __builtin_amdgcn_fdot2_f32_bf16(b, m1, r1, false);
+        h[j] = __builtin_bit_cast(unsigned, a);
+        m[j] = __builtin_bit_cast(unsigned, b);
+        l[j] = __builtin_bit_cast(unsigned, bf16x2{(__bf16)q0, (__bf16)q1});  // exact: at most 8 significant bits
+    }
+}
+
+// largest magnitude of the operand values a lane has split
+__device__ __forceinline__ void track_max(float &mx, const float (&x)[8])
+{
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x[j]), "v"(x[j + 1]));
+}
+
+// whether a six-product sum needs fp32 arithmetic: non-finite, or nonzero and below the bound
+struct SplitRange {
+    float small;
+    __device__ __forceinline__ SplitRange(float largest, int K) : small(2.f * (float)K * 0x1p-110f * largest) {}
+    __device__ __forceinline__ bool outside(float v) const
+    {
+        return !(fabsf(v) <= 3.4028234663852886e38f) || (fabsf(v) < small && v != 0.f);
+    }
+};
+
+// One operand X(o, k) of a workgroup: its T x 32 slabs from memory to registers to LDS.
+// A wave moves units of 16 rows (32 outer-contiguous ones); unit u belongs to wave u % NW.
+template <int MODE, int T, int NW>
+struct SplitLoader {
+    static constexpr int OW = MODE == SM_OC ? 32 : 16, UNITS = T / OW, UPW = (UNITS + NW - 1) / NW;
+    static constexpr int NR = MODE == SM_OC ? 16 : MODE == SM_PKB ? 4 : 8;
+    static constexpr int PL = MODE == SM_PKB ? 1 : 3, NB = T / 16;  // planes, 16-row blocks
+    typedef float regs_t[UPW][NR];
+
+    const float *X;
+    long so, sk;
+    int K, Olim;
+    int o[UPW], ou[UPW];    // this lane's (first) outer index, unclamped; its unit's first
+    const float *base[UPW]; // its address at k = 4 g (packed: the tile array)
+    long rt[UPW], RG;       // packed: row tile, row tiles
+
+    __device__ __forceinline__ static bool mine(int w, int q) { return UNITS % NW == 0 || w + q * NW < UNITS; }
+
+    __device__ __forceinline__ void init(const float *X_, const float *X2, long so_, long sk_, int o0, int Olim_, int K_,
+                                         int w, int lane)
+    {
+        X = X_, so = so_, sk = sk_, K = K_, Olim = Olim_;
+        const int i = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int q = 0; q < UPW; ++q) {
+            const int u = w + q * NW;
+            if constexpr (MODE == SM_PK || MODE == SM_PKB) {
+                RG = (Olim + 15) >> 4;
+                long t = min((long)(o0 >> 4) + u, RG - 1);
+                const float *Xm = X;
+                if (X2) {  // SwiGLU: virtual row tile 2f is gate tile f, 2f + 1 up tile f
+                    Xm = t & 1 ? X2 : X;
+                    t >>= 1;
+                    RG >>= 1;
+                }
+                rt[q] = t;
+                base[q] = Xm;
+            } else if constexpr (MODE == SM_OC) {
+                ou[q] = o0 + 32 * u;
+                o[q] = ou[q] + 2 * i;
+                base[q] = X + min(o[q], max(Olim - 2, 0)) + 4 * g * sk;
+            } else {
+                o[q] = min(o0 + 16 * u + i, Olim - 1);
+                base[q] = X + o[q] * so + 4 * g * sk;
+            }
+        }
+    }
+
+    // slab [k0, k0 + 32), inside K (packed bf16: inside K padded to 32)
+    __device__ __forceinline__ void load(regs_t &r, int k0, int w, int lane) const
+    {
+#pragma unroll
+        for (int q = 0; q < UPW; ++q) {
+            if (!mine(w, q)) continue;
+            if constexpr (MODE == SM_KC) {
+                const f32x4u a = *(const f32x4u *)(base[q] + k0), b = *(const f32x4u *)(base[q] + k0 + 16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[q][e] = a[e], r[q][4 + e] = b[e];
+            } else if constexpr (MODE == SM_OC) {
+                if (ou[q] + 32 <= Olim) {  // whole unit inside (wave-uniform)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const f32x2u v = *(const f32x2u *)(base[q] + (long)(k0 + j + (j < 4 ? 0 : 12)) * sk);
+                        r[q][2 * j] = v[0], r[q][2 * j + 1] = v[1];
+                    }
+                } else {
+                    load_edge(r, q, k0, lane);
+                }
+            } else if constexpr (MODE == SM_GEN) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) r[q][j] = base[q][(long)(k0 + j + (j < 4 ? 0 : 12)) * sk];
+            } else if constexpr (MODE == SM_PK) {
+                const int kb = k0 >> 4;
+                const floatx4 a = *(const floatx4 *)(base[q] + weight_tile_offset(rt[q], kb, K >> 4, RG) + lane * 4);
+                const floatx4 b = *(const floatx4 *)(base[q] + weight_tile_offset(rt[q], kb + 1, K >> 4, RG) + lane * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[q][e] = a[e], r[q][4 + e] = b[e];
+            } else {
+                const floatx4 a = *(const floatx4 *)((const uint16_t *)(const void *)base[q] +
+                                                     weight_tile_offset_b(rt[q], k0 >> 5, k32_of(K), RG) + lane * 8);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[q][e] = a[e];
+            }
+        }
+    }
+
+    // outer-contiguous unit that crosses the last row, or the last, partial slab: one element
+    // at a time, rows clamped, zeros from K on
+    __device__ __forceinline__ void load_edge(regs_t &r, int q, int k0, int lane) const
+    {
+        const int g = lane >> 4;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = k0 + 4 * g + j + (j < 4 ? 0 : 12), kc = k < K ? k : 0;
+            if constexpr (MODE == SM_OC) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const float v = X[min(o[q] + e, Olim - 1) + kc * sk];
+                    r[q][2 * j + e] = k < K ? v : 0.f;
+                }
+            } else {
+                const float v = X[o[q] * so + kc * sk];
+                r[q][j] = k < K ? v : 0.f;
+            }
+        }
+    }
+
+    __device__ __forceinline__ void load_tail(regs_t &r, int k0, int w, int lane) const
+    {
+        if constexpr (MODE == SM_PKB) {  // zero-padded to 32
+            load(r, k0, w, lane);
+        } else {
+#pragma unroll
+            for (int q = 0; q < UPW; ++q) {
+                if (!mine(w, q)) continue;
+                if constexpr (MODE == SM_PK) {  // K % 16 == 0: the first half slab exists
+                    const floatx4 a = *(const floatx4 *)(base[q] + weight_tile_offset(rt[q], k0 >> 4, K >> 4, RG) + lane * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) r[q][e] = a[e], r[q][4 + e] = 0.f;
+                } else {
+                    load_edge(r, q, k0, lane);
+                }
+            }
+        }
+    }
+
+    // operand registers of this lane for its q-th unit (K-contiguous, general or packed)
+    __device__ __forceinline__ static void planes(const regs_t &r, int q, float &mx, bf16x8 (&pl)[PL])
+    {
+        if constexpr (MODE == SM_PKB) {
+            pl[0] = __builtin_bit_cast(bf16x8, floatx4{r[q][0], r[q][1], r[q][2], r[q][3]});
+        } else {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = r[q][j];
+            track_max(mx, x);
+            u32x4 h, m, l;
+            split8(x, h, m, l);
+            pl[0] = __builtin_bit_cast(bf16x8, h);
+            pl[1] = __builtin_bit_cast(bf16x8, m);
+            pl[2] = __builtin_bit_cast(bf16x8, l);
+        }
+    }
+
+    // planes of the slab in registers -> LDS: plane pl, 16-row block b, lane slot: [(pl * NB + b)
+    // * 64 + slot].  Lanes 8..15 of a 16-row group swap pairs (slot ^ 1), which keeps the stores
+    // of outer-contiguous units (two rows per lane, every other slot) off each other's banks.
+    __device__ __forceinline__ static int slot_of(int r16, int g) { return (r16 + 16 * g) ^ (r16 >> 3); }
+
+    __device__ __forceinline__ void store(const regs_t &r, u32x4 *lds, int w, int lane, float &mx) const
+    {
+        const int i = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int q = 0; q < UPW; ++q) {
+            if (!mine(w, q)) continue;
+            const int u = w + q * NW;
+            if constexpr (MODE == SM_PKB) {
+                lds[u * 64 + slot_of(i, g)] = __builtin_bit_cast(u32x4, floatx4{r[q][0], r[q][1], r[q][2], r[q][3]});
+            } else {
+                constexpr int R = MODE == SM_OC ? 2 : 1;  // rows per lane
+#pragma unroll
+                for (int e = 0; e < R; ++e) {
+                    float x[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = r[q][R * j + e];
+                    u32x4 h, m, l;
+                    track_max(mx, x);
+                    split8(x, h, m, l);
+                    const int row = MODE == SM_OC ? 2 * (i & 7) + e : i, blk = MODE == SM_OC ? 2 * u + (i >> 3) : u;
+                    u32x4 *d = lds + blk * 64 + slot_of(row, g);
+                    d[0] = h;
+                    d[NB * 64] = m;
+                    d[2 * NB * 64] = l;
+                }
+            }
+        }
+    }
+
+    // one element (the fp32 recomputation); zero from K on
+    __device__ __forceinline__ static float element(const float *X, const float *X2, long so, long sk, int o, int k, int Olim,
+                                                    int K)
+    {
+        if (k >= K) return 0.f;
+        if constexpr (MODE == SM_PK || MODE == SM_PKB) {
+            long RG = (Olim + 15) >> 4;
+            const float *Xm = X;
+            if (X2) {
+                const int t = o >> 4;
+                Xm = t & 1 ? X2 : X;
+                o = (t >> 1) * 16 + (o & 15);
+                RG >>= 1;
+            }
+            if (MODE == SM_PK) return Xm[weight_pack_offset(o, k, K, RG)];
+            return bf16_to_f32(((const uint16_t *)(const void *)Xm)[weight_pack_offset_b(o, k, K, RG)]);
+        }
+        return X[o * so + k * sk];
+    }
+};
+
+// Workgroup ids are remapped so that each of the 8 XCDs (ids go round-robin over them)
+// works on a contiguous range of tiles, walked 4 tile rows at a time: the A rows and B
+// columns its workgroups share stay in that XCD's L2.
+__device__ __forceinline__ void tile_of_workgroup(int &bx, int &by)
+{
+    constexpr int XG = 4;
+    const int gx = gridDim.x, nt = gx * gridDim.y, per = nt / 8;
+    const int id = blockIdx.y * gx + blockIdx.x;
+    // a permutation of the ids: the first 8 * per go XCD-contiguous, the rest stay
+    const int lid = id < 8 * per ? (id % 8) * per + id / 8 : id;
+    const int grp = lid / (XG * gx), gy0 = grp * XG, rows = min(XG, (int)gridDim.y - gy0);
+    const int in = lid - grp * XG * gx;
+    by = gy0 + in % rows;
+    bx = in / rows;
+}
+
+// What the plain epilogue adds to output rows m .. m + 3 of column n: bias and residual (rows
+// past M: the last row's, not stored).
+struct EpiOperands {
+    float bias[4], resid[4];
+    __device__ __forceinline__ void load(const SplitArgs &p, const float *b, int m, int n)
+    {
+        const int mc = min(m, p.M - 1), nc = min(n, p.N - 1);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int mr = min(mc + r, p.M - 1);
+            bias[r] = b ? b[p.bias_mode == 1 ? mr : nc] : 0.f;
+            resid[r] = p.resid ? p.resid[(long)mr * p.rs0 + (long)nc * p.rs1] : 0.f;
+        }
+    }
+};
+
+// Output rows m .. m + 3, column n, from their sums a (SwiGLU: the gate sums, u the up sums of
+// the same outputs; m counts gate and up rows in alternating tiles of 16).
+__device__ __forceinline__ void split_epilogue(const SplitArgs &p, float *C, const float *bias, const EpiOperands &eo, int m,
+                                               int n, floatx4 a, floatx4 u)
+{
+    if (n >= p.N || m >= p.M) return;
+    if (p.fz.mode == FZ_SWIGLU) {
+        const int f = (m >> 5) * 16 + (m & 15);  // output feature of this lane's first row
+        *(float4 *)(C + f + (long)n * p.cs1) =
+            make_float4(silu_f(a[0]) * u[0], silu_f(a[1]) * u[1], silu_f(a[2]) * u[2], silu_f(a[3]) * u[3]);
+        return;
+    }
+    if (p.fz.mode == FZ_QKV) {
+        // rows [0, d) q, [d, 2d) k, [2d, 3d) v of token n: bias, rotary on q and k (pairs
+        // (2i, 2i+1) of a head are (0, 1) and (2, 3) here), the row, and k / v into the KV
+        // cache at the token's position
+        const PrefillFused &zf = p.fz;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = bias ? a[r] + bias[m + r] : a[r];
+        const int sec = m / zf.d, e = m % zf.dh, hh = (m % zf.d) / zf.dh;
+        const int t = zf.pos[n];
+        if (zf.rope && sec < 2) {
+#pragma unroll
+            for (int pr = 0; pr < 2; ++pr) {
+                const double2 cs = zf.rope_tab[(long)t * (zf.dh / 2) + (e >> 1) + pr];
+                const float x0 = v[2 * pr], x1 = v[2 * pr + 1];
+                v[2 * pr] = (float)(x0 * cs.x - x1 * cs.y);
+                v[2 * pr + 1] = (float)(x0 * cs.y + x1 * cs.x);
+            }
+        }
+        *(float4 *)(C + m + (long)n * p.cs1) = make_float4(v[0], v[1], v[2], v[3]);
+        if (sec >= 1) {
+            const int bseq = n / zf.P;
+            const long dst = (((long)bseq * zf.H + hh) * zf.ctx + t) * zf.dh + e;
+            *(float4 *)((sec == 1 ? zf.kc : zf.vc) + dst) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+        return;
+    }
+    const int nv = min(4, p.M - m);
+    float *cp = C + (long)m * p.cs0 + (long)n * p.cs1;
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float x = a[r];
+        if (bias) x = x + eo.bias[r];
+        x = apply_act(x, p.act);
+        if (p.resid) x = x + eo.resid[r];
+        v[r] = p.accumulate ? cp[min(r, nv - 1) * p.cs0] + x : x;
+    }
+    if (p.cs0 == 1 && nv == 4) {
+        *(f32x4u *)cp = f32x4u{v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r < nv) cp[r * p.cs0] = v[r];
+    }
+}
+
+// Large products.  TM x TN tile, NW waves in a WGM x (NW / WGM) grid, two slabs of LDS.  A
+// workgroup splits each element once; per slab and CU a 256 x 128 tile needs 3072 cycles of
+// matrix core, about 900 of vector ALU, 2100 of LDS.  MI355X, 4096^3: 1083 us on the fp32
+// matrix cores (127 TFLOP/s), 690 us here (199 TFLOP/s of fp32 products, 1.2 PFLOP/s of bf16
+// ones, the rate a plain bf16 product of this size reaches).
+template <int AM, int BM, int TM, int TN, int NW, int WGM>
+__global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs p)
+{
+    constexpr int WGN = NW / WGM, NBI = TM / WGM / 16, NBJ = TN / WGN / 16;
+    using LA = SplitLoader<AM, TM, NW>;
+    using LB = SplitLoader<BM, TN, NW>;
+    constexpr int PA = LA::PL, SA = PA * TM * 4, SB = 3 * TN * 4;  // 16-byte units per stage
+    static_assert(LB::PL == 3, "B is fp32");
+    __shared__ u32x4 lds[2 * (SA + SB)];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = w / WGN, wn = w % WGN, r16 = lane & 15, g = lane >> 4;
+
+    int bx, by;
+    tile_of_workgroup(bx, by);
+    const int m0 = by * TM, n0 = bx * TN;
+    const long bz = blockIdx.z;
+    const float *A = p.A + bz * p.abs_;
+    const float *B = p.B + bz * p.bbs;
+    const int K = p.K, nk = K / 32;
+
+    LA la;
+    LB lb;
+    const int wb = NW - 1 - w;  // B's units start from the last wave: small tiles use all waves
+    la.init(A, p.fz.A2, p.as0, p.as1, m0, p.M, K, w, lane);
+    lb.init(B, nullptr, p.bs1, p.bs0, n0, p.N, K, wb, lane);
+
+    floatx4 acc[NBI][NBJ];
+#pragma unroll
+    for (int i = 0; i < NBI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int rslot = LA::slot_of(r16, g);
+    auto compute = [&](const u32x4 *sa) {
+        const u32x4 *pa = sa + wm * NBI * 64 + rslot, *pb = sa + SA + wn * NBJ * 64 + rslot;
+        bf16x8 b[NBJ][3];
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl) b[j][pl] = __builtin_bit_cast(bf16x8, pb[(pl * LB::NB + j) * 64]);
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+            bf16x8 a[PA];
+#pragma unroll
+            for (int pl = 0; pl < PA; ++pl) a[pl] = __builtin_bit_cast(bf16x8, pa[(pl * LA::NB + i) * 64]);
+            // small products first; the NBJ accumulators innermost
+            auto mul = [&](int ia, int ib) {
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[j][ib], acc[i][j], 0, 0, 0);
+            };
+            if constexpr (PA == 3) {
+                mul(2, 0);
+                mul(0, 2);
+                mul(1, 1);
+                mul(1, 0);
+                mul(0, 1);
+                mul(0, 0);
+            } else {
+                mul(0, 0);
+                mul(0, 1);
+                mul(0, 2);
+            }
+        }
+    };
+
+    float mx = 0.f;  // largest magnitude this thread has staged
+    typename LA::regs_t ra;
+    typename LB::regs_t rb;
+    auto fetch = [&](int k0) {
+        la.load(ra, k0, w, lane);
+        lb.load(rb, k0, wb, lane);
+    };
+    // Slab s goes to stage s % 2, which was last read two slabs ago, before the barrier of the
+    // slab in between: one barrier per slab.  The loads of the next slab are issued whether or
+    // not it exists (past the last one: the last again), so the wait counts do not depend on
+    // the path.
+    auto step = [&](int s, bool more) {
+        u32x4 *sa = lds + (s & 1) * (SA + SB);
+        la.store(ra, sa, w, lane, mx);
+        lb.store(rb, sa + SA, wb, lane, mx);
+        if (more) fetch(min(s + 1, nk - 1) * 32);
+        __syncthreads();
+        compute(sa);
+    };
+    if (nk > 0) fetch(0);
+    for (int s = 0; s < nk; ++s) step(s, true);
+    if (nk * 32 < K) {  // partial last slab
+        la.load_tail(ra, nk * 32, w, lane);
+        lb.load_tail(rb, nk * 32, wb, lane);
+        step(nk, false);
+    }
+
+    // a sum outside the split's range anywhere in the tile: compute the tile again in fp32
+    __shared__ float smax[NW];
+    mx = wave_max(mx);
+    if (lane == 0) smax[w] = mx;
+    __syncthreads();
+    float largest = smax[0];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) largest = fmaxf(largest, smax[k]);
+    const SplitRange range(largest, K);
+    bool redo = false;
+#pragma unroll
+    for (int i = 0; i < NBI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) redo |= range.outside(acc[i][j][r]);
+    if (__syncthreads_or(redo)) {
+#pragma unroll
+        for (int i = 0; i < NBI; ++i)
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int k = g; k < K + g; k += 4) {
+            float av[NBI], bv[NBJ];
+#pragma unroll
+            for (int i = 0; i < NBI; ++i)
+                av[i] = LA::element(A, p.fz.A2, p.as0, p.as1, min(m0 + (wm * NBI + i) * 16 + r16, p.M - 1), k, p.M, K);
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j)
+                bv[j] = LB::element(B, nullptr, p.bs1, p.bs0, min(n0 + (wn * NBJ + j) * 16 + r16, p.N - 1), k, p.N, K);
+#pragma unroll
+            for (int i = 0; i < NBI; ++i)
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    // epilogue: block (i, j) of a lane holds rows 4 g .. 4 g + 3, column r16
+    float *C = p.C + bz * p.cbs;
+    const float *bias = p.bias ? p.bias + bz * p.biasbs : nullptr;
+    const int mw = m0 + wm * NBI * 16 + 4 * g, nw = n0 + wn * NBJ * 16 + r16;
+    if (p.fz.mode == FZ_SWIGLU) {
+#pragma unroll
+        for (int i = 0; i + 1 < NBI; i += 2)
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j)
+                split_epilogue(p, C, bias, EpiOperands{}, mw + 16 * i, nw + 16 * j, acc[i][j], acc[i + 1][j]);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < NBI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) {
+            EpiOperands eo;
+            eo.load(p, bias, mw + 16 * i, nw + 16 * j);
+            split_epilogue(p, C, bias, eo, mw + 16 * i, nw + 16 * j, acc[i][j], acc[i][j]);
+        }
+}
+
+// Small products: a workgroup's tile is 16 NBI x 16 NBJ, and its NW waves split K -- wave w
+// takes slabs w, w + NW, ... and holds the whole tile.  Operands go from memory straight to
+// the lanes that need them (no LDS, no barrier in the loop), so a short K is about one memory
+// round trip; the waves' sums meet in LDS and are added in wave order.
+template <int AM, int BM, int NBI, int NBJ, int NW, int PD>
+__global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArgs p)
+{
+    constexpr int TM = 16 * NBI, TN = 16 * NBJ, NBLK = NBI * NBJ;
+    using LA = SplitLoader<AM, TM, 1>;
+    using LB = SplitLoader<BM, TN, 1>;
+    constexpr int PA = LA::PL;
+    __shared__ floatx4 red[NW][NBLK][64];
+    __shared__ float smax[NW];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    int bx, by;
+    tile_of_workgroup(bx, by);
+    const int m0 = by * TM, n0 = bx * TN;
+    const long bz = blockIdx.z;
+    const float *A = p.A + bz * p.abs_;
+    const float *B = p.B + bz * p.bbs;
+    const int K = p.K;
+
+    LA la;
+    LB lb;
+    la.init(A, p.fz.A2, p.as0, p.as1, m0, p.M, K, 0, lane);
+    lb.init(B, nullptr, p.bs1, p.bs0, n0, p.N, K, 0, lane);
+    // this wave's first output block; its bias and residual are requested with the operands
+    const float *bias = p.bias ? p.bias + bz * p.biasbs : nullptr;
+    EpiOperands eo;
+    if (w < NBLK) eo.load(p, bias, m0 + 16 * (w / NBJ) + 4 * g, n0 + 16 * (w % NBJ) + r16);
+    floatx4 acc[NBI][NBJ];
+#pragma unroll
+    for (int i = 0; i < NBI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float mx = 0.f;
+    auto compute = [&](const typename LA::regs_t &ra, const typename LB::regs_t &rb) {
+        bf16x8 b[NBJ][3];
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) LB::planes(rb, j, mx, b[j]);
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+            bf16x8 a[PA];
+            LA::planes(ra, i, mx, a);
+            auto mul = [&](int ia, int ib) {
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[j][ib], acc[i][j], 0, 0, 0);
+            };
+            if constexpr (PA == 3) {
+                mul(2, 0);
+                mul(0, 2);
+                mul(1, 1);
+                mul(1, 0);
+                mul(0, 1);
+                mul(0, 0);
+            } else {
+                mul(0, 0);
+                mul(0, 1);
+                mul(0, 2);
+            }
+        }
+    };
+    const int nk = (K + 31) / 32;  // slabs; the last one may be partial
+    auto fetch = [&](int s, typename LA::regs_t &xa, typename LB::regs_t &xb) {
+        if (s * 32 + 32 <= K) {
+            la.load(xa, s * 32, 0, lane);
+            lb.load(xb, s * 32, 0, lane);
+        } else {
+            la.load_tail(xa, s * 32, 0, lane);
+            lb.load_tail(xb, s * 32, 0, lane);
+        }
+    };
+    if constexpr (PD == 0) {
+        // The next slab's operands are in flight while one is multiplied, then move over: one
+        // copy of the arithmetic in the code.  A short product executes it once or twice per
+        // wave, and fetching unrolled copies costs more than the moves (512 x 512 x 512: 8.0 us
+        // unrolled, 7.0 us so).
+        typename LA::regs_t ra, na;
+        typename LB::regs_t rb, nb;
+        if (w < nk) fetch(w, ra, rb);
+#pragma unroll 1
+        for (int s = w; s < nk; s += NW) {
+            if (s + NW < nk) fetch(s + NW, na, nb);
+            compute(ra, rb);
+#pragma unroll
+            for (int q = 0; q < LA::UPW; ++q)
+#pragma unroll
+                for (int e = 0; e < LA::NR; ++e) ra[q][e] = na[q][e];
+#pragma unroll
+            for (int q = 0; q < LB::UPW; ++q)
+#pragma unroll
+                for (int e = 0; e < LB::NR; ++e) rb[q][e] = nb[q][e];
+        }
+    } else {
+        // PD slabs of registers in flight, the loop unrolled over them; past the wave's last
+        // whole slab the last one is loaded again (path-independent wait counts)
+        constexpr int R = PD > 0 ? PD : 1;
+        typename LA::regs_t ra[R];
+        typename LB::regs_t rb[R];
+        const int nf = K / 32, ns = w < nf ? (nf - w + NW - 1) / NW : 0, kl = (w + (ns - 1) * NW) * 32;
+        auto refill = [&](int u, int t) {
+            const int k0 = min((w + t * NW) * 32, kl);
+            la.load(ra[u], k0, 0, lane);
+            lb.load(rb[u], k0, 0, lane);
+        };
+        if (ns > 0) {
+#pragma unroll
+            for (int u = 0; u < R; ++u) refill(u, u);
+        }
+        int t = 0;
+        for (; t + R <= ns; t += R) {
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                compute(ra[u], rb[u]);
+                refill(u, t + u + R);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < R - 1; ++u)
+            if (t + u < ns) compute(ra[u], rb[u]);
+        if (nf < nk && w == nf % NW) {
+            fetch(nf, ra[0], rb[0]);
+            compute(ra[0], rb[0]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NBI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) red[w][i * NBJ + j][lane] = acc[i][j];
+    mx = wave_max(mx);
+    if (lane == 0) smax[w] = mx;
+    __syncthreads();
+    float largest = smax[0];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) largest = fmaxf(largest, smax[k]);
+    const SplitRange range(largest, K);
+    float *C = p.C + bz * p.cbs;
+    const bool pairs = p.fz.mode == FZ_SWIGLU;  // gate block i with up block i + 1
+    const int n_items = pairs ? NBLK / 2 : NBLK;
+    for (int b = w; b < n_items; b += NW) {
+        const int i = pairs ? 2 * (b / NBJ) : b / NBJ, j = b % NBJ;
+        const int m = m0 + 16 * i + 4 * g, n = n0 + 16 * j + r16;
+        auto total = [&](int ii) {
+            floatx4 v = red[0][ii * NBJ + j][lane];
+#pragma unroll
+            for (int k = 1; k < NW; ++k) v += red[k][ii * NBJ + j][lane];
+            bool redo = false;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) redo |= range.outside(v[r]);
+            if (redo) {  // this lane's four sums again, in fp32
+                const int nc = min(n, p.N - 1);
+                floatx4 f = floatx4{0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < K; ++k) {
+                    const float bk = LB::element(B, nullptr, p.bs1, p.bs0, nc, k, p.N, K);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        f[r] = __builtin_fmaf(LA::element(A, p.fz.A2, p.as0, p.as1, min(m0 + 16 * ii + 4 * g + r, p.M - 1), k,
+                                                          p.M, K),
+                                              bk, f[r]);
+                }
+                v = f;
+            }
+            return v;
+        };
+        if (b != w) eo.load(p, bias, m, n);
+        const floatx4 v = total(i);
+        split_epilogue(p, C, bias, eo, m, n, v, pairs ? total(min(i + 1, NBI - 1)) : v);
+    }
+}
+
+template <int AM, int BM, int TM, int TN, int NW, int WGM>
+static void launch_tile(const SplitArgs &p, int batch, hipStream_t s)
+{
+    hipLaunchKernelGGL((gemm_split_kernel<AM, BM, TM, TN, NW, WGM>), dim3(ceil_div(p.N, TN), ceil_div(p.M, TM), batch),
+                       dim3(NW * 64), 0, s, p);
+}
+template <int AM, int BM, int NBI, int NBJ, int NW, int PD>
+static void launch_wave_split(const SplitArgs &p, int batch, hipStream_t s)
+{
+    // outer-contiguous operands load element by element here (16 rows of a slab per lane group)
+    constexpr int AD = AM == SM_OC ? (int)SM_GEN : AM, BD = BM == SM_OC ? (int)SM_GEN : BM;
+    hipLaunchKernelGGL((gemm_split_k_kernel<AD, BD, NBI, NBJ, NW, PD>),
+                       dim3(ceil_div(p.N, 16 * NBJ), ceil_div(p.M, 16 * NBI), batch), dim3(NW * 64), 0, s, p);
+}
+
+// Geometry by the number of tiles (256 CUs) and K; MI355X, us per product (M x N x K):
+//   256 x 128 tiles when their rounds over the CUs are at least four fifths full: 12288 x 2048
+//     x 4096 1075 (128 x 64: 1320, 64 x 64: 1250); but 2304 x 4096 x 768, 288 tiles, 166 (123)
+//   128 x 64 for a long K with two tiles per CU: 2048^3 109 (64 x 64: 153, 256 x 128: 175)
+//   64 x 64, four waves on K: 768 x 4096 x 768 and x 3072 138 (128 x 64: 171, 64 x 32: 146)
+//   64 x 32, four waves: 3072 x 509 x 768 28 (64 x 64: 37, 32 x 32: 38); 1024^3 22 (35, 32)
+//   64 x 32, eight waves, when that leaves CUs idle but 32 x 32 would need a second round:
+//     2304 x 100 x 768 12.4 (four waves 13.8, 32 x 32 16.2)
+//   32 x 32, eight waves: 512^3 7.0 (64 x 32: 8.4); four waves for K <= 128 (two slabs or less
+//     per wave: 8 x 192 x 512 x 64 7.0, eight waves 10.6)
+//   32 x 16, eight waves, when 32 x 32 would leave half the CUs idle: 12 GPT-2-small layers of
+//     100 tokens, all products, 880 (32 x 32: 960)
+template <int AM, int BM>
+static void launch_split(const SplitArgs &p, int batch, hipStream_t s)
+{
+    auto tiles = [&](int a, int b) { return (long)ceil_div(p.M, a) * ceil_div(p.N, b) * batch; };
+    const long big = tiles(256, 128);
+    if (big >= 256 && big * 5 >= (big + 255) / 256 * 256 * 4) launch_tile<AM, BM, 256, 128, 8, 4>(p, batch, s);
+    else if (tiles(128, 64) >= 512 && p.K >= 1024) launch_tile<AM, BM, 128, 64, 4, 2>(p, batch, s);
+    else if (tiles(64, 64) >= 768) launch_wave_split<AM, BM, 4, 4, 4, 1>(p, batch, s);
+    else if (p.K <= 128) launch_wave_split<AM, BM, 2, 2, 4, 0>(p, batch, s);
+    else if (tiles(64, 32) >= 256) launch_wave_split<AM, BM, 4, 2, 4, 2>(p, batch, s);
+    else if (tiles(32, 32) > 256) launch_wave_split<AM, BM, 4, 2, 8, 0>(p, batch, s);
+    else if (tiles(32, 32) > 128) launch_wave_split<AM, BM, 2, 2, 8, 0>(p, batch, s);
+    else launch_wave_split<AM, BM, 2, 1, 8, 0>(p, batch, s);
+}
+
+// staging mode of operand X(o, k) = X[o * so + k * sk]
+static int split_mode(long so, long sk) { return sk == 1 ? SM_KC : so == 1 ? SM_OC : SM_GEN; }
+
+jas_status gemm_split(SplitArgs p, bool a_packed, bool a_bf16, int batch, hipStream_t s)
+{
+    int am = a_packed ? (a_bf16 ? SM_PKB : SM_PK) : split_mode(p.as0, p.as1);
+    if (!a_packed && p.cs0 != 1 && p.cs1 == 1) {
+        // row-major C: the transposed product, whose lanes hold four consecutive elements
+        std::swap(p.M, p.N);
+        const float *A = p.A;
+        p.A = p.B, p.B = A;
+        const long a0 = p.as0, a1 = p.as1;
+        p.as0 = p.bs1, p.as1 = p.bs0, p.bs0 = a1, p.bs1 = a0;
+        std::swap(p.abs_, p.bbs);
+        std::swap(p.cs0, p.cs1);
+        std::swap(p.rs0, p.rs1);
+        if (p.bias_mode) p.bias_mode = 3 - p.bias_mode;
+        am = split_mode(p.as0, p.as1);
+    }
+    int bm = split_mode(p.bs1, p.bs0);
+    if (a_packed) {
+        JAS_CHECK(bm == SM_KC, JAS_ERR_INVALID, "gemm: packed weights take K-contiguous activations");
+        if (a_bf16) launch_split<SM_PKB, SM_KC>(p, batch, s);
+        else launch_split<SM_PK, SM_KC>(p, batch, s);
+    } else if (am == SM_GEN || bm == SM_GEN) {
+        launch_split<SM_GEN, SM_GEN>(p, batch, s);
+    } else if (am == SM_KC) {
+        if (bm == SM_KC) launch_split<SM_KC, SM_KC>(p, batch, s);
+        else launch_split<SM_KC, SM_OC>(p, batch, s);
+    } else {
+        if (bm == SM_KC) launch_split<SM_OC, SM_KC>(p, batch, s);
+        else launch_split<SM_OC, SM_OC>(p, batch, s);
+    }
+    JAS_LAUNCH_CHECK();
+    return JAS_OK;
+}
+
+} // namespace jas

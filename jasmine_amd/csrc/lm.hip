@@ -28,10 +28,9 @@ __global__ void prefill_positions_kernel(int32_t *pos, int B, int P)
     if (n < (long)B * P) pos[n] = (int32_t)(n % P);
 }
 
-// copy the k and v sections of the prefill QKV rows into the cache:
-// qkv[(b*P + t)*3d + sec*d + h*dh + e] -> cache[b][h][t][e]
-template <bool KB>
-__global__ void kv_scatter_kernel(const float *__restrict__ qkv, void *kc, void *vc, int B, int P, int H, int dh,
+// copy the k and v sections of the prefill QKV rows into the bf16 cache (round to nearest
+// even): qkv[(b*P + t)*3d + sec*d + h*dh + e] -> cache[b][h][t][e]
+__global__ void kv_scatter_kernel(const float *__restrict__ qkv, uint16_t *kc, uint16_t *vc, int B, int P, int H, int dh,
                                   int ctx)
 {
     long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -46,15 +45,10 @@ __global__ void kv_scatter_kernel(const float *__restrict__ qkv, void *kc, void 
     const float *row = qkv + n * 3L * d;
     long dst = (((long)b * H + h) * ctx + t) * dh + ee;
     const float4 k = *(const float4 *)(row + d + e), v = *(const float4 *)(row + 2 * d + e);
-    if (KB) {  // bf16 cache, round to nearest even
-        *(u32x2 *)((uint16_t *)kc + dst) = u32x2{(uint32_t)f32_to_bf16(k.x) | ((uint32_t)f32_to_bf16(k.y) << 16),
-                                                 (uint32_t)f32_to_bf16(k.z) | ((uint32_t)f32_to_bf16(k.w) << 16)};
-        *(u32x2 *)((uint16_t *)vc + dst) = u32x2{(uint32_t)f32_to_bf16(v.x) | ((uint32_t)f32_to_bf16(v.y) << 16),
-                                                 (uint32_t)f32_to_bf16(v.z) | ((uint32_t)f32_to_bf16(v.w) << 16)};
-    } else {
-        *(float4 *)((float *)kc + dst) = k;
-        *(float4 *)((float *)vc + dst) = v;
-    }
+    *(u32x2 *)(kc + dst) = u32x2{(uint32_t)f32_to_bf16(k.x) | ((uint32_t)f32_to_bf16(k.y) << 16),
+                                 (uint32_t)f32_to_bf16(k.z) | ((uint32_t)f32_to_bf16(k.w) << 16)};
+    *(u32x2 *)(vc + dst) = u32x2{(uint32_t)f32_to_bf16(v.x) | ((uint32_t)f32_to_bf16(v.y) << 16),
+                                 (uint32_t)f32_to_bf16(v.z) | ((uint32_t)f32_to_bf16(v.w) << 16)};
 }
 
 // rotary (cos, sin) per (position, frequency), the QKV epilogue's formula in double
@@ -66,12 +60,6 @@ __global__ void rope_table_kernel(double2 *tab, int ctx, int dh, float theta)
     const int i = (int)(g % hp), p = (int)(g / hp);
     const double a = (double)p * pow((double)theta, -2.0 * i / (double)dh);
     tab[g] = make_double2(cos(a), sin(a));
-}
-
-__global__ void swiglu_kernel(const float *__restrict__ gate, const float *__restrict__ up, float *out, long n)
-{
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = silu_f(gate[i]) * up[i];
 }
 
 // token embedding gather from a packed [V][d] table (GPT-2 ties it to the LM head)
@@ -259,7 +247,7 @@ jas_status ensure_prefill(jas_lm *lm, long tokens)
 {
     if (tokens <= lm->p_tokens) return JAS_OK;
     const jas_lm_config &c = lm->cfg;
-    float **bufs[] = {&lm->pX, &lm->pH, &lm->pQKV, &lm->pATT, &lm->pG, &lm->pU, &lm->pFF};
+    float **bufs[] = {&lm->pX, &lm->pH, &lm->pQKV, &lm->pATT, &lm->pFF};
     for (auto b : bufs) {
         if (*b) JAS_HIP(hipFree(*b));
         *b = nullptr;
@@ -268,8 +256,8 @@ jas_status ensure_prefill(jas_lm *lm, long tokens)
     if (lm->pPos) JAS_HIP(hipFree(lm->pPos));
     const long d = c.d_model, F = c.d_ff;
     size_t sz[] = {(size_t)(tokens * d), (size_t)(tokens * d), (size_t)(tokens * 3 * d), (size_t)(tokens * d),
-                   (size_t)(tokens * F), (size_t)(c.kind == 1 ? tokens * F : 4), (size_t)(c.kind == 1 ? tokens * F : 4)};
-    for (int k = 0; k < 7; ++k) TRY(jas_malloc((void **)bufs[k], sz[k] * sizeof(float)));
+                   (size_t)(tokens * F)};
+    for (int k = 0; k < 5; ++k) TRY(jas_malloc((void **)bufs[k], sz[k] * sizeof(float)));
     TRY(jas_malloc((void **)&lm->pIds, tokens * sizeof(int32_t)));
     TRY(jas_malloc((void **)&lm->pPos, tokens * sizeof(int32_t)));
     lm->p_tokens = tokens;
@@ -548,7 +536,7 @@ jas_status jas_lm_destroy(jas_lm *lm)
     if (lm->stream) (void)hipStreamSynchronize(lm->stream);
     if (lm->graph) (void)hipGraphExecDestroy(lm->graph);
     void *ptrs[] = {lm->amax_v, lm->amax_i, lm->dstate, lm->arena, lm->kc, lm->vc, lm->x, lm->h, lm->q, lm->att, lm->ff, lm->logits, lm->ids, lm->pos,
-                    lm->seqlens, lm->hist, lm->attn_ws, lm->attn_ctr, lm->part, lm->pX, lm->pH, lm->pQKV, lm->pATT, lm->pG, lm->pU, lm->pFF,
+                    lm->seqlens, lm->hist, lm->attn_ws, lm->attn_ctr, lm->part, lm->pX, lm->pH, lm->pQKV, lm->pATT, lm->pFF,
                     lm->pIds, lm->pPos, lm->rope_tab};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -660,29 +648,26 @@ jas_status jas_lm_prefill(jas_lm *lm, int B, int P, const int32_t *h_ids, int32_
         TRY(norm_rows(lm, lm->pX, lm->pH, (int)T, d, l, 1));
         const float *bq = lm->LW("b_qkv", l);
         float *kcl = lm->kv_layer_ptr(lm->kc, l), *vcl = lm->kv_layer_ptr(lm->vc, l);
-        // QKV[n][m] = sum_k w_qkv[m][k] H[n][k] (+ b[m]); weights in the packed layout.  On fp32
-        // weights the GEMM's epilogue also applies the rotary (LLaMA) and writes k and v into
-        // the KV cache; bf16 weights take the GEMM, then the rotary and scatter kernels.
-        DmaFused fq;
-        fq.mode = FZ_QKV;
-        fq.pos = lm->pPos;
-        fq.rope_tab = lm->rope_tab;
-        fq.rope = c.kind == 1;
-        fq.kc = kcl;
-        fq.vc = vcl;
-        fq.kv_bf16 = c.kv_bf16;
-        fq.d = d, fq.dh = dh, fq.H = H, fq.P = P, fq.ctx = c.max_ctx;
-        if (lm->wbf16() || !gemm_prefill_fused(3 * d, (int)T, d, lm->LW("w_qkv", l), lm->pH, lm->pQKV, 3L * d, bq, fq, s)) {
-            TRY(gemm_general(3 * d, (int)T, d, lm->LW("w_qkv", l), d, 1, lm->pH, 1, d, lm->pQKV, 1, 3L * d, bq,
-                             bq ? 1 : 0, JAS_ACT_NONE, 0, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
+        // QKV[n][m] = sum_k w_qkv[m][k] H[n][k] (+ b[m]); weights in the packed layout.  With an
+        // fp32 cache the GEMM's epilogue also applies the rotary (LLaMA) and writes k and v into
+        // the KV cache; a bf16 cache takes the product on the fp32 matrix cores (see
+        // gemm_prefill_fp32), then the rotary and scatter kernels.
+        if (c.kv_bf16) {
+            TRY(gemm_prefill_fp32(3 * d, (int)T, d, lm->LW("w_qkv", l), lm->wbf16(), lm->pH, lm->pQKV, 3L * d, bq, s));
             if (c.kind == 1)  // q and k sections are 2H consecutive heads of each row
                 TRY(jas_rope_llama(lm->pQKV, lm->pPos, (int)T, 2 * H, dh, 3L * d, c.rope_theta, s));
-            if (c.kv_bf16)
-                hipLaunchKernelGGL(kv_scatter_kernel<true>, dim3(ceil_div(T * (d / 4), 256)), dim3(256), 0, s,
-                                   lm->pQKV, kcl, vcl, B, P, H, dh, c.max_ctx);
-            else
-                hipLaunchKernelGGL(kv_scatter_kernel<false>, dim3(ceil_div(T * (d / 4), 256)), dim3(256), 0, s,
-                                   lm->pQKV, kcl, vcl, B, P, H, dh, c.max_ctx);
+            hipLaunchKernelGGL(kv_scatter_kernel, dim3(ceil_div(T * (d / 4), 256)), dim3(256), 0, s, lm->pQKV,
+                               (uint16_t *)kcl, (uint16_t *)vcl, B, P, H, dh, c.max_ctx);
+        } else {
+            PrefillFused fq;
+            fq.mode = FZ_QKV;
+            fq.pos = lm->pPos;
+            fq.rope_tab = lm->rope_tab;
+            fq.rope = c.kind == 1;
+            fq.kc = kcl;
+            fq.vc = vcl;
+            fq.d = d, fq.dh = dh, fq.H = H, fq.P = P, fq.ctx = c.max_ctx;
+            TRY(gemm_prefill_fused(3 * d, (int)T, d, lm->LW("w_qkv", l), lm->wbf16(), lm->pH, lm->pQKV, 3L * d, bq, fq, s));
         }
         // the prompt attends over the keys/values just computed (fp32, in the QKV rows);
         // the cache keeps them for the decode steps (rounded when it is bf16)
@@ -694,24 +679,16 @@ jas_status jas_lm_prefill(jas_lm *lm, int B, int P, const int32_t *h_ids, int32_
                          JAS_ACT_NONE, 1, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
         TRY(norm_rows(lm, lm->pX, lm->pH, (int)T, d, l, 2));
         if (c.kind == 0) {
-            TRY(gemm_general(F, (int)T, d, lm->LW("w_fc", l), d, 1, lm->pH, 1, d, lm->pG, 1, F, lm->LW("b_fc", l), 1,
+            TRY(gemm_general(F, (int)T, d, lm->LW("w_fc", l), d, 1, lm->pH, 1, d, lm->pFF, 1, F, lm->LW("b_fc", l), 1,
                              JAS_ACT_GELU, 0, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
-            TRY(gemm_general(d, (int)T, F, lm->LW("w_proj", l), F, 1, lm->pG, 1, F, lm->pX, 1, d,
+            TRY(gemm_general(d, (int)T, F, lm->LW("w_proj", l), F, 1, lm->pFF, 1, F, lm->pX, 1, d,
                              lm->LW("b_proj", l), 1, JAS_ACT_NONE, 1, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
         } else {
-            // SwiGLU: gate and up in one GEMM whose epilogue writes silu(gate) * up (fp32 weights)
-            DmaFused fs;
+            // SwiGLU: gate and up in one GEMM whose epilogue writes silu(gate) * up
+            PrefillFused fs;
             fs.mode = FZ_SWIGLU;
             fs.A2 = lm->LW("w_up", l);
-            if (lm->wbf16() ||
-                !gemm_prefill_fused(2 * F, (int)T, d, lm->LW("w_gate", l), lm->pH, lm->pFF, F, nullptr, fs, s)) {
-                TRY(gemm_general(F, (int)T, d, lm->LW("w_gate", l), d, 1, lm->pH, 1, d, lm->pG, 1, F, nullptr, 0,
-                                 JAS_ACT_NONE, 0, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
-                TRY(gemm_general(F, (int)T, d, lm->LW("w_up", l), d, 1, lm->pH, 1, d, lm->pU, 1, F, nullptr, 0,
-                                 JAS_ACT_NONE, 0, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
-                hipLaunchKernelGGL(swiglu_kernel, dim3(ceil_div(T * F, 256)), dim3(256), 0, s, lm->pG, lm->pU,
-                                   lm->pFF, T * F);
-            }
+            TRY(gemm_prefill_fused(2 * F, (int)T, d, lm->LW("w_gate", l), lm->wbf16(), lm->pH, lm->pFF, F, nullptr, fs, s));
             TRY(gemm_general(d, (int)T, F, lm->LW("w_down", l), F, 1, lm->pFF, 1, F, lm->pX, 1, d, nullptr, 0,
                              JAS_ACT_NONE, 1, 1, 0, 0, 0, 0, s, true, lm->wbf16()));
         }

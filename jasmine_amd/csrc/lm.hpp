@@ -64,7 +64,7 @@ struct jas_lm {
     int ks_o = 1, ks_d = 1;
     size_t attn_ws_bytes = 0;
     // prefill buffers (grown on demand)
-    float *pX = nullptr, *pH = nullptr, *pQKV = nullptr, *pATT = nullptr, *pG = nullptr, *pU = nullptr, *pFF = nullptr;
+    float *pX = nullptr, *pH = nullptr, *pQKV = nullptr, *pATT = nullptr, *pFF = nullptr;
     int32_t *pIds = nullptr, *pPos = nullptr;
     long p_tokens = 0;
     int B = 0;         // active batch

@@ -484,6 +484,76 @@ def test_gemm_residual(jas, M, N, K, act, rcol, bstride, ccol):
     assert np.array_equal(g_, w + R)
 
 
+# every geometry of launch_split (gemm_split.hip) at its edges: partial tiles in both
+# dimensions, K tails, K of less than a slab, rows that are not 16-byte aligned (odd leading
+# dimensions), general strides (a step of 2 in both dimensions), both orders of C, batches
+@pytest.mark.parametrize("M,N,K,batch", [
+    (4100, 2050, 70, 1),    # 256 x 128, whole rounds
+    (4097, 1023, 1057, 1),  # 128 x 64, long K
+    (1537, 2049, 90, 1),    # 64 x 64
+    (65, 33, 65, 40), (65, 33, 128, 1),  # K <= 128: 32 x 32, four waves
+    (1023, 515, 333, 1),    # 64 x 32, four waves
+    (600, 501, 257, 1),     # 64 x 32, eight waves
+    (333, 450, 300, 1),     # 32 x 32, eight waves
+    (33, 17, 4101, 1), (1, 1, 31, 1), (5, 300, 1, 2)])  # 32 x 16
+@pytest.mark.parametrize("la,lb,lc", [(0, 0, 0), (0, 1, 1), (1, 0, 1), (1, 1, 0), (2, 0, 0), (0, 2, 1)])
+def test_gemm_split_geometries(jas, M, N, K, batch, la, lb, lc):
+    # layout 0: row-major, 1: column-major, 2: every second element of every second row
+    def make(r, c, lay, sid):
+        if lay == 2:
+            buf = normal((batch, 2 * r, 2 * c), 31, sid)
+            return buf, buf[:, ::2, ::2], (4 * c, 2), 4 * r * c
+        buf = normal((batch, r, c) if lay == 0 else (batch, c, r), 31, sid)
+        return buf, buf if lay == 0 else np.swapaxes(buf, 1, 2), (c, 1) if lay == 0 else (1, r), r * c
+
+    Ab, A, (as0, as1), ab = make(M, K, la, 0)
+    Bb, B, (bs0, bs1), bb = make(K, N, lb, 1)
+    Cb, Cv, (cs0, cs1), cb = make(M, N, lc, 2)
+    dA, dB, dC = jas.to_device(Ab), jas.to_device(Bb), jas.to_device(Cb)
+    jas.check(jas.lib.jas_gemm(M, N, K, dA.p, as0, as1, dB.p, bs0, bs1, dC.p, cs0, cs1, None, 0, 0, 0, batch, ab, bb, cb, 0,
+                               None))
+    got = dC.numpy() if lc == 0 else np.swapaxes(dC.numpy(), 1, 2)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    # K products, each with at most one rounding of the running sum (2^-24 of it, below the sum
+    # of magnitudes), and 2^-26 of each product left out by the split
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
+    assert np.all(np.abs(got - want) <= bound + 1e-30), float(np.max(np.abs(got - want) / (bound + 1e-30)))
+
+
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (1024, 4096, 1056), (2048, 1536, 96), (96, 64, 640), (200, 90, 120)])
+def test_gemm_split_range(jas, M, N, K):
+    """Values outside the bf16 split's range: infinities, NaN, magnitudes that round to infinity
+    in bf16, products that overflow, and operands so small that their parts underflow -- each
+    in rows or columns of its own, next to ordinary ones."""
+    A, B = normal((M, K), 32, 0), normal((K, N), 32, 1)
+    A[3, 5], A[7, K - 1], B[2, 9] = np.inf, np.nan, -np.inf
+    B[2, :9], B[2, 10:] = 0.5, 0.5                      # keep 0 * inf out of the other columns
+    A[11] = 0.0
+    A[11, 4] = 3.4e38                                   # rounds to infinity in bf16
+    B[4] = np.where(np.arange(N) % 2, 0.25, -0.5)
+    A[20] = 3e38                                        # overflows against B[:, 30], which sums to 16
+    B[:, 30] = 16.0 / K
+    A[33] *= np.float32(2.0 ** -118)                    # parts below the smallest bf16
+    A[50] *= np.float32(2.0 ** -100)
+    B[:, 40] *= np.float32(2.0 ** -20)
+    dA, dB, dC = jas.to_device(A), jas.to_device(B), jas.DeviceArray((M, N))
+    jas.check(jas.lib.jas_gemm(M, N, K, dA.p, K, 1, dB.p, N, 1, dC.p, N, 1, None, 0, 0, 0, 1, 0, 0, 0, 0, None))
+    got = dC.numpy()
+    with np.errstate(all="ignore"):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        mag = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    assert np.array_equal(np.isnan(got[[3, 7]]), np.isnan(want[[3, 7]]))
+    assert np.array_equal(got[3][np.isinf(want[3])], want[3][np.isinf(want[3])])
+    rows = np.setdiff1d(np.arange(M), [3, 7, 20])
+    g, w, m = got[rows], want[rows], mag[rows]
+    fin = np.isfinite(m)  # the column with -inf: an infinity or NaN everywhere
+    assert np.all(fin[:, np.arange(N) != 9]) and not np.any(np.isfinite(g[:, 9][A[rows, 2] != 0]))
+    # as above; fp32 sums of products of 2^-118 also round at the smallest denormal, 2^-149
+    bound = (K + 2) * (2.0 ** -24 * m[fin] + 2.0 ** -149)
+    assert np.all(np.abs(g[fin] - w[fin]) <= bound), float(np.max(np.abs(g[fin] - w[fin]) / bound))
+    assert np.isinf(got[20, 30]) and got[20, 30] > 0
+
+
 def test_gemm_dma_k_tail_padded_rows(jas):
     """K not a multiple of 4 with 16-byte aligned, padded rows (K-contiguous operands take the
     direct-to-LDS path): the tail slab reads element by element and zero-fills past K."""
