@@ -4,14 +4,14 @@
 // S = Q'K / sqrt(d) matrix, masks j > i to -inf (:58-67), runs hsoftmax and multiplies
 // V P'.  Decoding (test_transformer_t::predict, transformer_test.hpp:194-242) recomputes
 // the whole prefix every step.  Here:
-//  * prefill never materialises S: each workgroup owns 64 queries (16 per wave), streams
-//    64-key K/V tiles through LDS and keeps an online softmax.  The wave computes
-//    S^T = K Q^T on the matrix cores so that the probabilities land in exactly the operand
-//    layout of the second product (O += P V, or O^T += V^T P^T for bf16) -- P never leaves
-//    registers.
+//  * prefill never materialises S: each workgroup owns 64 or 128 queries, streams K/V tiles
+//    through LDS and keeps an online softmax.  The wave computes S^T = K Q^T on the matrix
+//    cores so that the probabilities land in exactly the operand layout of the second product,
+//    O^T += V^T P^T -- P never leaves registers.
 //  * decode splits each (sequence, head)'s keys over workgroups (flash-decoding), each
 //    reading its K/V slice once from HBM, then merges the partial softmaxes by log-sum-exp.
 #include "jas_common.hpp"
+#include "split.hpp"
 
 #include <cfloat>
 #include <atomic>
@@ -21,40 +21,9 @@
 
 namespace jas {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <bool BF16>
-__device__ __forceinline__ float4 load4(const void *base, long idx)
-{
-    if (BF16) {
-        uint2 u = *(const uint2 *)((const uint16_t *)base + idx);
-        return make_float4(bf16_to_f32(u.x & 0xffff), bf16_to_f32(u.x >> 16), bf16_to_f32(u.y & 0xffff),
-                           bf16_to_f32(u.y >> 16));
-    }
-    return *(const float4 *)((const float *)base + idx);
-}
-
-template <bool BF16>
-__device__ __forceinline__ void store4(void *base, long idx, float4 v)
-{
-    if (BF16) {
-        auto cvt = [](float f) -> uint32_t {  // round to nearest even
-            uint32_t u = __float_as_uint(f);
-            if ((u & 0x7fffffff) > 0x7f800000) return 0x7fc0;
-            return (u + 0x7fff + ((u >> 16) & 1)) >> 16;
-        };
-        uint2 o;
-        o.x = cvt(v.x) | (cvt(v.y) << 16);
-        o.y = cvt(v.z) | (cvt(v.w) << 16);
-        *(uint2 *)((uint16_t *)base + idx) = o;
-    } else {
-        *(float4 *)((float *)base + idx) = v;
-    }
 }
 
 struct PrefillArgs {
@@ -64,20 +33,18 @@ struct PrefillArgs {
     int B, H, Sq, Sk;
     float scale_log2;  // scale * log2(e)
     int causal;
-    // key split (non-causal only): work item `split` attends over keys
-    // [split * kchunk, min(Sk, (split + 1) * kchunk)) and writes its unnormalised output with
-    // its row max and row sum to part[split][b*H + h][q][D + 2]; a merge kernel combines them
+    // key split: work item `split` attends over keys [split * kchunk, min(Sk, (split + 1) *
+    // kchunk)) and writes its unnormalised output with its exponent base and row sum to
+    // part[split][b*H + h][q][D + 4] (at D and D + 1); a merge kernel combines them
     int nsplit = 1, kchunk = 0;
     float *part = nullptr;
     // > 0: the CU count of a launch whose workgroups sit two to a CU (see fa_work_item)
     int fold = 0;
 };
 
-// waves per workgroup (16 queries each), measured with the heaviest-first work order: 4 or
-// 16 waves are slower for bf16, and 8 beats 4 for fp32 (by 17 % at D = 128)
+// waves per workgroup of the bf16 kernel (16 queries each), measured with the heaviest-first
+// work order: 4 or 16 waves are slower
 constexpr int FA_WAVES = 8;
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 
 // 2^x on the hardware exp unit (v_exp_f32): results below 2^-126 flush to zero.  Used for
@@ -92,9 +59,6 @@ __device__ __forceinline__ float max_across_rows(float v)
     const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-
-// a 16-byte chunk as a native vector (HIP's uint4 struct defeats register promotion)
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Work item of this workgroup: query blocks in order of decreasing causal cost (the last
 // query block first), then (batch, head).  Workgroups are dispatched in id order, so the
@@ -120,26 +84,25 @@ __device__ __forceinline__ bool fa_work_item(int nqb, int BH, int nsplit, int fo
     return true;
 }
 
-// One workgroup = 64 queries of one (batch, head), 16 per wave.  Key/value tiles of 64
-// rows are double-staged: the global loads of tile t+1 are issued into registers before
-// tile t is computed from LDS, so HBM latency hides behind the matrix work.  Rows past
-// Sk are read clamped (finite data) and masked to probability 0.  fp32: S^T = K Q^T and
-// O += P V on v_mfma_f32_16x16x4_f32.  bf16: S^T = K Q^T and O^T += V^T P^T on
+// bf16 attention.  One workgroup = 16 NW queries of one (batch, head), 16 per wave.  Key/value
+// tiles of 64 rows are double-staged: the global loads of tile t+1 are issued into registers
+// before tile t is computed from LDS, so HBM latency hides behind the matrix work.  Rows past
+// Sk are read clamped (finite data) and masked to probability 0.  S^T = K Q^T and O^T += V^T P^T on
 // v_mfma_f32_16x16x32_bf16 (fp32 accumulate, softmax in fp32, P rounded to bf16 for the
 // second product), so every accumulator entry of a lane belongs to the lane's own query and
 // the rescale needs no cross-lane traffic; the reduction index of each product is permuted
 // identically in both operands so that S lands in the P operand's registers with no shuffle.
-template <int D, bool BF16, int BK, int NW = FA_WAVES>
+template <int D, int BK, int NW = FA_WAVES>
 __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_prefill_kernel(const PrefillArgs p)
 {
     constexpr int FA_NW = NW, FA_BQ = 16 * FA_NW;
     constexpr int NT = 64 * FA_NW;
-    using T = typename std::conditional<BF16, uint16_t, float>::type;
-    constexpr int EPC = 16 / (int)sizeof(T);    // elements per 16-byte chunk
-    constexpr int KLD = D + (BF16 ? 8 : 4);    // padded row strides (elements)
+    using T = uint16_t;
+    constexpr int EPC = 8;                      // elements per 16-byte chunk
+    constexpr int KLD = D + 8;                  // padded row strides (elements)
     // bf16 V rows are read with the transposing ds_read_b64_tr_b16: 16 rows x 4 column chunks
     // per 16 lanes; a 40-dword row stride puts the four rows of a lane quad on disjoint banks
-    constexpr int KLDV = BF16 ? D + 16 : KLD;
+    constexpr int KLDV = D + 16;
     constexpr int CPR = D / EPC;                // 16-byte chunks per key row
     constexpr int NCH = BK * CPR;            // 16-byte chunks per tile and tensor
     constexpr int NLD = (NCH + NT - 1) / NT;    // chunks per thread per tensor and tile
@@ -148,8 +111,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
     static_assert(NCH % NT == 0 || NLD == 1, "tile/thread mismatch");
     // two tile buffers: tile t+1 is written while tile t is read, one barrier per tile
     __shared__ __attribute__((aligned(16))) T Ks[2][BK * KLD];
-    // V row-major [BK][D] like K: the O = P V product reads its operand per key row (fp32:
-    // one float per lane and key; bf16: the LDS transpose read, ds_read_b64_tr_b16)
+    // V row-major [BK][D] like K: the O^T product reads its operand with the LDS transpose read
     __shared__ __attribute__((aligned(16))) T Vt[2][BK * KLDV];
 
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
@@ -203,28 +165,18 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
     floatx4 oacc[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) oacc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // running max (raw score units) and this lane's partial row sum: the lanes g = 0..3 of
-    // one query each sum their own keys; the four partials are combined once at the end
-    float m_run = -INFINITY, l_part = 0.f;
-    // bf16: the row sums come out of the matrix core too (P times a ones operand), already in
+    // the row sums come out of the matrix core too (P times a ones operand), already in
     // the accumulator's query layout -- no per-score adds, no final shuffles
     floatx4 lacc = floatx4{0.f, 0.f, 0.f, 0.f};
     const float sl2 = p.scale_log2;
-    // bf16: the exponent base mb of this lane's query (exponent units, shared by the row's
+    // the exponent base mb of this lane's query (exponent units, shared by the row's
     // four lanes) and this lane's running max of its scores relative to it
     float mb = 0.f, m_lane = -INFINITY;
 
     // Q fragments (B operand of S^T = K Q^T), raw (the scale is applied in the exponent)
-    float4 qf[BF16 ? 1 : NC];
-    bf16x8 qb16[BF16 ? D / 32 : 1];
-    if constexpr (BF16) {
+    bf16x8 qb16[D / 32];
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c)
-            qb16[c] = *(const bf16x8 *)((const uint16_t *)p.Q + qbase + 32 * c + 8 * g);
-    } else {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) qf[c] = *(const float4 *)((const float *)p.Q + qbase + 16 * c + 4 * g);
-    }
+    for (int c = 0; c < D / 32; ++c) qb16[c] = *(const bf16x8 *)((const uint16_t *)p.Q + qbase + 32 * c + 8 * g);
 
 #define FA_LSTORE(BUF, KR, VR)                                                               \
     _Pragma("unroll") for (int it = 0; it < NLD; ++it)                                     \
@@ -232,15 +184,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
         const int idx = tid + it * NT, key = idx / CPR, ch = idx % CPR;                    \
         if (NCH % NT != 0 && idx >= NCH) break;                                            \
         *(u32x4 *)(&Ks[BUF][key * KLD + ch * EPC]) = KR[it];                               \
-        if constexpr (BF16) {                                                                   \
-            *(u32x4 *)(&Vt[BUF][key * KLDV + ch * EPC]) = VR[it];                              \
-        } else { /* fp32 V rows interleaved: element d at (d % 16) * NC + d / 16 */            \
-            _Pragma("unroll") for (int e = 0; e < 4; ++e)                                      \
-            {                                                                                  \
-                const int d = ch * EPC + e;                                                    \
-                Vt[BUF][key * KLDV + (d % 16) * NC + d / 16] = __uint_as_float(VR[it][e]);    \
-            }                                                                                  \
-        }                                                                                      \
+        *(u32x4 *)(&Vt[BUF][key * KLDV + ch * EPC]) = VR[it];                              \
     }
 
     // Pipeline: tile t is computed from LDS buffer t%2 while tile t+1 waits in registers
@@ -263,191 +207,103 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
 
         // S^T tile: lane holds S^T[key = kv0 + 16j + 4g + r][query = qi] (raw scores)
         floatx4 s[NJ];
-        // bf16: the K fragments of the tile are requested first; the V fragments after the
+        // the K fragments of the tile are requested first; the V fragments after the
         // score products have been issued (reusing the K fragments' registers), and their
         // reads complete behind the softmax
-        bf16x8 kfr[BF16 ? NJ : 1][BF16 ? D / 32 : 1];
-        if constexpr (BF16) {
+        bf16x8 kfr[NJ][D / 32];
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int c = 0; c < D / 32; ++c)
-                    kfr[j][c] = *(const bf16x8 *)(Kc + (16 * j + r16) * KLD + 32 * c + 8 * g);
-        }
+            for (int c = 0; c < D / 32; ++c) kfr[j][c] = *(const bf16x8 *)(Kc + (16 * j + r16) * KLD + 32 * c + 8 * g);
         // masking only on tiles that reach past Sk or cross this wave's causal diagonal: key
         // kv0 + 16j + 4g + r is visible iff 16j + r <= lim, one compare per score
         const bool need_mask = kv0 + BK > p.Sk || (p.causal && kv0 + BK - 1 > q0 + shift);
         const int lim = (p.causal ? min(qi + shift, p.Sk - 1) : p.Sk - 1) - kv0 - 4 * g;
-        if constexpr (BF16) {
-            // raw scores; the NJ key blocks are independent accumulators, innermost so that
-            // consecutive matrix ops never wait on each other's result
+        // raw scores; the NJ key blocks are independent accumulators, innermost so that
+        // consecutive matrix ops never wait on each other's result
 #pragma unroll
-            for (int c = 0; c < D / 32; ++c)
+        for (int c = 0; c < D / 32; ++c)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kfr[j][c], qb16[c], c == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : s[j], 0, 0, 0);
-            bf16x8 vfr[NC][NJ / 2];
-            // A operand of O^T = V^T P^T for key block m, head-dim block c: lane (n = l%16, g) needs
-            // V[key][16c + n] for keys 32m + 4g + 0..3 and 32m + 16 + 4g + 0..3.  The transpose
-            // read hands lane n of each 16-lane group element n%4 of the 4-element chunks that
-            // lanes n/4 + 4e address (e = 0..3), so lane i addresses row (key base + i/4),
-            // columns 16c + 4(i%4) .. +3.
-            typedef short s16x4 __attribute__((ext_vector_type(4)));
-            typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+            for (int j = 0; j < NJ; ++j)
+                s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kfr[j][c], qb16[c], c == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : s[j], 0, 0, 0);
+        bf16x8 vfr[NC][NJ / 2];
+        // A operand of O^T = V^T P^T for key block m, head-dim block c: lane (n = l%16, g) needs
+        // V[key][16c + n] for keys 32m + 4g + 0..3 and 32m + 16 + 4g + 0..3.  The transpose
+        // read hands lane n of each 16-lane group element n%4 of the 4-element chunks that
+        // lanes n/4 + 4e address (e = 0..3), so lane i addresses row (key base + i/4),
+        // columns 16c + 4(i%4) .. +3.
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 #pragma unroll
-            for (int c = 0; c < NC; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int m = 0; m < NJ / 2; ++m) {
-                    const uint16_t *v0 = Vc + (32 * m + 4 * g + (r16 >> 2)) * KLDV + 16 * c + 4 * (r16 & 3);
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)v0);
-                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(v0 + 16 * KLDV));
-                    vfr[c][m] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                }
-            if (need_mask) {
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s[j][r] = 16 * j + r <= lim ? s[j][r] : -INFINITY;
+            for (int m = 0; m < NJ / 2; ++m) {
+                const uint16_t *v0 = Vc + (32 * m + 4 * g + (r16 >> 2)) * KLDV + 16 * c + 4 * (r16 & 3);
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)v0);
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(v0 + 16 * KLDV));
+                vfr[c][m] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
-            // exponent units relative to the base: s <- sl2 s - mb (p = 2^s below)
+        if (need_mask) {
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) s[j][r] = __builtin_fmaf(s[j][r], sl2, -mb);
-            // Lazy rescaling with a per-lane test: the base mb moves only when the row's running
-            // max leaves [mb - 64, mb + 8].  Meanwhile p stays below 2^8, numerator and row sum
-            // share the base, and O / l is unchanged.  Each lane tests only its own running max
-            // (taken after the fma: arithmetic results need no NaN canonicalisation before a
-            // max); the row max across the four lanes, and the move itself, are computed only
-            // when some lane trips, which for most inputs happens on no tile at all.  A query
-            // with no visible key keeps -inf maxima.
-            const float m_prev = m_lane;
+                for (int r = 0; r < 4; ++r) s[j][r] = 16 * j + r <= lim ? s[j][r] : -INFINITY;
+        }
+        // exponent units relative to the base: s <- sl2 s - mb (p = 2^s below)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) m_lane = fmaxf(fmaxf(m_lane, fmaxf(s[j][0], s[j][1])), fmaxf(s[j][2], s[j][3]));
-            if (__builtin_amdgcn_ballot_w64(m_lane > 8.f || (m_lane < -64.f && m_lane != -INFINITY))) {
-                const float row_prev = max_across_rows(m_prev), row = max_across_rows(m_lane);
-                if (row > 8.f || (row < -64.f && row != -INFINITY)) {
-                    // nothing accumulated yet (row_prev = -inf): factor 0, not 2^-row, which
-                    // overflows when the base moves far down
-                    const float corr = row_prev == -INFINITY ? 0.f : exp2_fast(-row);
-                    mb += row;
-                    m_lane -= row;
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) s[j] -= row;
+            for (int r = 0; r < 4; ++r) s[j][r] = __builtin_fmaf(s[j][r], sl2, -mb);
+        // Lazy rescaling with a per-lane test: the base mb moves only when the row's running
+        // max leaves [mb - 64, mb + 8].  Meanwhile p stays below 2^8, numerator and row sum
+        // share the base, and O / l is unchanged.  Each lane tests only its own running max
+        // (taken after the fma: arithmetic results need no NaN canonicalisation before a
+        // max); the row max across the four lanes, and the move itself, are computed only
+        // when some lane trips, which for most inputs happens on no tile at all.  A query
+        // with no visible key keeps -inf maxima.
+        const float m_prev = m_lane;
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) oacc[c] *= corr;  // O^T: the lane's own query
-                    lacc *= corr;
-                }
+        for (int j = 0; j < NJ; ++j) m_lane = fmaxf(fmaxf(m_lane, fmaxf(s[j][0], s[j][1])), fmaxf(s[j][2], s[j][3]));
+        if (__builtin_amdgcn_ballot_w64(m_lane > 8.f || (m_lane < -64.f && m_lane != -INFINITY))) {
+            const float row_prev = max_across_rows(m_prev), row = max_across_rows(m_lane);
+            if (row > 8.f || (row < -64.f && row != -INFINITY)) {
+                // nothing accumulated yet (row_prev = -inf): factor 0, not 2^-row, which
+                // overflows when the base moves far down
+                const float corr = row_prev == -INFINITY ? 0.f : exp2_fast(-row);
+                mb += row;
+                m_lane -= row;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) s[j] -= row;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) oacc[c] *= corr;  // O^T: the lane's own query
+                lacc *= corr;
             }
-            // P^T operand for key block m (32 keys): slot t <-> key 32m + 16(t/4) + 4g + t%4,
-            // which are exactly s[2m][t] and s[2m+1][t-4] of this lane
-            bf16x8 pb[NJ / 2];
+        }
+        // P^T operand for key block m (32 keys): slot t <-> key 32m + 16(t/4) + 4g + t%4,
+        // which are exactly s[2m][t] and s[2m+1][t-4] of this lane
+        bf16x8 pb[NJ / 2];
+#pragma unroll
+        for (int m = 0; m < NJ / 2; ++m)
+        {
+            float e[8];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                e[r] = exp2_fast(s[2 * m][r]);
+                e[4 + r] = exp2_fast(s[2 * m + 1][r]);
+            }
+            pb[m] = bf16x8{(__bf16)e[0], (__bf16)e[1], (__bf16)e[2], (__bf16)e[3],
+                           (__bf16)e[4], (__bf16)e[5], (__bf16)e[6], (__bf16)e[7]};
+        }
+        // O^T += V^T P^T; row sums as P^T times a ones operand
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int m = 0; m < NJ / 2; ++m)
-            {
-                float e[8];
+                oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfr[c][m], pb[m], oacc[c], 0, 0, 0);
+        const bf16x8 ones = bf16x8{(__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f,
+                                   (__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    e[r] = exp2_fast(s[2 * m][r]);
-                    e[4 + r] = exp2_fast(s[2 * m + 1][r]);
-                }
-                pb[m] = bf16x8{(__bf16)e[0], (__bf16)e[1], (__bf16)e[2], (__bf16)e[3],
-                               (__bf16)e[4], (__bf16)e[5], (__bf16)e[6], (__bf16)e[7]};
-            }
-            // O^T += V^T P^T; row sums as P^T times a ones operand
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-#pragma unroll
-                for (int m = 0; m < NJ / 2; ++m)
-                    oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfr[c][m], pb[m], oacc[c], 0, 0, 0);
-            const bf16x8 ones = bf16x8{(__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f,
-                                       (__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
-#pragma unroll
-            for (int m = 0; m < NJ / 2; ++m) lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[m], lacc, 0, 0, 0);
-        } else {
-            // raw scores; the NJ key blocks are independent accumulators (j innermost)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) s[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                float4 kf[NJ];
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) kf[j] = *(const float4 *)(Kc + (16 * j + r16) * KLD + 16 * c + 4 * g);
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) s[j] = mfma4(kf[j].x, qf[c].x, s[j]);
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) s[j] = mfma4(kf[j].y, qf[c].y, s[j]);
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) s[j] = mfma4(kf[j].z, qf[c].z, s[j]);
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) s[j] = mfma4(kf[j].w, qf[c].w, s[j]);
-            }
-            if (need_mask) {
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s[j][r] = 16 * j + r <= lim ? s[j][r] : -INFINITY;
-            }
-            float tmax = s[0][0];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = (j == 0 ? 1 : 0); r < 4; ++r) tmax = fmaxf(tmax, s[j][r]);
-            tmax = max_across_rows(tmax);
-            // lazy rescaling: the base m_run moves only when some query's max has grown by
-            // more than 2^8 in exponent units (or was -inf); p = 2^(sl2 (s - m_run)) stays below
-            // 256 meanwhile, and numerator and row sum share the stale base.  A query with
-            // every key masked so far keeps m = -inf and gets p = 0 from the -inf scores.
-            const float m_cand = fmaxf(m_run, tmax);
-            const float m_new = (m_cand - m_run) * sl2 > 8.f ? m_cand : m_run;  // NaN (-inf - -inf): keep
-            const float mb = m_new == -INFINITY ? 0.f : m_new * sl2;
-            const float corr = exp2_fast(m_run * sl2 - mb);  // 1 when kept; 0 from m_run = -inf
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) s[j][r] = exp2_fast(__builtin_fmaf(s[j][r], sl2, -mb));
-            float psum = 0.f;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) psum += (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
-            l_part = l_part * corr + psum;
-            m_run = m_new;
-            if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
-                // oacc[c][r] is query 4g + r (O, not O^T), whose factor lives in lane 4g + r,
-                // the lane that owns that query's scores
-                floatx4 cr;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) cr[r] = __shfl(corr, 4 * g + r, WAVE);
-#pragma unroll
-                for (int c = 0; c < NC; ++c) oacc[c] *= cr;
-            }
-            // O[q][d = 16c + n] += sum_key P[q][key] V[key][d]: in product t of key block j the
-            // lanes of group g contribute key 16j + 4g + t -- their own score s[j][t] as A and
-            // V[16j + 4g + t][16c + n] as B.  The staged V rows are interleaved (element d at
-            // (d % 16) * NC + d / 16), so a lane's NC values for c = 0..NC-1 are adjacent: one
-            // 16-byte LDS read per four of them instead of one read per value
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float *vrow = Vc + (16 * j + 4 * g + t) * KLDV + r16 * NC;
-                    float vv[NC];
-                    if constexpr (NC % 4 == 0) {
-#pragma unroll
-                        for (int c = 0; c < NC; c += 4) {
-                            const float4 f = *(const float4 *)(vrow + c);
-                            vv[c] = f.x, vv[c + 1] = f.y, vv[c + 2] = f.z, vv[c + 3] = f.w;
-                        }
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < NC; c += 2) {
-                            const float2 f = *(const float2 *)(vrow + c);
-                            vv[c] = f.x, vv[c + 1] = f.y;
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) oacc[c] = mfma4(s[j][t], vv[c], oacc[c]);
-                }
-        }
+        for (int m = 0; m < NJ / 2; ++m) lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[m], lacc, 0, 0, 0);
     };
     // step for tile kv0 in LDS buffer BUF: stage tile kv0+BK from (KR, VR) into the other
     // buffer, refill (KR, VR) with tile kv0+3BK, compute, and wait until every wave is done
@@ -467,101 +323,387 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
     }
 #undef FA_STEP
 
-    if constexpr (BF16) {
-        // O^T accumulators: lane holds O[query = q0 + r16][d = 16c + 4g + r], its own query's
-        // row sum in lacc (every entry) and its base in m_run
-        if (qi >= p.Sq) return;
-        if (p.nsplit > 1) {  // unnormalised partial: O, then the row max (raw units) and row sum
-            float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qi) * (D + 2);
+    // O^T accumulators: lane holds O[query = q0 + r16][d = 16c + 4g + r], its own query's
+    // row sum in lacc (every entry) and its base in m_run
+    if (qi >= p.Sq) return;
+    if (p.nsplit > 1) {  // unnormalised partial: O, then the row max (raw units) and row sum
+        float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qi) * (D + 4);
 #pragma unroll
-            for (int c = 0; c < NC; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) row[16 * c + 4 * g + r] = oacc[c][r];
-            if (g == 0) {  // the base in exponent units (-inf: no visible key)
-                row[D] = lacc[0] > 0.f ? mb : -INFINITY;
-                row[D + 1] = lacc[0];
-            }
-            return;
-        }
-        const float inv = lacc[0] > 0.f ? 1.0f / lacc[0] : 0.f;
-        const long orow = (long)b * p.o_sb + (long)h * p.o_sh + (long)qi * p.o_ss;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            uint2 o;
-            o.x = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][0] * inv)) |
-                  ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][1] * inv)) << 16);
-            o.y = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][2] * inv)) |
-                  ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][3] * inv)) << 16);
-            *(uint2 *)((uint16_t *)p.O + orow + 16 * c + 4 * g) = o;
+            for (int r = 0; r < 4; ++r) row[16 * c + 4 * g + r] = oacc[c][r];
+        if (g == 0) {  // the base in exponent units (-inf: no visible key)
+            row[D] = lacc[0] > 0.f ? mb : -INFINITY;
+            row[D + 1] = lacc[0];
         }
         return;
-    } else {
-        float l_run = l_part + __shfl_xor(l_part, 16, WAVE);
-        l_run += __shfl_xor(l_run, 32, WAVE);
-        if (p.nsplit > 1) {  // unnormalised partial: O, then the row max (raw units) and row sum
+    }
+    const float inv = lacc[0] > 0.f ? 1.0f / lacc[0] : 0.f;
+    const long orow = (long)b * p.o_sb + (long)h * p.o_sh + (long)qi * p.o_ss;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float lr = __shfl(l_run, 4 * g + r, WAVE);
-                const float mr = __shfl(m_run, 4 * g + r, WAVE);
-                const int qo = q0 + 4 * g + r;
-                if (qo >= p.Sq) continue;
-                float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qo) * (D + 2);
-#pragma unroll
-                for (int c = 0; c < NC; ++c) row[16 * c + r16] = oacc[c][r];
-                if (r16 == 0) {
-                    row[D] = mr;
-                    row[D + 1] = lr;
-                }
-            }
-            return;
-        }
-        // lane holds O[query = q0 + 4g + r][d = 16c + r16]; 1/l of query 4g + r from lane 4g + r
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float lr = __shfl(l_run, 4 * g + r, WAVE);
-            const int qo = q0 + 4 * g + r;
-            if (qo >= p.Sq) continue;
-            const float inv = lr > 0.f ? 1.0f / lr : 0.f;
-            const long orow = (long)b * p.o_sb + (long)h * p.o_sh + (long)qo * p.o_ss;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) ((float *)p.O)[orow + 16 * c + r16] = oacc[c][r] * inv;
-        }
+    for (int c = 0; c < NC; ++c) {
+        uint2 o;
+        o.x = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][0] * inv)) |
+              ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][1] * inv)) << 16);
+        o.y = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][2] * inv)) |
+              ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][3] * inv)) << 16);
+        *(uint2 *)((uint16_t *)p.O + orow + 16 * c + 4 * g) = o;
     }
 #undef FA_GLOAD
 #undef FA_LSTORE
 }
 
-// Combines the key-split partials of a prefill launch: one thread per (row, head-dim
-// element); O = sum_i 2^((m_i - M) s) O_i / sum_i 2^((m_i - M) s) l_i with M = max_i m_i
-// (s = 1 for bf16 partials, whose m_i are already in exponent units).
-template <bool BF16>
+// One query row in fp32 arithmetic by one wave (flash_split_kernel's rare path): n keys;
+// partial: the unnormalised row, then its exponent base and sum.
+template <int D>
+__device__ __attribute__((noinline)) void attend_row_fp32(const float *q, const float *K, const float *V, long k_ss, int n,
+                                                          float scale_log2, float *row, int partial)
+{
+    const int lane = threadIdx.x & 63;
+    constexpr int E = (D + 63) / 64;  // output elements per lane: lane + 64 e
+    float m = -INFINITY, l = 0.f, acc[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = 0.f;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+        const int nk = min(64, n - k0);
+        float s = -INFINITY;
+        if (lane < nk) {
+            const float *kr = K + (long)(k0 + lane) * k_ss;
+            float d = 0.f;
+            for (int e = 0; e < D; ++e) d = __builtin_fmaf(q[e], kr[e], d);
+            s = d * scale_log2;
+        }
+        const float mx = fmaxf(m, wave_max(s)), base = mx == -INFINITY ? 0.f : mx;
+        const float corr = exp2_fast(m - base), pv = lane < nk ? exp2_fast(s - base) : 0.f;
+        l = l * corr + wave_sum(pv);
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[e] *= corr;
+        for (int k = 0; k < nk; ++k) {
+            const float pk = __shfl(pv, k, WAVE);
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if (lane + 64 * e < D) acc[e] = __builtin_fmaf(pk, V[(long)(k0 + k) * k_ss + lane + 64 * e], acc[e]);
+        }
+        m = mx;
+    }
+    if (partial && lane == 0) row[D] = m, row[D + 1] = l;
+    const float inv = partial ? 1.f : l != 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (lane + 64 * e < D) row[lane + 64 * e] = acc[e] * inv;
+}
+
+// fp32 attention on the bf16 matrix cores: Q, K, V and the probabilities as three-way bf16
+// splits, six products per step (gemm_split.hip), softmax in fp32.  Four waves of NQ x 16
+// queries; K and V tiles of BK keys are split once per workgroup on their way to LDS, where
+// both lie in operand order (one ds_read_b128 per fragment and plane; V is transposed by the
+// lanes that stage it: two d of eight keys each).  S^T = K Q^T and O^T += V^T P^T as in the
+// bf16 form above, with its lazily moved exponent base, so P stays in the lane that made it.
+// One buffer of LDS (48 KB at D = 64): two workgroups per CU cover each other's barriers.
+//
+// What bounds it at D = 64: per wave and tile of 32 queries x 64 keys, 192 MFMAs (3072
+// cycles), about 400 vector instructions (1600) and 48 KB of LDS reads (384 of the CU's
+// cycles).  One 16-query block per wave reads as much LDS for half the products, so NQ = 2
+// where registers allow it (D <= 64) and the launch fills the chip.  MI355X, B 8, H 12,
+// S 1024, D 64, causal: 82.7 us, 156 TFLOP/s (128.8 us on the fp32 matrix cores, whose peak
+// is 157); not causal 134 us, 192 TFLOP/s (210).  D 128, 2 x 32 heads, causal: 108 us (159).
+//
+// Operands outside the split's range (gemm_split.hip) end in a non-finite row or sum, in an
+// output below 2^-108 of its row's weight, or show as magnitudes above 2^90 in Q or K (whose
+// partners could then be small enough to have lost parts that matter); a wave that sees one
+// computes its queries again in fp32.
+template <int D, int NQ, int BK>
+__global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p)
+{
+    constexpr int NW = 4, BQ = 16 * NQ * NW, CD = D / 32, NC = D / 16, NJ = BK / 16, NM = BK / 32;
+    constexpr int UK = NJ * CD, UV = CD * NM;  // staging units: 16 keys x 32 d, 32 d x 32 keys
+    constexpr int KU = (UK + NW - 1) / NW, VU = (UV + NW - 1) / NW;
+    __shared__ u32x4 Kp[3][NJ * CD * 64];
+    __shared__ u32x4 Vp[3][NC * NM * 64];
+    __shared__ int s_large;
+    const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int bh, qb, split;
+    const int nqb = (p.Sq + BQ - 1) / BQ;
+    if (!fa_work_item(nqb, p.B * p.H, p.nsplit, p.fold, bh, qb, split)) return;
+    const int b = bh / p.H, h = bh % p.H, shift = p.Sk - p.Sq;
+    const int q0 = qb * BQ + w * 16 * NQ;
+    const int q_last = min(qb * BQ + BQ - 1, p.Sq - 1);
+    const int k_lo = p.nsplit > 1 ? split * p.kchunk : 0;
+    const int k_end = p.nsplit > 1 ? min(p.Sk, k_lo + p.kchunk) : p.causal ? min(p.Sk, q_last + shift + 1) : p.Sk;
+    const int wave_kend = min(k_end, p.causal ? min(p.Sk, min(q0 + 16 * NQ - 1, p.Sq - 1) + shift + 1) : p.Sk);
+    const float *Kb = (const float *)p.K + (long)b * p.k_sb + (long)h * p.k_sh;
+    const float *Vb = (const float *)p.V + (long)b * p.k_sb + (long)h * p.k_sh;
+    auto slot_of = [](int row, int grp) { return (row + 16 * grp) ^ (row >> 3); };  // as in gemm_split.hip
+    if (tid == 0) s_large = 0;
+
+    // Q planes (B operand): slots j < 4 hold d = 32 c + 4 g + j, j >= 4 d = 32 c + 16 + 4 g + j - 4
+    bf16x8 qf[NQ][CD][3];
+    float qmax = 0.f;
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        const int qq = min(q0 + 16 * a + r16, p.Sq - 1);
+        const float *qr = (const float *)p.Q + (long)b * p.q_sb + (long)h * p.q_sh + (long)qq * p.q_ss;
+#pragma unroll
+        for (int c = 0; c < CD; ++c) {
+            const floatx4 x0 = *(const floatx4 *)(qr + 32 * c + 4 * g), x1 = *(const floatx4 *)(qr + 32 * c + 16 + 4 * g);
+            const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+            u32x4 hh, mm, ll;
+            track_max(qmax, x);
+            split8(x, hh, mm, ll);
+            qf[a][c][0] = __builtin_bit_cast(bf16x8, hh);
+            qf[a][c][1] = __builtin_bit_cast(bf16x8, mm);
+            qf[a][c][2] = __builtin_bit_cast(bf16x8, ll);
+        }
+    }
+
+    // staging: registers of the tile in flight
+    float kr[KU][8], vr[VU][16];
+    auto gload = [&](int kv0) {
+        const bool whole = kv0 + BK <= p.Sk;  // rows past Sk: the last row (finite, masked below)
+#pragma unroll
+        for (int q = 0; q < KU; ++q) {
+            const int u = w + NW * q;
+            if (UK % NW != 0 && u >= UK) continue;
+            const int key = kv0 + 16 * (u / CD) + r16;
+            const float *src = Kb + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss + 32 * (u % CD) + 4 * g;
+            const floatx4 x0 = *(const floatx4 *)src, x1 = *(const floatx4 *)(src + 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kr[q][e] = x0[e], kr[q][4 + e] = x1[e];
+        }
+#pragma unroll
+        for (int q = 0; q < VU; ++q) {
+            const int u = w + NW * q;
+            if (UV % NW != 0 && u >= UV) continue;
+            const int key0 = kv0 + 32 * (u / CD) + 4 * g;
+            const float *src = Vb + 32 * (u % CD) + 2 * r16;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int key = key0 + j + (j < 4 ? 0 : 12);
+                typedef float f32x2 __attribute__((ext_vector_type(2)));
+                const f32x2 x = *(const f32x2 *)(src + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss);
+                vr[q][2 * j] = x[0], vr[q][2 * j + 1] = x[1];
+            }
+        }
+    };
+    float kmax = 0.f;
+    auto lstore = [&]() {
+#pragma unroll
+        for (int q = 0; q < KU; ++q) {
+            const int u = w + NW * q;
+            if (UK % NW != 0 && u >= UK) continue;
+            u32x4 hh, mm, ll;
+            track_max(kmax, kr[q]);
+            split8(kr[q], hh, mm, ll);
+            const int at = u * 64 + slot_of(r16, g);
+            Kp[0][at] = hh, Kp[1][at] = mm, Kp[2][at] = ll;
+        }
+#pragma unroll
+        for (int q = 0; q < VU; ++q) {
+            const int u = w + NW * q;
+            if (UV % NW != 0 && u >= UV) continue;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = vr[q][2 * j + e];
+                u32x4 hh, mm, ll;
+                split8(x, hh, mm, ll);
+                const int blk = 2 * (u % CD) + (r16 >> 3);  // 16-row block of d
+                const int at = (blk * NM + u / CD) * 64 + slot_of(2 * (r16 & 7) + e, g);
+                Vp[0][at] = hh, Vp[1][at] = mm, Vp[2][at] = ll;
+            }
+        }
+    };
+
+    floatx4 oacc[NC][NQ];
+    float l_part[NQ], mb[NQ], m_lane[NQ];  // row sums, exponent base and running max (as above)
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        l_part[a] = 0.f, mb[a] = 0.f, m_lane[a] = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) oacc[c][a] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    const float sl2 = p.scale_log2;
+    const int rslot = slot_of(r16, g);
+    auto frag = [&](const u32x4 *const pl, int blk) { return __builtin_bit_cast(bf16x8, pl[blk * 64 + rslot]); };
+
+    gload(k_lo);
+    for (int kv0 = k_lo; kv0 < k_end; kv0 += BK) {
+        __syncthreads();  // every wave is done with the previous tile
+        lstore();
+        gload(min(kv0 + BK, k_lo + (k_end - k_lo - 1) / BK * BK));  // (past the last tile: it again)
+        __syncthreads();
+        if (kv0 >= wave_kend) continue;  // every key masked for this wave
+        floatx4 s[NJ][NQ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int c = 0; c < CD; ++c) {
+                bf16x8 kf[3];
+#pragma unroll
+                for (int pl = 0; pl < 3; ++pl) kf[pl] = frag(Kp[pl], j * CD + c);
+#pragma unroll
+                for (int a = 0; a < NQ; ++a)
+                    s[j][a] = mfma_split(kf, qf[a][c], c == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : s[j][a]);
+            }
+        bf16x8 pf[NM][NQ][3];
+#pragma unroll
+        for (int a = 0; a < NQ; ++a) {
+            const int qi = q0 + 16 * a + r16;
+            if (kv0 + BK > p.Sk || (p.causal && kv0 + BK - 1 > q0 + 16 * a + shift)) {
+                const int lim = (p.causal ? min(qi + shift, p.Sk - 1) : p.Sk - 1) - kv0 - 4 * g;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[j][a][r] = 16 * j + r <= lim ? s[j][a][r] : -INFINITY;
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[j][a][r] = __builtin_fmaf(s[j][a][r], sl2, -mb[a]);
+            const float m_prev = m_lane[a];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                m_lane[a] = fmaxf(fmaxf(m_lane[a], fmaxf(s[j][a][0], s[j][a][1])), fmaxf(s[j][a][2], s[j][a][3]));
+            if (__builtin_amdgcn_ballot_w64(m_lane[a] > 8.f || (m_lane[a] < -64.f && m_lane[a] != -INFINITY))) {
+                const float row_prev = max_across_rows(m_prev), row = max_across_rows(m_lane[a]);
+                if (row > 8.f || (row < -64.f && row != -INFINITY)) {
+                    // nothing accumulated yet (row_prev = -inf): factor 0
+                    const float corr = row_prev == -INFINITY ? 0.f : exp2_fast(-row);
+                    mb[a] += row;
+                    m_lane[a] -= row;
+                    l_part[a] *= corr;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) s[j][a] -= row;
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) oacc[c][a] *= corr;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                float e[8];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    e[r] = exp2_fast(s[2 * m][a][r]);
+                    e[4 + r] = exp2_fast(s[2 * m + 1][a][r]);
+                }
+                l_part[a] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+                u32x4 hh, mm, ll;
+                split8(e, hh, mm, ll);
+                pf[m][a][0] = __builtin_bit_cast(bf16x8, hh);
+                pf[m][a][1] = __builtin_bit_cast(bf16x8, mm);
+                pf[m][a][2] = __builtin_bit_cast(bf16x8, ll);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                bf16x8 vf[3];
+#pragma unroll
+                for (int pl = 0; pl < 3; ++pl) vf[pl] = frag(Vp[pl], c * NM + m);
+#pragma unroll
+                for (int a = 0; a < NQ; ++a) oacc[c][a] = mfma_split(vf, pf[m][a], oacc[c][a]);
+            }
+    }
+    if (kmax > 0x1p90f) s_large = 1;
+    __syncthreads();
+
+    bool bad = s_large || qmax > 0x1p90f;
+    float l[NQ];
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        l[a] = l_part[a] + __shfl_xor(l_part[a], 16, WAVE);
+        l[a] += __shfl_xor(l[a], 32, WAVE);
+        bad |= !(l[a] <= FLT_MAX);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float o = fabsf(oacc[c][a][r]);
+                bad |= !(o <= FLT_MAX) || (o < l[a] * 0x1p-108f && o != 0.f);
+            }
+    }
+    if (__builtin_amdgcn_ballot_w64(bad)) {
+        for (int q = q0; q < min(q0 + 16 * NQ, p.Sq); ++q) {
+            float *row = p.nsplit > 1 ? p.part + (((long)split * p.B * p.H + bh) * p.Sq + q) * (D + 4)
+                                      : (float *)p.O + (long)b * p.o_sb + (long)h * p.o_sh + (long)q * p.o_ss;
+            attend_row_fp32<D>((const float *)p.Q + (long)b * p.q_sb + (long)h * p.q_sh + (long)q * p.q_ss,
+                               Kb + (long)k_lo * p.k_ss, Vb + (long)k_lo * p.k_ss, p.k_ss,
+                               max(0, (p.causal ? min(k_end, q + shift + 1) : k_end) - k_lo), p.scale_log2, row, p.nsplit > 1);
+        }
+        return;
+    }
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        const int qi = q0 + 16 * a + r16;
+        if (qi >= p.Sq) continue;
+        if (p.nsplit > 1) {  // unnormalised partial: O, then the base (exponent units) and row sum
+            float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qi) * (D + 4);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) *(floatx4 *)(row + 16 * c + 4 * g) = oacc[c][a];
+            if (g == 0) {
+                row[D] = l[a] > 0.f ? mb[a] : -INFINITY;
+                row[D + 1] = l[a];
+            }
+            continue;
+        }
+        const float inv = l[a] > 0.f ? 1.0f / l[a] : 0.f;
+        float *o = (float *)p.O + (long)b * p.o_sb + (long)h * p.o_sh + (long)qi * p.o_ss;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) *(floatx4 *)(o + 16 * c + 4 * g) = oacc[c][a] * inv;
+    }
+}
+
+// Combines the key-split partials of a prefill launch: one thread per row and four head-dim
+// elements; O = sum_i 2^(m_i - M) O_i / sum_i 2^(m_i - M) l_i with M = max_i m_i.  Every
+// split's numbers are requested before the first is used (one memory round trip).
+constexpr int FA_MAX_SPLITS = 4;
+template <typename T>
 __global__ void __launch_bounds__(256) flash_merge_kernel(const PrefillArgs p, int D)
 {
     const long g = (long)blockIdx.x * 256 + threadIdx.x;
     const long rows = (long)p.B * p.H * p.Sq;
-    if (g >= rows * D) return;
-    const long row = g / D;
-    const int e = (int)(g % D);
-    const int bh = (int)(row / p.Sq), q = (int)(row % p.Sq);
-    const long sstride = rows * (D + 2);
-    const float *pr = p.part + row * (D + 2);
-    float mx = -INFINITY;
-    for (int i = 0; i < p.nsplit; ++i) mx = fmaxf(mx, pr[i * sstride + D]);
-    float o = 0.f, l = 0.f;
-    for (int i = 0; i < p.nsplit; ++i) {
-        const float mi = pr[i * sstride + D];
-        // bf16 partials carry their base in exponent units, fp32 ones their row max raw
-        const float w = mi == -INFINITY ? 0.f : exp2_fast(BF16 ? mi - mx : (mi - mx) * p.scale_log2);
-        o += w * pr[i * sstride + e];
-        l += w * pr[i * sstride + D + 1];
+    if (g >= rows * (D / 4)) return;
+    const long row = g / (D / 4);
+    const int e = 4 * (int)(g % (D / 4));
+    const long sstride = rows * (D + 4);
+    const float *pr = p.part + row * (D + 4);
+    float mi[FA_MAX_SPLITS], li[FA_MAX_SPLITS];
+    floatx4 oi[FA_MAX_SPLITS];
+#pragma unroll
+    for (int i = 0; i < FA_MAX_SPLITS; ++i) {
+        const float *q = pr + min(i, p.nsplit - 1) * sstride;
+        mi[i] = i < p.nsplit ? q[D] : -INFINITY;
+        li[i] = q[D + 1];
+        oi[i] = *(const floatx4 *)(q + e);
     }
-    const float v = l > 0.f ? o / l : 0.f;
-    const int b = bh / p.H, h = bh % p.H;
-    const long oi = (long)b * p.o_sb + (long)h * p.o_sh + (long)q * p.o_ss + e;
-    if constexpr (BF16)
-        ((uint16_t *)p.O)[oi] = __builtin_bit_cast(uint16_t, (__bf16)v);
-    else
-        ((float *)p.O)[oi] = v;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < FA_MAX_SPLITS; ++i) mx = fmaxf(mx, mi[i]);
+    floatx4 o = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+#pragma unroll
+    for (int i = 0; i < FA_MAX_SPLITS; ++i) {
+        if (mi[i] == -INFINITY) continue;  // no such split, or no key visible in it
+        const float w = exp2_fast(mi[i] - mx);
+        o += w * oi[i];
+        l += w * li[i];
+    }
+    const floatx4 v = l != 0.f ? o / l : floatx4{0.f, 0.f, 0.f, 0.f};
+    const int bh = (int)(row / p.Sq), q = (int)(row % p.Sq), b = bh / p.H, h = bh % p.H;
+    const long at = (long)b * p.o_sb + (long)h * p.o_sh + (long)q * p.o_ss + e;
+    if constexpr (std::is_same_v<T, float>) {
+        *(floatx4 *)((float *)p.O + at) = v;
+    } else {
+        u32x2 u;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            u[k] = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v[2 * k]) |
+                   ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v[2 * k + 1]) << 16);
+        *(u32x2 *)((uint16_t *)p.O + at) = u;
+    }
 }
 
 // ---------------------------------------------------------------- decode
@@ -999,47 +1141,49 @@ jas_status jas_attn_prefill(const void *Q, const void *K, const void *V, void *O
                   scale * 1.4426950408889634f, causal};
     hipStream_t s = stream_or_default(stream);
     // grid: one workgroup per (query block, batch x head), padded to a multiple of the 8 XCDs.
-    // When 8-wave workgroups (128 queries) would not give every CU one, 4-wave workgroups
-    // (64 queries) double the count -- where a thread's K/V staging stays at four 16-byte
-    // loads per tile (not fp32 with D = 128).  A launch that still leaves CUs idle also
+    // When workgroups of 128 queries would not give every CU one, 64-query ones double the
+    // count (fp32 with D = 128 always takes those).  A launch that still leaves CUs idle also
     // splits its keys over up to 4 work items (at least two 64-key tiles each), merged by a
     // second kernel; with a causal mask the splits past a query block's diagonal find every
     // key masked and leave a zero-weight partial (decoder self-attention of jasmine's
     // Transformer-base, 8 heads x 512 tokens: forward 0.63 -> 0.57 ms).
-    const bool few = (long)ceil_div(Sq, 16 * FA_WAVES) * B * H < 256;
-    const int nw = few && (dtype == JAS_BF16 || D <= 64) ? 4 : FA_WAVES;
-    const long items = (long)ceil_div(Sq, 16 * nw) * B * H;
+    const bool few = (long)ceil_div(Sq, 128) * B * H < 256;
+    const bool narrow = few || (dtype == JAS_F32 && D == 128);  // 64 queries
+    const long items = (long)ceil_div(Sq, narrow ? 64 : 128) * B * H;
     if (items < 256 && Sk >= 4 * 64) {
-        int ns = (int)std::min<long>(4, (512 + items - 1) / items);
+        int ns = (int)std::min<long>(FA_MAX_SPLITS, (512 + items - 1) / items);
         ns = std::min(ns, Sk / 128);
         if (ns > 1) {
             p.kchunk = ceil_div(ceil_div(Sk, ns), 64) * 64;
             p.nsplit = ceil_div(Sk, p.kchunk);
-            p.part = (float *)workspace(sizeof(float) * (size_t)p.nsplit * B * H * Sq * (D + 2), s);
+            p.part = (float *)workspace(sizeof(float) * (size_t)p.nsplit * B * H * Sq * (D + 4), s);
             JAS_CHECK(p.part, JAS_ERR_OOM, "jas_attn_prefill: workspace allocation failed");
         }
     }
-#define JAS_FA_LAUNCH(DD, BF, NWV)                                                                     \
+#define JAS_FA_LAUNCH(KERNEL, NT)                                                                       \
     {                                                                                                  \
-        const int total = ceil_div(Sq, 16 * (NWV)) * B * H * p.nsplit;                                 \
-        p.fold = causal && p.nsplit == 1 ? fa_fold((const void *)flash_prefill_kernel<DD, BF, 64, NWV>, 64 * (NWV), total) : 0; \
-        hipLaunchKernelGGL((flash_prefill_kernel<DD, BF, 64, NWV>), dim3((total + 7) / 8 * 8), dim3(64 * (NWV)), 0, s, p); \
+        const int total = (int)items * p.nsplit;                                                       \
+        p.fold = causal && p.nsplit == 1 ? fa_fold((const void *)KERNEL, NT, total) : 0;               \
+        hipLaunchKernelGGL(KERNEL, dim3((total + 7) / 8 * 8), dim3(NT), 0, s, p);                      \
     }
 #define JAS_FA(DD)                                                                                     \
     if (D == DD) {                                                                                     \
+        constexpr int BKV = DD == 128 ? 32 : 64, NQV = DD == 128 ? 1 : 2;                              \
         if (dtype == JAS_BF16) {                                                                       \
-            if (nw == 4) JAS_FA_LAUNCH(DD, true, 4) else JAS_FA_LAUNCH(DD, true, FA_WAVES)             \
+            if (narrow) JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, 4>), 256)                          \
+            else JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, FA_WAVES>), 64 * FA_WAVES)                \
         } else {                                                                                       \
-            if (nw == 4 && DD <= 64) JAS_FA_LAUNCH(DD, false, 4) else JAS_FA_LAUNCH(DD, false, FA_WAVES) \
+            if (narrow) JAS_FA_LAUNCH((flash_split_kernel<DD, 1, BKV>), 256)                           \
+            else JAS_FA_LAUNCH((flash_split_kernel<DD, NQV, BKV>), 256)                                \
         }                                                                                              \
     }
     JAS_FA(32) JAS_FA(64) JAS_FA(128)
 #undef JAS_FA
 #undef JAS_FA_LAUNCH
     if (p.nsplit > 1) {
-        const long n = (long)B * H * Sq * D;
-        if (dtype == JAS_BF16) hipLaunchKernelGGL(flash_merge_kernel<true>, dim3(ceil_div(n, 256)), dim3(256), 0, s, p, D);
-        else hipLaunchKernelGGL(flash_merge_kernel<false>, dim3(ceil_div(n, 256)), dim3(256), 0, s, p, D);
+        const dim3 grid(ceil_div((long)B * H * Sq * (D / 4), 256));
+        if (dtype == JAS_BF16) hipLaunchKernelGGL(flash_merge_kernel<uint16_t>, grid, dim3(256), 0, s, p, D);
+        else hipLaunchKernelGGL(flash_merge_kernel<float>, grid, dim3(256), 0, s, p, D);
     }
     JAS_LAUNCH_CHECK();
     return JAS_OK;

@@ -657,6 +657,70 @@ def test_attn_prefill_long_causal(jas, B, H, Sq, Sk, D, dt):
             close(do.numpy(), want, atol=1e-5, rtol=1e-4)
 
 
+def _attention64(Q, K, V, causal):
+    """[B, H, S, D] attention in 64 bits, causal aligned to the last key; masked keys carry nothing."""
+    Q, K, V = (x.astype(np.float64) for x in (Q, K, V))
+    out = np.zeros(Q.shape)
+    Sq, Sk = Q.shape[2], K.shape[2]
+    with np.errstate(all="ignore"):
+        for b, h, i in np.ndindex(*Q.shape[:3]):
+            n = min(Sk, i + Sk - Sq + 1) if causal else Sk
+            s = K[b, h, :n] @ Q[b, h, i] / math.sqrt(Q.shape[3])
+            e = np.exp(s - s.max())
+            out[b, h, i] = (e[:, None] * V[b, h, :n]).sum(0) / e.sum()
+    return out
+
+
+def _run_attention_f32(jas, Q, K, V, causal):
+    import ctypes as C
+    B, H, Sq, D = Q.shape
+    Sk = K.shape[2]
+    dq, dk, dv, do = jas.to_device(Q), jas.to_device(K), jas.to_device(V), jas.DeviceArray(Q.shape)
+    qs, ks = (H * Sq * D, Sq * D, D), (H * Sk * D, Sk * D, D)
+    jas.check(jas.lib.jas_attn_prefill(dq.p, dk.p, dv.p, do.p, B, H, Sq, Sk, D, *qs, *ks, *qs, C.c_float(1 / math.sqrt(D)),
+                                       causal, 0, None))
+    return do.numpy()
+
+
+# both widths of flash_split_kernel (32 queries per wave from 256 blocks of 128; 16 below), the
+# edges of its query blocks and key tiles, and its key split (few items, at least 256 keys)
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal", [(8, 33, 97, 97, 32, 1), (16, 17, 65, 130, 64, 0), (4, 33, 129, 129, 64, 1),
+                                                (3, 5, 63, 95, 128, 1), (1, 3, 130, 130, 128, 0), (1, 2, 17, 300, 64, 1),
+                                                (1, 2, 70, 257, 32, 0), (1, 1, 1, 1, 64, 1)])
+def test_attn_prefill_split(jas, B, H, Sq, Sk, D, causal):
+    Q, K, V = normal((B, H, Sq, D), 41, 0), normal((B, H, Sk, D), 41, 1), normal((B, H, Sk, D), 41, 2)
+    got = _run_attention_f32(jas, Q, K, V, causal)
+    want = _attention64(Q, K, V, causal)
+    # a score of magnitude sum |q||k| / sqrt(D) <= 12 here carries at most D roundings of 2^-24
+    # of it, a probability that relative error twice (its own and its row sum's)
+    bound = 2 * 12 * D * 2.0 ** -24 * np.abs(V).max()
+    assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
+
+
+@pytest.mark.parametrize("B,H,S,D", [(1, 2, 70, 64), (1, 1, 300, 32), (1, 1, 80, 128), (16, 17, 66, 64)])
+def test_attn_prefill_split_range(jas, B, H, S, D):
+    """Rows outside the bf16 split's range: infinities and NaN in Q, K and V, values of V whose
+    parts underflow, and small Q against large K."""
+    Q, K, V = (normal((B, H, S, D), 42, k) for k in range(3))
+    Q[0, 0, 5, 3] = np.inf
+    K[0, 0, 40, 0] = np.nan   # reaches queries 40 and up
+    V[0, 0, 60, 1] = np.inf   # and 60 and up
+    if B * H > 1:
+        b, h = (0, 1) if B == 1 else (B - 1, H - 1)
+        V[b, h] *= np.float32(2.0 ** -119)
+        Q[b, h] *= np.float32(2.0 ** -112)
+        K[b, h] *= np.float32(2.0 ** 112)
+    got = _run_attention_f32(jas, Q, K, V, 1)
+    want = _attention64(Q, K, V, 1)
+    # row 5's one infinite query element gives infinite scores: no finite output
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    fin = np.isfinite(want)
+    scale = np.broadcast_to(np.nanmax(np.where(np.isfinite(V), np.abs(V), np.nan), axis=(2, 3), keepdims=True), V.shape)
+    # as above, and sums of products below 2^-126 round at 2^-149
+    bound = 2 * 12 * D * 2.0 ** -24 * scale[fin] + S * 2.0 ** -149
+    assert np.all(np.abs(got[fin] - want[fin]) <= bound), np.max(np.abs(got[fin] - want[fin]) / bound)
+
+
 @pytest.mark.parametrize("D,dt,causal", [(64, 0, 1), (64, 3, 1), (128, 3, 0), (32, 3, 1), (128, 0, 0)])
 def test_attn_prefill_growing_scores(jas, D, dt, causal):
     """Keys whose scale grows along the sequence, so the running row max keeps rising by more
