@@ -239,7 +239,11 @@ __device__ __forceinline__ void argmax_rows(float &bv, int &bi)
 // packed weight and activation layouts put in that lane.  One such MFMA does the work of
 // eight fp32 16x16x4 ones, so halving the weight bytes does not make the kernel
 // matrix-core bound.
-template <int NT, int WPB, int DEPTH, bool DUAL, bool PACKED, bool WB>
+//
+// EPI: the epilogue (SkinnyEpi; SE_HEAD is EPI_STORE plus the workgroup's greedy picks) is a
+// template parameter: a GPT-2-size launch runs each instruction once, and what it fetches of
+// a 20 KB body with every epilogue in it (tanh, the row maxima) cost more than its arithmetic.
+template <int NT, int WPB, int DEPTH, bool DUAL, bool PACKED, bool WB, int EPI>
 __global__ void __launch_bounds__(WPB * 64)
 skinny_kernel(const void *__restrict__ W, const void *__restrict__ W2, const float *__restrict__ X, long ldx, int M,
               int N, int K, const SkinnyEpiArgs epi)
@@ -423,15 +427,14 @@ skinny_kernel(const void *__restrict__ W, const void *__restrict__ W2, const flo
         for (int ww = 1; ww < WPB; ++ww) s0 += red[ww][t][ln];
         v[0] = s0[0], v[1] = s0[1], v[2] = s0[2], v[3] = s0[3];
     }
-    if constexpr (!DUAL) {
-        if (epi.amax_v) {  // first maximum of the stored values over this workgroup's rows
+    if constexpr (EPI == SE_HEAD) {
+        {  // first maximum of the stored values over this workgroup's rows
             __shared__ float sbv[NH * 16];
             __shared__ int sbi[NH * 16];
             float bv = -INFINITY;
             int bi = 0x7fffffff;
             for (int r = 0; r < nv; ++r) {
-                float x = epi.bias ? v[r] + epi.bias[m + r] : v[r];
-                x = apply_act(x, epi.act);
+                const float x = epi.bias ? v[r] + epi.bias[m + r] : v[r];
                 if (x > bv) { bv = x; bi = m + r; }
             }
             // the four lanes of a token in each wave (ln, ln ^ 16, ln ^ 32, ln ^ 48) combine in
@@ -452,14 +455,14 @@ skinny_kernel(const void *__restrict__ W, const void *__restrict__ W2, const flo
     }
     if (!live) return;
 
-    if (epi.mode == EPI_PARTIAL) {  // raw split-K partial, [split][16][M]; the consumer reduces
+    if constexpr (EPI == EPI_PARTIAL) {  // raw split-K partial, [split][16][M]; the consumer reduces
         float *o = epi.out + ((long)blockIdx.y * 16 + n) * M + m;
         if (nv == 4 && (M & 3) == 0) *(float4 *)o = make_float4(v[0], v[1], v[2], v[3]);
         else
             for (int r = 0; r < nv; ++r) o[r] = v[r];
         return;
     }
-    if constexpr (DUAL) {  // SwiGLU: silu(gate) * up
+    if constexpr (EPI == EPI_SWIGLU) {  // silu(gate) * up
         floatx4 s1 = red[0][t + NH][ln];
 #pragma unroll
         for (int ww = 1; ww < WPB; ++ww) s1 += red[ww][t + NH][ln];
@@ -470,64 +473,54 @@ skinny_kernel(const void *__restrict__ W, const void *__restrict__ W2, const flo
         }
         float *o = epi.out + (long)n * epi.ldo + m;
         for (int r = 0; r < nv; ++r) o[r] = silu_f(v[r]) * s1[r];
-        return;
-    } else {
+    }
+    if constexpr (EPI != EPI_PARTIAL && EPI != EPI_SWIGLU) {
         if (epi.bias)
             for (int r = 0; r < nv; ++r) v[r] = v[r] + epi.bias[m + r];
-        if (epi.mode == EPI_STORE) {
-            if (epi.out_packed && nv == 4) {
-                *(float4 *)(epi.out + packed_b_offset(n, m)) = make_float4(
-                    apply_act(v[0], epi.act), apply_act(v[1], epi.act), apply_act(v[2], epi.act), apply_act(v[3], epi.act));
-                return;
-            }
-            float *o = epi.out + (long)n * epi.ldo + m;
-            for (int r = 0; r < nv; ++r) o[r] = apply_act(v[r], epi.act);
-        } else if (epi.mode == EPI_RESID) {
-            float *o = epi.out + (long)n * epi.ldo + m;
-            for (int r = 0; r < nv; ++r) o[r] = o[r] + v[r];
-        } else {  // EPI_QKV (m % 4 == 0, d % 16 == 0, dh even: the 4 rows share a section and head)
-            const int sec = m / epi.d, e = m - sec * epi.d, h = e / epi.dh, ee = e - h * epi.dh;
-            const int pos = epi.pos[n];
-            if (epi.rope && sec < 2) {
+    }
+    if constexpr (EPI == EPI_STORE || EPI == SE_GELU || EPI == SE_HEAD) {
+        auto act = [&](float x) { return EPI == EPI_STORE ? apply_act(x, epi.act) : EPI == SE_GELU ? gelu_f(x) : x; };
+        if (epi.out_packed && nv == 4) {
+            *(float4 *)(epi.out + packed_b_offset(n, m)) = make_float4(act(v[0]), act(v[1]), act(v[2]), act(v[3]));
+            return;
+        }
+        float *o = epi.out + (long)n * epi.ldo + m;
+        for (int r = 0; r < nv; ++r) o[r] = act(v[r]);
+    }
+    if constexpr (EPI == EPI_QKV) {  // (m % 4 == 0, d % 16 == 0, dh even: the 4 rows share a section and head)
+        const int sec = m / epi.d, e = m - sec * epi.d, h = e / epi.dh, ee = e - h * epi.dh;
+        const int pos = epi.pos[n];
+        if (epi.rope_tab && sec < 2) {
 #pragma unroll
-                for (int pr = 0; pr < 2; ++pr) {
-                    int i = (ee + 2 * pr) / 2;
-                    double cs, sn;
-                    if (epi.rope_tab) {
-                        const double2 cst = epi.rope_tab[(long)pos * (epi.dh / 2) + i];
-                        cs = cst.x, sn = cst.y;
-                    } else {
-                        const double a = (double)pos * pow((double)epi.theta, -2.0 * i / (double)epi.dh);
-                        cs = cos(a), sn = sin(a);
-                    }
-                    double x0 = v[2 * pr], x1 = v[2 * pr + 1];
-                    v[2 * pr] = (float)(x0 * cs - x1 * sn);
-                    v[2 * pr + 1] = (float)(x0 * sn + x1 * cs);
-                }
+            for (int pr = 0; pr < 2; ++pr) {
+                const double2 cst = epi.rope_tab[(long)pos * (epi.dh / 2) + (ee + 2 * pr) / 2];
+                const double cs = cst.x, sn = cst.y, x0 = v[2 * pr], x1 = v[2 * pr + 1];
+                v[2 * pr] = (float)(x0 * cs - x1 * sn);
+                v[2 * pr + 1] = (float)(x0 * sn + x1 * cs);
             }
-            if (sec == 0) {
-                *(float4 *)(epi.q_out + (long)n * epi.d + e) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-                const long ce = (long)n * epi.kv_sb + (long)h * epi.kv_sh + (long)pos * epi.dh + ee;
-                float *cache = sec == 1 ? epi.k_cache : epi.v_cache;
-                if (epi.kv_bf16)
-                    *(u32x2 *)((uint16_t *)cache + ce) =
-                        u32x2{(uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
-                              (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16)};
-                else
-                    *(float4 *)(cache + ce) = make_float4(v[0], v[1], v[2], v[3]);
-            }
+        }
+        if (sec == 0) {
+            *(float4 *)(epi.q_out + (long)n * epi.d + e) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+            const long ce = (long)n * epi.kv_sb + (long)h * epi.kv_sh + (long)pos * epi.dh + ee;
+            float *cache = sec == 1 ? epi.k_cache : epi.v_cache;
+            if (epi.kv_bf16)
+                *(u32x2 *)((uint16_t *)cache + ce) =
+                    u32x2{(uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
+                          (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16)};
+            else
+                *(float4 *)(cache + ce) = make_float4(v[0], v[1], v[2], v[3]);
         }
     }
 }
 
-template <int NT, int WPB, int DEPTH, bool DUAL, bool PACKED, bool WB = false>
+template <int NT, int WPB, int DEPTH, bool DUAL, bool PACKED, bool WB, int EPI>
 static void launch_skinny(const void *W, const void *W2, const float *X, long ldx, int M, int N, int K,
                           const SkinnyEpiArgs &epi, hipStream_t s)
 {
     const int rows = DUAL ? 16 * (NT / 2) : NT * 16;
-    const int ks = epi.mode == EPI_PARTIAL ? std::max(1, epi.ksplit) : 1;
-    hipLaunchKernelGGL((skinny_kernel<NT, WPB, DEPTH, DUAL, PACKED, WB>), dim3((M + rows - 1) / rows, ks),
+    const int ks = EPI == EPI_PARTIAL ? std::max(1, epi.ksplit) : 1;
+    hipLaunchKernelGGL((skinny_kernel<NT, WPB, DEPTH, DUAL, PACKED, WB, EPI>), dim3((M + rows - 1) / rows, ks),
                        dim3(WPB * 64), 0, s, W, W2, X, ldx, M, N, K, epi);
 }
 
@@ -595,7 +588,7 @@ int skinny_pick_ksplit(int M, int K, bool wbf16)
 }
 
 jas_status skinny_gemm(const void *W, const void *W2, const float *X, long ldx, int M, int N, int K,
-                       const SkinnyEpiArgs &epi, hipStream_t s, bool packed, const SkinnyTuning *tune, bool wbf16)
+                       const SkinnyEpiArgs &epi, hipStream_t s, bool packed, bool wbf16)
 {
     JAS_CHECK(!wbf16 || packed, JAS_ERR_INVALID, "skinny_gemm: bf16 weights only in the packed layout");
     JAS_CHECK(N >= 1 && N <= 16 && M > 0 && K > 0 && K % 4 == 0 && ldx % 4 == 0, JAS_ERR_INVALID,
@@ -608,9 +601,11 @@ jas_status skinny_gemm(const void *W, const void *W2, const float *X, long ldx, 
     if (epi.mode == EPI_QKV)
         JAS_CHECK(epi.d % 16 == 0 && epi.dh % 4 == 0 && M == 3 * epi.d, JAS_ERR_INVALID, "skinny_gemm: bad QKV shape");
     if (dual) JAS_CHECK(W2 != nullptr, JAS_ERR_INVALID, "skinny_gemm: SwiGLU needs both weights");
-    SkinnyTuning tu = tune ? *tune : skinny_default_tuning(M, K, dual, epi.mode == EPI_PARTIAL, wbf16);
-    if (!tune && !packed && tu.nt > 2) tu.nt = 2;  // more tiles: packed weights only
-    const int nt = dual && (tu.nt < 2 || tu.nt % 2) ? 2 : tu.nt;
+    // row-major weights serve jas_gemm's few-token products only (store with any activation)
+    JAS_CHECK(packed || (epi.mode == EPI_STORE && !epi.amax_v), JAS_ERR_INVALID, "skinny_gemm: packed weights only");
+    JAS_CHECK(!epi.amax_v || (epi.mode == EPI_STORE && epi.act == JAS_ACT_NONE), JAS_ERR_INVALID, "skinny_gemm: bad LM head");
+    SkinnyTuning tu = skinny_default_tuning(M, K, dual, epi.mode == EPI_PARTIAL, wbf16);
+    if (!packed && tu.nt > 2) tu.nt = 2;  // more tiles: packed weights only
     SkinnyEpiArgs ep = epi;
     const int nchunk = (K + 63) / 64;
     if (ep.mode == EPI_PARTIAL) {
@@ -622,40 +617,32 @@ jas_status skinny_gemm(const void *W, const void *W2, const float *X, long ldx, 
         ep.cpb = nchunk;
         ep.ksplit = 1;
     }
-#define JAS_SK(NTV, WPBV, DV, PV, DEP)                                                         \
-    if (nt == NTV && tu.wpb == WPBV && dual == DV && packed == PV && tu.depth == DEP) {       \
-        launch_skinny<NTV, WPBV, DEP, DV, PV>(W, W2, X, ldx, M, N, K, ep, s);                 \
-        JAS_LAUNCH_CHECK();                                                                    \
-        return JAS_OK;                                                                         \
+    const int kind = epi.amax_v ? (int)SE_HEAD : epi.mode == EPI_STORE && packed && epi.act == JAS_ACT_GELU ? (int)SE_GELU : epi.mode;
+    // the geometries that skinny_default_tuning picks, each with the epilogues that reach it
+#define JAS_SK(NTV, WPBV, DEP, DV, PV, WBV, EPIV)                                                          \
+    if (tu.nt == NTV && tu.wpb == WPBV && tu.depth == DEP && packed == PV && wbf16 == WBV && kind == EPIV) { \
+        launch_skinny<NTV, WPBV, DEP, DV, PV, WBV, EPIV>(W, W2, X, ldx, M, N, K, ep, s);                   \
+        JAS_LAUNCH_CHECK();                                                                                \
+        return JAS_OK;                                                                                     \
     }
-#define JAS_SK_D(NTV, WPBV, DV, PV) JAS_SK(NTV, WPBV, DV, PV, 2) JAS_SK(NTV, WPBV, DV, PV, 3) JAS_SK(NTV, WPBV, DV, PV, 4)
-#define JAS_SK_P(NTV, WPBV, DV) JAS_SK_D(NTV, WPBV, DV, true) JAS_SK_D(NTV, WPBV, DV, false)
-    if (wbf16) {  // the geometries the default tuning picks
-#define JAS_SKB(NTV, WPBV, DV, DEP)                                                           \
-    if (nt == NTV && tu.wpb == WPBV && dual == DV && tu.depth == DEP) {                      \
-        launch_skinny<NTV, WPBV, DEP, DV, true, true>(W, W2, X, ldx, M, N, K, ep, s);         \
-        JAS_LAUNCH_CHECK();                                                                    \
-        return JAS_OK;                                                                         \
-    }
-        JAS_SKB(2, 4, true, 3) JAS_SKB(2, 4, true, 4) JAS_SKB(2, 4, false, 2) JAS_SKB(2, 4, false, 3)
-        JAS_SKB(2, 4, false, 4) JAS_SKB(2, 8, false, 2) JAS_SKB(2, 8, false, 3) JAS_SKB(4, 4, false, 2)
-        JAS_SKB(4, 4, false, 3) JAS_SKB(4, 4, false, 4) JAS_SKB(1, 8, false, 3) JAS_SKB(1, 8, false, 4)
-        JAS_SKB(3, 4, false, 3) JAS_SKB(3, 4, false, 4) JAS_SKB(6, 4, true, 2)
-#undef JAS_SKB
-        return fail(JAS_ERR_INVALID, "skinny_gemm: unsupported tuning for bf16 weights");
-    }
-    JAS_SK_P(1, 4, false) JAS_SK_P(1, 8, false) JAS_SK_P(2, 4, false) JAS_SK_P(2, 8, false) JAS_SK_P(2, 4, true)
-    JAS_SK_P(2, 8, true)
-    // 1024-thread workgroups get 128 VGPRs: depth 4 would spill
-    JAS_SK(1, 16, false, true, 2) JAS_SK(1, 16, false, true, 3) JAS_SK(1, 16, false, false, 2)
-    JAS_SK(1, 16, false, false, 3)
-    // four row tiles per workgroup share each activation chunk (packed weights only)
-    JAS_SK(4, 4, false, true, 2) JAS_SK(4, 4, false, true, 3) JAS_SK(4, 8, false, true, 2)
-    JAS_SK(3, 4, false, true, 2) JAS_SK(3, 4, false, true, 3) JAS_SK(3, 8, false, true, 2)
-    // dual with three (gate, up) pairs per workgroup (packed weights only)
-    JAS_SK(6, 4, true, true, 2)
-#undef JAS_SK_P
+    // whole projections: QKV, FC (GELU), LM head, and plain stores (jas_lm_project)
+#define JAS_SK_W(NTV, WPBV, DEP, WBV)                                                                       \
+    JAS_SK(NTV, WPBV, DEP, false, true, WBV, EPI_QKV) JAS_SK(NTV, WPBV, DEP, false, true, WBV, SE_GELU)     \
+    JAS_SK(NTV, WPBV, DEP, false, true, WBV, SE_HEAD) JAS_SK(NTV, WPBV, DEP, false, true, WBV, EPI_STORE)
+#define JAS_SK_P(NTV, WPBV, DEP, WBV) JAS_SK(NTV, WPBV, DEP, false, true, WBV, EPI_PARTIAL)
+#define JAS_SK_D(NTV, WPBV, DEP, WBV) JAS_SK(NTV, WPBV, DEP, true, true, WBV, EPI_SWIGLU)
+    JAS_SK_W(1, 8, 3, false) JAS_SK_W(2, 8, 2, false) JAS_SK_W(3, 4, 2, false) JAS_SK_W(4, 4, 3, false)
+    JAS_SK_P(2, 8, 2, false) JAS_SK_P(2, 4, 2, false) JAS_SK_P(2, 4, 3, false)
+    JAS_SK_D(2, 4, 3, false) JAS_SK_D(6, 4, 2, false)
+    JAS_SK_W(1, 8, 3, true) JAS_SK_W(3, 4, 4, true) JAS_SK_W(4, 4, 2, true) JAS_SK_W(4, 4, 3, true)
+    JAS_SK_P(2, 8, 2, true) JAS_SK_P(4, 4, 4, true)
+    JAS_SK_D(2, 4, 3, true) JAS_SK_D(6, 4, 2, true)
+    // row-major weights (nt clamped to two)
+    JAS_SK(1, 8, 3, false, false, false, EPI_STORE) JAS_SK(2, 8, 2, false, false, false, EPI_STORE)
+    JAS_SK(2, 4, 2, false, false, false, EPI_STORE) JAS_SK(2, 4, 3, false, false, false, EPI_STORE)
 #undef JAS_SK_D
+#undef JAS_SK_P
+#undef JAS_SK_W
 #undef JAS_SK
     return fail(JAS_ERR_INVALID, "skinny_gemm: unsupported tuning");
 }
@@ -828,7 +815,7 @@ extern "C" jas_status jas_gemm(int M, int N, int K, const float *A, long as0, lo
         e.bias = bias_mode == 1 ? bias : nullptr;
         e.out = C;
         e.ldo = cs1;
-        return skinny_gemm(A, nullptr, B, bs1, M, N, K, e, s, false, nullptr);
+        return skinny_gemm(A, nullptr, B, bs1, M, N, K, e, s, false);
     }
     return gemm_general(M, N, K, A, as0, as1, B, bs0, bs1, C, cs0, cs1, bias, bias_mode, act, accumulate, batch, abs_,
                         bbs, cbs, biasbs, s, false);

@@ -8,13 +8,15 @@ namespace jas {
 // output feature, column n a token.
 enum SkinnyEpi : int {
     EPI_STORE = 0,   // out[n*ldo + m] = act(acc + bias[m])
-    EPI_RESID = 1,   // out[n*ldo + m] += acc + bias[m]        (residual stream update)
     EPI_SWIGLU = 2,  // out[n*ldo + m] = silu(acc_gate) * acc_up  (W = gate rows, W2 = up rows)
     EPI_QKV = 3,     // rows [0,d) q, [d,2d) k, [2d,3d) v: (+bias) (+RoPE on q,k), q -> q_out,
                      // k/v -> KV cache at the token's position
     EPI_PARTIAL = 4  // K split over `ksplit` workgroups; out[(s*16 + n)*M + m] = partial sum of
                      // split s (no bias/activation); the consumer adds the splits in order
 };
+
+// epilogues of the kernel that the arguments' mode and act select together
+enum SkinnyKernelEpi : int { SE_HEAD = 8 /* EPI_STORE with greedy picks */, SE_GELU = 9 /* EPI_STORE, GELU */ };
 
 struct SkinnyEpiArgs {
     int mode = EPI_STORE;
@@ -34,10 +36,7 @@ struct SkinnyEpiArgs {
     const int32_t *pos = nullptr;
     long kv_sb = 0, kv_sh = 0;
     int d = 0, dh = 0;
-    int rope = 0;
-    float theta = 10000.f;
-    // optional [position][dh / 2] (cos, sin) of the rotary angles, the same double values
-    // the epilogue would compute; saves the pow / cos / sin at the end of every workgroup
+    // [position][dh / 2] (cos, sin) of the rotary angles, in double; null: no rotary
     const double2 *rope_tab = nullptr;
     // EPI_STORE: also the first maximum over this workgroup's rows per token (the LM head's
     // greedy pick), [token][workgroup]; argmax_finish reduces them
@@ -136,8 +135,7 @@ jas_status fill_normal_packed(void *x, int M, int K, uint64_t seed, uint64_t str
 // W2 (EPI_SWIGLU only) has the same shape and layout as W.
 // wbf16 (packed only): W/W2 hold bf16 elements in the packed layout, widened to fp32 on load.
 jas_status skinny_gemm(const void *W, const void *W2, const float *X, long ldx, int M, int N, int K,
-                       const SkinnyEpiArgs &epi, hipStream_t s, bool packed = false,
-                       const SkinnyTuning *tune = nullptr, bool wbf16 = false);
+                       const SkinnyEpiArgs &epi, hipStream_t s, bool packed = false, bool wbf16 = false);
 
 // Fused epilogues of the prefill GEMMs on packed weights (token-major output).
 enum FusedMode : int { FZ_NONE = 0, FZ_QKV = 1, FZ_SWIGLU = 2 };

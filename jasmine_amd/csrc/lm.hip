@@ -239,7 +239,7 @@ jas_status norm_rows(jas_lm *lm, const float *x, float *y, int n_vec, long vstri
 jas_status proj(jas_lm *lm, const float *Wt, const float *X, int N, int M, int K, const SkinnyEpiArgs &e)
 {
     TRY(prof_begin(lm, 0));
-    TRY(skinny_gemm(Wt, nullptr, X, K, M, N, K, e, lm->stream, true, nullptr, lm->wbf16()));
+    TRY(skinny_gemm(Wt, nullptr, X, K, M, N, K, e, lm->stream, true, lm->wbf16()));
     return prof_end(lm);
 }
 
@@ -331,9 +331,7 @@ jas_status decode_step(jas_lm *lm, bool device_pos)
         eq.kv_sh = lm->kv_sh;
         eq.d = d;
         eq.dh = dh;
-        eq.rope = c.kind == 1;
-        eq.theta = c.rope_theta;
-        eq.rope_tab = lm->rope_tab;
+        eq.rope_tab = lm->rope_tab;  // LLaMA only
         TRY(proj(lm, lm->LW("w_qkv", l), lm->h, B, 3 * d, d, eq));
         TRY(prof_begin(lm, 1));
         TRY(attn_decode_impl(lm->q, lm->kv_layer_ptr(lm->kc, l), lm->kv_layer_ptr(lm->vc, l), lm->att, lm->seqlens, B, H,
@@ -371,8 +369,7 @@ jas_status decode_step(jas_lm *lm, bool device_pos)
             eg.ldo = F;
             eg.out_packed = 1;
             TRY(prof_begin(lm, 0));
-            TRY(skinny_gemm(lm->LW("w_gate", l), lm->LW("w_up", l), lm->h, d, F, B, d, eg, s, true, nullptr,
-                            lm->wbf16()));
+            TRY(skinny_gemm(lm->LW("w_gate", l), lm->LW("w_up", l), lm->h, d, F, B, d, eg, s, true, lm->wbf16()));
             TRY(prof_end(lm));
             TRY(proj(lm, lm->LW("w_down", l), lm->ff, B, d, F, ed));
             pend_bias = nullptr;
@@ -704,8 +701,7 @@ jas_status jas_lm_prefill(jas_lm *lm, int B, int P, const int32_t *h_ids, int32_
     eh.ldo = V;
     eh.amax_v = lm->amax_v;
     eh.amax_i = lm->amax_i;
-    TRY(skinny_gemm(c.kind == 0 ? lm->W("wte") : lm->W("w_head"), nullptr, lm->h, d, V, B, d, eh, s, true, nullptr,
-                    lm->wbf16()));
+    TRY(skinny_gemm(c.kind == 0 ? lm->W("wte") : lm->W("w_head"), nullptr, lm->h, d, V, B, d, eh, s, true, lm->wbf16()));
     hipLaunchKernelGGL(argmax_finish_kernel, dim3(B), dim3(256), 0, s, lm->amax_v, lm->amax_i,
                        skinny_row_groups(V, d, false, false, lm->wbf16()), lm->ids, nullptr, nullptr, nullptr, B, 0);
     JAS_LAUNCH_CHECK();
@@ -836,7 +832,7 @@ jas_status jas_lm_project(jas_lm *lm, const char *name, int layer, int B, const 
         e.out = d_y;
         e.ldo = M;
     }
-    TRY(skinny_gemm(W, dual ? lm->LW("w_up", layer) : nullptr, xp, K, M, B, K, e, s, true, nullptr, lm->wbf16()));
+    TRY(skinny_gemm(W, dual ? lm->LW("w_up", layer) : nullptr, xp, K, M, B, K, e, s, true, lm->wbf16()));
     if (ks)
         hipLaunchKernelGGL(sum_splits_kernel, dim3(ceil_div((long)B * M, 256)), dim3(256), 0, s, lm->part, ks, B, M, d_y);
     JAS_LAUNCH_CHECK();
