@@ -353,6 +353,234 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
 #undef FA_LSTORE
 }
 
+// bf16 attention at D = 128, inputs and output bf16, fp32 accumulate, softmax in fp32, P rounded
+// to bf16 for the second product.  Four waves of NQ x 16 queries; K and V tiles of 64 keys lie in
+// LDS in operand order (one ds_read_b128 per fragment), V transposed by the lanes that stage it.
+// flash_prefill_kernel's 16 queries per wave read 32 KB of LDS for 544 cycles of matrix core
+// (2048 of the CU's LDS cycles against 1088); 32 queries per wave read it for twice as many.
+// MI355X, 32 heads of S 2048, not causal: 94 -> 85 us (806 TFLOP/s); 128 heads of S 1024,
+// causal: 71 -> 56.  Its four waves leave a SIMD one wave when a workgroup is alone on its CU,
+// so a causal launch of two workgroups per CU, heavy ones beside light ones, stays with the
+// eight-wave kernel (32 heads of S 2048: 55 against 64 us), as do D = 64 and 32 (28.0 against
+// 27.4, 28.8 against 24.4).
+// S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_bf16, the reduction index permuted
+// identically in both operands, so that S lands in the P operand's registers and every
+// accumulator entry of a lane belongs to the lane's own query.  Two buffers of LDS: tile t + 1
+// is written while tile t is read, one barrier per tile; loads run one tile ahead of that.
+template <int D, int NQ>
+__global__ void __launch_bounds__(256, 2) flash_bf16_kernel(const PrefillArgs p)
+{
+    constexpr int NW = 4, BK = 64, BQ = 16 * NQ * NW, CD = D / 32, NC = D / 16, NJ = BK / 16, NM = BK / 32;
+    constexpr int DW = D == 128 ? 4 : 2;           // V: adjacent d per lane and key
+    constexpr int UK = NJ * CD, UV = D / (16 * DW) * NM;  // staging units: 16 keys x 32 d, 16 DW d x 32 keys
+    constexpr int KU = (UK + NW - 1) / NW, VU = (UV + NW - 1) / NW;
+    typedef uint32_t vchunk __attribute__((ext_vector_type(DW / 2 < 2 ? 1 : 2)));
+    __shared__ u32x4 Ks[2][NJ * CD * 64];
+    __shared__ u32x4 Vs[2][NC * NM * 64];
+    const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int bh, qb, split;
+    const int nqb = (p.Sq + BQ - 1) / BQ;
+    if (!fa_work_item(nqb, p.B * p.H, p.nsplit, p.fold, bh, qb, split)) return;
+    const int b = bh / p.H, h = bh % p.H, shift = p.Sk - p.Sq;
+    const int q0 = qb * BQ + w * 16 * NQ;
+    const int q_last = min(qb * BQ + BQ - 1, p.Sq - 1);
+    const int k_lo = p.nsplit > 1 ? split * p.kchunk : 0;
+    const int k_end = p.nsplit > 1 ? min(p.Sk, k_lo + p.kchunk) : p.causal ? min(p.Sk, q_last + shift + 1) : p.Sk;
+    const int wave_kend = min(k_end, p.causal ? min(p.Sk, min(q0 + 16 * NQ - 1, p.Sq - 1) + shift + 1) : p.Sk);
+    const uint16_t *Kb = (const uint16_t *)p.K + (long)b * p.k_sb + (long)h * p.k_sh;
+    const uint16_t *Vb = (const uint16_t *)p.V + (long)b * p.k_sb + (long)h * p.k_sh;
+    // slot of row `row` of V's 16-row block blk: the lanes that store together (every DW-th row
+    // of two or more blocks) fall on different banks
+    auto vslot = [](int row, int blk) { return DW == 4 ? row ^ (row >> 2) ^ (blk & 1) : row ^ (row >> 3); };
+
+    // Q (B operand): lane (query r16, g) holds d = 32 c + 8 g .. + 7
+    bf16x8 qf[NQ][CD];
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        const int qq = min(q0 + 16 * a + r16, p.Sq - 1);
+        const uint16_t *qr = (const uint16_t *)p.Q + (long)b * p.q_sb + (long)h * p.q_sh + (long)qq * p.q_ss;
+#pragma unroll
+        for (int c = 0; c < CD; ++c) qf[a][c] = *(const bf16x8 *)(qr + 32 * c + 8 * g);
+    }
+
+    u32x4 kr[KU];
+    vchunk vr[VU][8];
+    auto gload = [&](int kv0) {
+        const bool whole = kv0 + BK <= p.Sk;  // rows past Sk: the last row (finite, masked below)
+#pragma unroll
+        for (int q = 0; q < KU; ++q) {
+            const int u = w + NW * q;
+            if (UK % NW != 0 && u >= UK) continue;
+            const int key = kv0 + 16 * (u / CD) + r16;
+            kr[q] = *(const u32x4 *)(Kb + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss + 32 * (u % CD) + 8 * g);
+        }
+#pragma unroll
+        for (int q = 0; q < VU; ++q) {
+            const int u = w + NW * q;
+            if (UV % NW != 0 && u >= UV) continue;
+            const int key0 = kv0 + 32 * (u % NM) + 4 * g;
+            const uint16_t *src = Vb + 16 * DW * (u / NM) + DW * r16;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int key = key0 + j + (j < 4 ? 0 : 12);
+                vr[q][j] = *(const vchunk *)(src + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss);
+            }
+        }
+    };
+    auto lstore = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < KU; ++q) {
+            const int u = w + NW * q;
+            if (UK % NW != 0 && u >= UK) continue;
+            Ks[buf][u * 64 + lane] = kr[q];
+        }
+#pragma unroll
+        for (int q = 0; q < VU; ++q) {
+            const int u = w + NW * q;
+            if (UV % NW != 0 && u >= UV) continue;
+#pragma unroll
+            for (int e = 0; e < DW; ++e) {
+                // element e of the eight keys: the low or high halves of word e / 2
+                u32x4 t;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    t[k] = __builtin_amdgcn_perm(vr[q][2 * k + 1][e / 2], vr[q][2 * k][e / 2], e % 2 ? 0x07060302u : 0x05040100u);
+                const int d = 16 * DW * (u / NM) + DW * r16 + e, blk = d >> 4;
+                Vs[buf][(blk * NM + u % NM) * 64 + 16 * g + vslot(d & 15, blk)] = t;
+            }
+        }
+    };
+
+    floatx4 oacc[NC][NQ], lacc[NQ];  // O^T, and the row sums as P^T times a ones operand
+    float mb[NQ], m_lane[NQ];        // exponent base and this lane's running max relative to it
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        lacc[a] = floatx4{0.f, 0.f, 0.f, 0.f}, mb[a] = 0.f, m_lane[a] = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) oacc[c][a] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    const float sl2 = p.scale_log2;
+    const bf16x8 ones = bf16x8{(__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f,
+                               (__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
+    const int vs0 = 16 * g + vslot(r16, 0), vs1 = 16 * g + vslot(r16, 1);
+
+    gload(k_lo);
+    for (int kv0 = k_lo, buf = 0; kv0 < k_end; kv0 += BK, buf ^= 1) {
+        // buffer `buf` was last read two tiles ago, before the barrier of the tile in between
+        lstore(buf);
+        gload(min(kv0 + BK, k_lo + (k_end - k_lo - 1) / BK * BK));  // (past the last tile: it again)
+        __syncthreads();
+        if (kv0 >= wave_kend) continue;  // every key masked for this wave
+        floatx4 s[NJ][NQ];
+#pragma unroll
+        for (int c = 0; c < CD; ++c)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const bf16x8 kf = __builtin_bit_cast(bf16x8, Ks[buf][(j * CD + c) * 64 + lane]);
+#pragma unroll
+                for (int a = 0; a < NQ; ++a)
+                    s[j][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        kf, qf[a][c], c == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : s[j][a], 0, 0, 0);
+            }
+        bf16x8 pf[NM][NQ];
+#pragma unroll
+        for (int a = 0; a < NQ; ++a) {
+            const int qi = q0 + 16 * a + r16;
+            // masking only on tiles that reach past Sk or cross this wave's causal diagonal: key
+            // kv0 + 16j + 4g + r is visible iff 16j + r <= lim, one compare per score
+            if (kv0 + BK > p.Sk || (p.causal && kv0 + BK - 1 > q0 + 16 * a + shift)) {
+                const int lim = (p.causal ? min(qi + shift, p.Sk - 1) : p.Sk - 1) - kv0 - 4 * g;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[j][a][r] = 16 * j + r <= lim ? s[j][a][r] : -INFINITY;
+            }
+            // exponent units relative to the base: s <- sl2 s - mb (p = 2^s below)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[j][a][r] = __builtin_fmaf(s[j][a][r], sl2, -mb[a]);
+            // Lazy rescaling with a per-lane test: the base mb moves only when the row's running
+            // max leaves [mb - 64, mb + 8].  Meanwhile p stays below 2^8, numerator and row sum
+            // share the base, and O / l is unchanged.  Each lane tests only its own running max
+            // (taken after the fma: arithmetic results need no NaN canonicalisation before a
+            // max); the row max across the four lanes, and the move itself, are computed only
+            // when some lane trips, which for most inputs happens on no tile at all.  A query
+            // with no visible key keeps -inf maxima.
+            const float m_prev = m_lane[a];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                m_lane[a] = fmaxf(fmaxf(m_lane[a], fmaxf(s[j][a][0], s[j][a][1])), fmaxf(s[j][a][2], s[j][a][3]));
+            if (__builtin_amdgcn_ballot_w64(m_lane[a] > 8.f || (m_lane[a] < -64.f && m_lane[a] != -INFINITY))) {
+                const float row_prev = max_across_rows(m_prev), row = max_across_rows(m_lane[a]);
+                if (row > 8.f || (row < -64.f && row != -INFINITY)) {
+                    // nothing accumulated yet (row_prev = -inf): factor 0, not 2^-row, which
+                    // overflows when the base moves far down
+                    const float corr = row_prev == -INFINITY ? 0.f : exp2_fast(-row);
+                    mb[a] += row;
+                    m_lane[a] -= row;
+                    lacc[a] *= corr;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) s[j][a] -= row;
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) oacc[c][a] *= corr;
+                }
+            }
+            // P^T operand for key block m (32 keys): slot t <-> key 32m + 16(t/4) + 4g + t%4,
+            // which are exactly s[2m][t] and s[2m+1][t-4] of this lane
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                float e[8];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    e[r] = exp2_fast(s[2 * m][a][r]);
+                    e[4 + r] = exp2_fast(s[2 * m + 1][a][r]);
+                }
+                pf[m][a] = bf16x8{(__bf16)e[0], (__bf16)e[1], (__bf16)e[2], (__bf16)e[3],
+                                  (__bf16)e[4], (__bf16)e[5], (__bf16)e[6], (__bf16)e[7]};
+                lacc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[m][a], lacc[a], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const bf16x8 vf = __builtin_bit_cast(bf16x8, Vs[buf][(c * NM + m) * 64 + (c & 1 ? vs1 : vs0)]);
+#pragma unroll
+                for (int a = 0; a < NQ; ++a) oacc[c][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[m][a], oacc[c][a], 0, 0, 0);
+            }
+    }
+
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        const int qi = q0 + 16 * a + r16;
+        if (qi >= p.Sq) continue;
+        const float l = lacc[a][0];
+        if (p.nsplit > 1) {  // unnormalised partial: O, then the base (exponent units) and row sum
+            float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qi) * (D + 4);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) *(floatx4 *)(row + 16 * c + 4 * g) = oacc[c][a];
+            if (g == 0) {  // (-inf: no visible key)
+                row[D] = l > 0.f ? mb[a] : -INFINITY;
+                row[D + 1] = l;
+            }
+            continue;
+        }
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        uint16_t *o = (uint16_t *)p.O + (long)b * p.o_sb + (long)h * p.o_sh + (long)qi * p.o_ss;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            u32x2 v;
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                v[k] = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][a][2 * k] * inv)) |
+                       ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(oacc[c][a][2 * k + 1] * inv)) << 16);
+            *(u32x2 *)(o + 16 * c + 4 * g) = v;
+        }
+    }
+}
+
 // One query row in fp32 arithmetic by one wave (flash_split_kernel's rare path): n keys;
 // partial: the unnormalised row, then its exponent base and sum.
 template <int D>
@@ -1170,7 +1398,9 @@ jas_status jas_attn_prefill(const void *Q, const void *K, const void *V, void *O
     if (D == DD) {                                                                                     \
         constexpr int BKV = DD == 128 ? 32 : 64, NQV = DD == 128 ? 1 : 2;                              \
         if (dtype == JAS_BF16) {                                                                       \
-            if (narrow) JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, 4>), 256)                          \
+            if (DD == 128 && narrow) JAS_FA_LAUNCH((flash_bf16_kernel<DD, 1>), 256)                    \
+            else if (DD == 128 && (!causal || items >= 1024)) JAS_FA_LAUNCH((flash_bf16_kernel<DD, 2>), 256) \
+            else if (narrow) JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, 4>), 256)                     \
             else JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, FA_WAVES>), 64 * FA_WAVES)                \
         } else {                                                                                       \
             if (narrow) JAS_FA_LAUNCH((flash_split_kernel<DD, 1, BKV>), 256)                           \

@@ -657,6 +657,30 @@ def test_attn_prefill_long_causal(jas, B, H, Sq, Sk, D, dt):
             close(do.numpy(), want, atol=1e-5, rtol=1e-4)
 
 
+# flash_bf16_kernel (D = 128) with 32 queries per wave: not causal from 256 blocks of 128
+# queries, causal from 1024; partial query blocks and key tiles
+@pytest.mark.parametrize("B,H,Sq,Sk,causal", [(4, 33, 130, 130, 0), (2, 128, 65, 200, 0), (16, 33, 129, 193, 1), (32, 32, 33, 33, 1)])
+def test_attn_prefill_bf16_wide(jas, B, H, Sq, Sk, causal):
+    import ctypes as C
+    D = 128
+
+    def bf(shape, sid):
+        x = normal(shape, 43, sid).view(np.uint32)
+        u = ((x + 0x7FFF + ((x >> 16) & 1)) >> 16).astype(np.uint16)
+        return u, (u.astype(np.uint32) << 16).view(np.float32)
+
+    (qu, Q), (ku, K), (vu, V) = bf((B, H, Sq, D), 0), bf((B, H, Sk, D), 1), bf((B, H, Sk, D), 2)
+    dq, dk, dv, do = jas.to_device(qu), jas.to_device(ku), jas.to_device(vu), jas.DeviceArray(Q.shape, np.uint16)
+    qs, ks = (H * Sq * D, Sq * D, D), (H * Sk * D, Sk * D, D)
+    jas.check(jas.lib.jas_attn_prefill(dq.p, dk.p, dv.p, do.p, B, H, Sq, Sk, D, *qs, *ks, *qs, C.c_float(1 / math.sqrt(D)),
+                                       causal, 3, None))
+    got = (do.numpy().astype(np.uint32) << 16).view(np.float32)
+    for b, h in [(0, 0), (B - 1, H - 1), (B // 2, 7)]:
+        want = _attention64(Q[b:b + 1, h:h + 1], K[b:b + 1, h:h + 1], V[b:b + 1, h:h + 1], causal)[0, 0]
+        # probabilities and the output rounded to bf16 (2^-9 each), the row sum over the rounded ones
+        assert np.abs(got[b, h] - want).max() <= 3 * 2.0 ** -9 * np.abs(V[b, h]).max()
+
+
 def _attention64(Q, K, V, causal):
     """[B, H, S, D] attention in 64 bits, causal aligned to the last key; masked keys carry nothing."""
     Q, K, V = (x.astype(np.float64) for x in (Q, K, V))
