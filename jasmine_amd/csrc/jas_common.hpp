@@ -20,9 +20,23 @@ void *workspace(size_t bytes, hipStream_t s);
 unsigned *arrival_counters(size_t n, hipStream_t s);
 // frees the stream's scratch and counters after its queued work has drained
 jas_status release_workspace(hipStream_t s);
+// The decode step's token embedding, done by its first norm: x[n] = table row ids[n] (+ wpe row
+// p), pos[n] = p and seqlens[n] = p + 1, where p is state[0] (device state under graph replay)
+// or host_pos.  layout: row-major fp32 table (LLaMA), or GPT-2's tied, packed fp32 / bf16 wte.
+enum EmbedLayout : int { EMB_NONE = 0, EMB_ROWS = 1, EMB_PACKED = 2, EMB_PACKED_B = 3 };
+struct EmbedArgs {
+    int layout = EMB_NONE;
+    const void *table = nullptr;
+    const float *wpe = nullptr;
+    const int32_t *ids = nullptr, *state = nullptr;
+    int host_pos = 0, V = 0;
+    int32_t *pos = nullptr, *seqlens = nullptr;
+};
 // x[n] += sum_s part[(s*16 + n)*d ...] + bias; y = norm(x) (RMSNorm, or LayerNorm with b)
+// emb (with ks = 0): x is the embedding, written instead of read
 jas_status resid_norm(float *x, const float *part, int ks, const float *bias, const float *g, const float *b, float *y,
-                      int N, int d, float eps, bool rms, hipStream_t s, bool y_packed = false);
+                      int N, int d, float eps, bool rms, hipStream_t s, bool y_packed = false,
+                      const EmbedArgs &emb = EmbedArgs());
 // decode attention with an optional packed-B output (o_packed_d = H*D features) for the
 // next packed GEMM; 0 = the jas_attn_decode layout O[b][h][D]
 // kv_bf16: K/V hold bf16 elements (same element strides)

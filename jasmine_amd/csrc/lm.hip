@@ -88,34 +88,6 @@ __global__ void embed_packed_kernel(const void *__restrict__ wte, const float *_
     out[g] = v;
 }
 
-
-// The decode step's first kernel: the position (from the host, or from the device state
-// under graph replay) into pos / seqlens, and the embedding of every token at it.  PACKED:
-// GPT-2's tied, packed wte plus learned positions; else LLaMA's row-major table.
-template <bool PACKED, bool WB>
-__global__ void embed_step_kernel(const void *__restrict__ wte, const float *__restrict__ wpe,
-                                  const int32_t *__restrict__ ids, const int32_t *__restrict__ state, int host_pos,
-                                  int32_t *pos, int32_t *seqlens, float *__restrict__ out, int B, int d, int V)
-{
-    const int p = state ? state[0] : host_pos;
-    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < B) {
-        pos[g] = p;
-        seqlens[g] = p + 1;
-    }
-    if (g >= (long)B * d) return;
-    const int t = (int)(g / d), e = (int)(g % d);
-    float v;
-    if (PACKED) {
-        const long off = WB ? weight_pack_offset_b(ids[t], e, d, (V + 15) >> 4) : weight_pack_offset(ids[t], e, d, (V + 15) >> 4);
-        v = WB ? bf16_to_f32(((const uint16_t *)wte)[off]) : ((const float *)wte)[off];
-    } else {
-        v = ((const float *)wte)[(long)ids[t] * d + e];
-    }
-    if (wpe) v = v + wpe[(long)p * d + e];
-    out[g] = v;
-}
-
 // The decode step's last kernel, one workgroup per sequence: the first maximum over the LM
 // head's per-workgroup picks (ties to the lowest index) into ids; under graph replay also the
 // id into the history at step pos - state[1], and (sequence 0) the device position advanced.
@@ -305,22 +277,16 @@ jas_status decode_step(jas_lm *lm, bool device_pos)
     JAS_CHECK(device_pos || lm->position < c.max_ctx, JAS_ERR_RANGE,
               "jas_lm_decode: KV cache full (max_ctx reached)");
     hipStream_t s = lm->stream;
-    {  // positions and embeddings in one launch
-        TRY(prof_begin(lm, 2));
-        const dim3 grid(ceil_div((long)B * d, 256));
-        const int32_t *st = device_pos ? lm->dstate : nullptr;
-        if (c.kind == 0 && lm->wbf16())
-            hipLaunchKernelGGL((embed_step_kernel<true, true>), grid, dim3(256), 0, s, lm->W("wte"), lm->W("wpe"),
-                               lm->ids, st, lm->position, lm->pos, lm->seqlens, lm->x, B, d, V);
-        else if (c.kind == 0)
-            hipLaunchKernelGGL((embed_step_kernel<true, false>), grid, dim3(256), 0, s, lm->W("wte"), lm->W("wpe"),
-                               lm->ids, st, lm->position, lm->pos, lm->seqlens, lm->x, B, d, V);
-        else
-            hipLaunchKernelGGL((embed_step_kernel<false, false>), grid, dim3(256), 0, s, lm->W("wte"), nullptr,
-                               lm->ids, st, lm->position, lm->pos, lm->seqlens, lm->x, B, d, V);
-        JAS_LAUNCH_CHECK();
-        TRY(prof_end(lm));
-    }
+    EmbedArgs emb;  // positions and embeddings: layer 0's first norm
+    emb.layout = c.kind == 1 ? EMB_ROWS : lm->wbf16() ? EMB_PACKED_B : EMB_PACKED;
+    emb.table = lm->W("wte");
+    emb.wpe = c.kind == 0 ? lm->W("wpe") : nullptr;
+    emb.ids = lm->ids;
+    emb.state = device_pos ? lm->dstate : nullptr;
+    emb.host_pos = lm->position;
+    emb.V = V;
+    emb.pos = lm->pos;
+    emb.seqlens = lm->seqlens;
     // The projections that feed the residual stream (O and down/proj) run K-split and leave
     // their partial sums in lm->part; the next norm kernel adds them (plus the bias) to x.
     int pend_ks = 0;
@@ -328,7 +294,7 @@ jas_status decode_step(jas_lm *lm, bool device_pos)
     for (int l = 0; l < c.n_layer; ++l) {
         TRY(prof_begin(lm, 2));
         TRY(resid_norm(lm->x, lm->part, pend_ks, pend_bias, lm->LW("ln1_g", l), lm->LW("ln1_b", l), lm->h, B, d,
-                       c.eps, c.kind == 1, s, true));
+                       c.eps, c.kind == 1, s, true, l == 0 ? emb : EmbedArgs()));
         TRY(prof_end(lm));
         SkinnyEpiArgs eq;
         eq.mode = EPI_QKV;

@@ -7,6 +7,7 @@
 // HBM once and written once: wave64 shuffles (DPP) reduce inside a wave, LDS across waves.
 // Column-wise forms (jasmine's feature-major [d, T] LayerNorm normalises each column) map
 // one thread per column so the loads stay coalesced across columns.
+#include "gemm.hpp"
 #include "jas_leaf.hpp"
 
 #include <cfloat>
@@ -706,16 +707,24 @@ static jas_status reduce_t(const jas_leaf *in, int op, int axis, void *d_out, hi
 // x[n] += (sum_s part[s][n] + bias); y[n] = norm(x[n]) * g (+ b).  `part` holds the K-split
 // partial sums of the projection that feeds the residual stream ([split][16][d], split
 // order), so the split-K reduction costs no launch of its own.  One workgroup per token.
+// EMB: the step's first norm makes the embedding itself (EmbedArgs).  It waits for ids and then
+// for the table row, where a kernel of its own waited for the same and cost a launch more:
+// 3 us per step on MI355X (two-layer d 128 model, 32 tokens: 2009 -> 1911 us).
 constexpr int RN_MAX_SPLITS = 8;  // the decode projections split K at most 8 ways
-template <int PER, bool RMS, int NT>
+template <int PER, bool RMS, int NT, int EMB>
 __global__ void __launch_bounds__(NT)
 resid_norm_kernel(float *__restrict__ x, const float *__restrict__ part, int ks, const float *__restrict__ bias,
                   const float *__restrict__ g, const float *__restrict__ bta, float *__restrict__ y, int d, float eps,
-                  int y_packed)
+                  int y_packed, EmbedArgs emb)
 {
     __shared__ float red[NT / 64];
     const int n = blockIdx.x, t = threadIdx.x;
     float *xr = x + (long)n * d;
+    const int id = EMB ? emb.ids[n] : 0, p = EMB ? (emb.state ? emb.state[0] : emb.host_pos) : 0;
+    if (EMB && t == 0) {
+        emb.pos[n] = p;
+        emb.seqlens[n] = p + 1;
+    }
     float v[PER];
     // the norm's gain (and bias) are requested together with the row, not after the
     // reductions: one memory round trip fewer on the critical path
@@ -731,8 +740,24 @@ resid_norm_kernel(float *__restrict__ x, const float *__restrict__ part, int ks,
         const int e = (k * NT + t) * 4;
         float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
         if (e < d) {
-            a = *(const float4 *)(xr + e);
-            if (ks > 0) {
+            if (EMB) {  // features e..e+3 of a row are adjacent in each layout
+                if (EMB == EMB_PACKED_B) {
+                    const long off = weight_pack_offset_b(id, e, d, (emb.V + 15) >> 4);
+                    const floatx4 w = widen_bf16x4(*(const u32x2 *)((const uint16_t *)emb.table + off));
+                    a = make_float4(w[0], w[1], w[2], w[3]);
+                } else {
+                    const long off = EMB == EMB_PACKED ? weight_pack_offset(id, e, d, (emb.V + 15) >> 4) : (long)id * d + e;
+                    a = *(const float4 *)((const float *)emb.table + off);
+                }
+                if (emb.wpe) {
+                    const float4 w = *(const float4 *)(emb.wpe + (long)p * d + e);
+                    a.x += w.x; a.y += w.y; a.z += w.z; a.w += w.w;
+                }
+                *(float4 *)(xr + e) = a;
+            } else {
+                a = *(const float4 *)(xr + e);
+            }
+            if (!EMB && ks > 0) {
                 // every split's partial is requested before the first is added (one round
                 // trip, not ks); the sum keeps split order
                 float4 q[RN_MAX_SPLITS];
@@ -787,25 +812,32 @@ resid_norm_kernel(float *__restrict__ x, const float *__restrict__ part, int ks,
 }
 
 jas_status resid_norm(float *x, const float *part, int ks, const float *bias, const float *g, const float *b, float *y,
-                      int N, int d, float eps, bool rms, hipStream_t s, bool y_packed)
+                      int N, int d, float eps, bool rms, hipStream_t s, bool y_packed, const EmbedArgs &emb)
 {
     JAS_CHECK(d % 4 == 0 && d <= 8192 && N >= 1 && N <= 16 && g, JAS_ERR_INVALID, "resid_norm: unsupported shape");
     JAS_CHECK(ks <= RN_MAX_SPLITS, JAS_ERR_INVALID, "resid_norm: more K splits than supported");
     JAS_CHECK(!y_packed || d % 16 == 0, JAS_ERR_INVALID, "resid_norm: packed output needs d % 16 == 0");
+    JAS_CHECK(emb.layout == EMB_NONE || (ks == 0 && rms == (emb.layout == EMB_ROWS)), JAS_ERR_INVALID,
+              "resid_norm: embedding layout does not go with this norm");
     const int yp = y_packed ? 1 : 0;
-#define JAS_RN(PER, NT)                                                                                      \
-    if (d <= PER * NT) {                                                                                     \
-        if (rms) hipLaunchKernelGGL((resid_norm_kernel<PER, true, NT>), dim3(N), dim3(NT), 0, s, x, part, ks, \
-                                    bias, g, b, y, d, eps, yp);                                              \
-        else hipLaunchKernelGGL((resid_norm_kernel<PER, false, NT>), dim3(N), dim3(NT), 0, s, x, part, ks,   \
-                                bias, g, b, y, d, eps, yp);                                                  \
-        JAS_LAUNCH_CHECK();                                                                                  \
-        return JAS_OK;                                                                                       \
+#define JAS_RN_GO(PER, RMS, NT, EMB)                                                                          \
+    hipLaunchKernelGGL((resid_norm_kernel<PER, RMS, NT, EMB>), dim3(N), dim3(NT), 0, s, x, part, ks, bias, g, \
+                       b, y, d, eps, yp, emb)
+#define JAS_RN(PER, NT)                                                                                       \
+    if (d <= PER * NT) {                                                                                      \
+        if (rms && emb.layout == EMB_NONE) JAS_RN_GO(PER, true, NT, EMB_NONE);                                \
+        else if (rms) JAS_RN_GO(PER, true, NT, EMB_ROWS);                                                     \
+        else if (emb.layout == EMB_NONE) JAS_RN_GO(PER, false, NT, EMB_NONE);                                 \
+        else if (emb.layout == EMB_PACKED) JAS_RN_GO(PER, false, NT, EMB_PACKED);                             \
+        else JAS_RN_GO(PER, false, NT, EMB_PACKED_B);                                                         \
+        JAS_LAUNCH_CHECK();                                                                                   \
+        return JAS_OK;                                                                                        \
     }
     // one float4 per thread up to d = 4096 (more waves per token: the partial loads are
     // spread over 16 waves instead of 4); wider rows take 8 features per thread
     JAS_RN(4, 256) JAS_RN(4, 512) JAS_RN(4, 1024) JAS_RN(8, 1024)
 #undef JAS_RN
+#undef JAS_RN_GO
     return fail(JAS_ERR_INVALID, "resid_norm: d too large");
 }
 

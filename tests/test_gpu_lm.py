@@ -87,6 +87,25 @@ def test_ragged_chunk_widths(jas, kind, d, H, F, V):
     run_parity(jas, cfg, seed=9, B=4, P=13, steps=6, prompt_seed=9)
 
 
+@pytest.mark.parametrize("d,H", [(64, 2), (1088, 17), (4160, 65)])
+@pytest.mark.parametrize("kind,wb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_decode_embedding(jas, kind, wb, d, H):
+    """The embedding made by layer 0's norm: partly idle, two- and four-round workgroups (256,
+    512 and 1024 threads of four or eight features), vocabularies of one row past a packed tile,
+    each table layout, decoded up to the last cache position (last wpe row), eager against the
+    oracle (run_parity's tolerance) and then replayed as a graph against the eager ids."""
+    B, P = 3, 5
+    cfg = jas.LmConfig(kind, 1, d, H, 32, 17, 12, B, 1e-5, 10000.0, wb, 0)
+    lm, prompt, cpu_ids, ties = run_parity(jas, cfg, seed=31 + d, B=B, P=P, steps=8, prompt_seed=9)
+    first, _ = lm.prefill(prompt)
+    eager, nxt = [first], first
+    for _ in range(7):
+        nxt, _ = lm.decode(nxt)
+        eager.append(nxt)
+    first, _ = lm.prefill(prompt)
+    assert np.array_equal(np.concatenate([first[:, None], lm.generate(7, B).T], 1), np.stack(eager, 1))
+
+
 def bf16_round(a):
     """fp32 -> bf16 -> fp32, round to nearest even (finite inputs)."""
     u = np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.uint64)
