@@ -340,20 +340,20 @@ __device__ __forceinline__ void split_epilogue(const SplitArgs &p, float *C, con
     }
 }
 
-// Large products.  TM x TN tile, NW waves in a WGM x (NW / WGM) grid, ST slabs of LDS.  A
+// Large products.  TM x TN tile, NW waves in a WGM x (NW / WGM) grid, two slabs of LDS.  A
 // workgroup splits each element once; per slab and CU a 256 x 128 tile needs 3072 cycles of
 // matrix core, about 900 of vector ALU, 2100 of LDS.  MI355X, 4096^3: 1083 us on the fp32
 // matrix cores (127 TFLOP/s), 690 us here (199 TFLOP/s of fp32 products, 1.2 PFLOP/s of bf16
 // ones, the rate a plain bf16 product of this size reaches).
-template <int AM, int BM, int TM, int TN, int NW, int WGM, int ST>
-__global__ void __launch_bounds__(NW * 64, ST == 2 ? 2 : 3) gemm_split_kernel(const SplitArgs p)
+template <int AM, int BM, int TM, int TN, int NW, int WGM>
+__global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs p)
 {
     constexpr int WGN = NW / WGM, NBI = TM / WGM / 16, NBJ = TN / WGN / 16;
     using LA = SplitLoader<AM, TM, NW>;
     using LB = SplitLoader<BM, TN, NW>;
     constexpr int PA = LA::PL, SA = PA * TM * 4, SB = 3 * TN * 4;  // 16-byte units per stage
     static_assert(LB::PL == 3, "B is fp32");
-    __shared__ u32x4 lds[ST * (SA + SB)];
+    __shared__ u32x4 lds[2 * (SA + SB)];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = w / WGN, wn = w % WGN, r16 = lane & 15, g = lane >> 4;
@@ -418,14 +418,12 @@ __global__ void __launch_bounds__(NW * 64, ST == 2 ? 2 : 3) gemm_split_kernel(co
         la.load(ra, k0, w, lane);
         lb.load(rb, k0, wb, lane);
     };
-    // Two stages: slab s goes to stage s % 2, which was last read two slabs ago, before the
-    // barrier of the slab in between, so one barrier per slab does.  One stage: a barrier before
-    // the store too, and up to four workgroups per CU that cover it.  The loads of the next slab are issued whether or
+    // Slab s goes to stage s % 2, which was last read two slabs ago, before the barrier of the
+    // slab in between: one barrier per slab.  The loads of the next slab are issued whether or
     // not it exists (past the last one: the last again), so the wait counts do not depend on
     // the path.
     auto step = [&](int s, bool more) {
-        u32x4 *sa = lds + (ST == 2 ? s & 1 : 0) * (SA + SB);
-        if (ST == 1) __syncthreads();  // every wave has read the previous slab
+        u32x4 *sa = lds + (s & 1) * (SA + SB);
         la.store(ra, sa, w, lane, mx);
         lb.store(rb, sa + SA, wb, lane, mx);
         if (more) fetch(min(s + 1, nk - 1) * 32);
@@ -672,10 +670,10 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
     }
 }
 
-template <int AM, int BM, int TM, int TN, int NW, int WGM, int ST>
+template <int AM, int BM, int TM, int TN, int NW, int WGM>
 static void launch_tile(const SplitArgs &p, int batch, hipStream_t s)
 {
-    hipLaunchKernelGGL((gemm_split_kernel<AM, BM, TM, TN, NW, WGM, ST>), dim3(ceil_div(p.N, TN), ceil_div(p.M, TM), batch),
+    hipLaunchKernelGGL((gemm_split_kernel<AM, BM, TM, TN, NW, WGM>), dim3(ceil_div(p.N, TN), ceil_div(p.M, TM), batch),
                        dim3(NW * 64), 0, s, p);
 }
 template <int AM, int BM, int NBI, int NBJ, int NW, int PD>
@@ -691,8 +689,6 @@ static void launch_wave_split(const SplitArgs &p, int batch, hipStream_t s)
 //   256 x 128 tiles when their rounds over the CUs are at least four fifths full: 12288 x 2048
 //     x 4096 1075 (128 x 64: 1320, 64 x 64: 1250); but 2304 x 4096 x 768, 288 tiles, 166 (123)
 //   128 x 64 for a long K with two tiles per CU: 2048^3 109 (64 x 64: 153, 256 x 128: 175)
-//   128 x 64 in one stage for a short K with four tiles per CU: 2304 x 4096 x 768 116 (64 x 64:
-//     125), 3072 x 4096 x 768 139 (160)
 //   64 x 64, four waves on K: 768 x 4096 x 768 and x 3072 138 (128 x 64: 171, 64 x 32: 146)
 //   64 x 32, four waves: 3072 x 509 x 768 28 (64 x 64: 37, 32 x 32: 38); 1024^3 22 (35, 32)
 //   64 x 32, eight waves, when that leaves CUs idle but 32 x 32 would need a second round:
@@ -706,9 +702,8 @@ static void launch_split(const SplitArgs &p, int batch, hipStream_t s)
 {
     auto tiles = [&](int a, int b) { return (long)ceil_div(p.M, a) * ceil_div(p.N, b) * batch; };
     const long big = tiles(256, 128);
-    if (big >= 256 && big * 5 >= (big + 255) / 256 * 256 * 4) launch_tile<AM, BM, 256, 128, 8, 4, 2>(p, batch, s);
-    else if (tiles(128, 64) >= 512 && p.K >= 1024) launch_tile<AM, BM, 128, 64, 4, 2, 2>(p, batch, s);
-    else if (tiles(128, 64) >= 1024) launch_tile<AM, BM, 128, 64, 4, 4, 1>(p, batch, s);
+    if (big >= 256 && big * 5 >= (big + 255) / 256 * 256 * 4) launch_tile<AM, BM, 256, 128, 8, 4>(p, batch, s);
+    else if (tiles(128, 64) >= 512 && p.K >= 1024) launch_tile<AM, BM, 128, 64, 4, 2>(p, batch, s);
     else if (tiles(64, 64) >= 768) launch_wave_split<AM, BM, 4, 4, 4, 1>(p, batch, s);
     else if (p.K <= 128) launch_wave_split<AM, BM, 2, 2, 4, 0>(p, batch, s);
     else if (tiles(64, 32) >= 256) launch_wave_split<AM, BM, 4, 2, 4, 2>(p, batch, s);
