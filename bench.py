@@ -346,7 +346,7 @@ def run_kernel_legs(jas, reps=10):
         chk(lib.jas_attn_prefill(q.p, k.p, v.p, o.p, Bb, H, S, S, Dh, *st, *st, *st, C.c_float(0.125), 1, dt, None))
 
     ms = time_launches(lambda: prefill(Q, K, V, O, 0), reps)
-    out["attn_prefill_f32"] = line("flash_prefill_kernel<64> fp32 causal, B8 H12 S1024 D64", ms, None, "mfma",
+    out["attn_prefill_f32"] = line("flash_split_kernel<64> fp32 causal, B8 H12 S1024 D64", ms, None, "mfma",
                                    causal_flops, FP32_MFMA_TFLOPS)
 
     def bf(x):

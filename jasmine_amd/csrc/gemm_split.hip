@@ -690,6 +690,9 @@ static void launch_wave_split(const SplitArgs &p, int batch, hipStream_t s)
 //     x 4096 1075 (128 x 64: 1320, 64 x 64: 1250); but 2304 x 4096 x 768, 288 tiles, 166 (123)
 //   128 x 64 for a long K with two tiles per CU: 2048^3 109 (64 x 64: 153, 256 x 128: 175)
 //   64 x 64, four waves on K: 768 x 4096 x 768 and x 3072 138 (128 x 64: 171, 64 x 32: 146)
+//     (128 x 64 in one LDS stage is 7-13 % faster for a short K with many tiles, but the error
+//     of its one long chain does not average out over the keys that attention sums:
+//     GPT-2-small decode logits 6.0e-7 from 64 bits, against 5.1e-7 here and on fp32 MFMA)
 //   64 x 32, four waves: 3072 x 509 x 768 28 (64 x 64: 37, 32 x 32: 38); 1024^3 22 (35, 32)
 //   64 x 32, eight waves, when that leaves CUs idle but 32 x 32 would need a second round:
 //     2304 x 100 x 768 12.4 (four waves 13.8, 32 x 32 16.2)
