@@ -25,13 +25,17 @@
 //
 // Numbers outside the split's range.  Infinities, NaN and magnitudes that round to infinity
 // in bf16 make the six-product sum non-finite.  Magnitudes below 2^-110 lose the bits of m and
-// l under bf16's smallest step: at most 2^-134 per element, so an error of at most
-// K 2^-134 (max|A| + max|B|) in a sum -- more than 2^-24 of it only if the sum is below
-// K 2^-110 (max|A| + max|B|).  Sums that are non-finite or that small (and not zero) are
-// computed again in fp32 arithmetic (SplitRange).
+// l under bf16's smallest step, below 2^-134 all of h too: at most 2^-134 per element, so an
+// error of at most K 2^-134 (max|A| + max|B|) in a sum -- more than 2^-24 of it only if the sum
+// is below K 2^-110 (max|A| + max|B|), which a sum of zero always is.  A tile with such a sum is
+// looked over for operands below 2^-110 that are not zero; if it has one, or a sum that is not
+// finite, it is computed again on the fp32 matrix cores (SplitRange).  MI355X, 1024^3, 24 us: 31
+// where every tile is looked over (a row of zeros in each), 55 where every one is computed again;
+// 4096 x 4096 x 1024, 212 us: 255 and 670.
 #include "gemm.hpp"
 #include "split.hpp"
 
+#include <cfloat>
 #include <type_traits>
 #include <utility>
 
@@ -40,13 +44,22 @@ namespace jas {
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // rows need not be aligned
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// whether a six-product sum needs fp32 arithmetic: non-finite, or nonzero and below the bound
+// Extremes of a lane's six-product sums, and what they call for
 struct SplitRange {
-    float small;
-    __device__ __forceinline__ SplitRange(float largest, int K) : small(2.f * (float)K * 0x1p-110f * largest) {}
-    __device__ __forceinline__ bool outside(float v) const
+    float hi = 0.f, lo = INFINITY;
+    __device__ __forceinline__ void add(floatx4 v)
     {
-        return !(fabsf(v) <= 3.4028234663852886e38f) || (fabsf(v) < small && v != 0.f);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            hi = __builtin_elementwise_maximum(hi, fabsf(v[r]));  // propagates NaN
+            lo = fminf(lo, fabsf(v[r]));
+        }
+    }
+    enum : int { OK = 0, LOOK = 1, REDO = 2 };
+    // limit: the largest number, or less where further sums follow; largest: operand magnitude
+    __device__ __forceinline__ int check(float limit, float largest, int K) const
+    {
+        return !(hi <= limit) ? REDO : lo < 2.f * (float)K * 0x1p-110f * largest ? LOOK : OK;
     }
 };
 
@@ -228,6 +241,21 @@ struct SplitLoader {
         }
     }
 
+    // whether a slab in registers has a nonzero value below 2^-110 (bf16 weights need no split)
+    __device__ __forceinline__ static bool has_tiny(const regs_t &r, int w)
+    {
+        bool tiny = false;
+        if constexpr (MODE != SM_PKB) {
+#pragma unroll
+            for (int q = 0; q < UPW; ++q)
+                if (mine(w, q)) {
+#pragma unroll
+                    for (int e = 0; e < NR; ++e) tiny |= 2 * __float_as_uint(r[q][e]) - 1 < 2 * __float_as_uint(0x1p-110f) - 1;
+                }
+        }
+        return tiny;
+    }
+
     // one element (the fp32 recomputation); zero from K on
     __device__ __forceinline__ static float element(const float *X, const float *X2, long so, long sk, int o, int k, int Olim,
                                                     int K)
@@ -248,6 +276,59 @@ struct SplitLoader {
         return X[o * so + k * sk];
     }
 };
+
+// acc += A B over k = first + g, first + stride + g, ... below K on the fp32 matrix cores, operands
+// element by element: blocks of 16 rows from m on and 16 columns from n on
+template <typename LA, typename LB, int NBI, int NBJ>
+__device__ __forceinline__ void multiply_fp32(const SplitArgs &p, const float *A, const float *B, int m, int n, int first,
+                                              int stride, int lane, floatx4 (&acc)[NBI][NBJ])
+{
+    // addresses of its own: those of the main loop would otherwise be kept in registers throughout
+    asm volatile("" : "+v"(lane));
+    const int r16 = lane & 15, g = lane >> 4;
+#pragma unroll 1
+    for (int k = first; k < p.K; k += stride) {  // (the same count for every lane; element() is zero from K on)
+        float av[NBI], bv[NBJ];
+#pragma unroll
+        for (int i = 0; i < NBI; ++i)
+            av[i] = LA::element(A, p.fz.A2, p.as0, p.as1, min(m + 16 * i + r16, p.M - 1), k + g, p.M, p.K);
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j)
+            bv[j] = LB::element(B, nullptr, p.bs1, p.bs0, min(n + 16 * j + r16, p.N - 1), k + g, p.N, p.K);
+#pragma unroll
+        for (int i = 0; i < NBI; ++i)
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+}
+
+// Whether slabs first, first + step, ... of a tile hold a nonzero operand below 2^-110, in wave wa's
+// units of A and wave wb's of B
+template <typename LA, typename LB>
+__device__ __forceinline__ bool tiny_operand(const SplitArgs &p, const float *A, const float *B, int m0, int n0, int first,
+                                             int step, int wa, int wb, int lane)
+{
+    asm volatile("" : "+v"(lane));  // (as above)
+    LA la;
+    LB lb;
+    la.init(A, p.fz.A2, p.as0, p.as1, m0, p.M, p.K, wa, lane);
+    lb.init(B, nullptr, p.bs1, p.bs0, n0, p.N, p.K, wb, lane);
+    bool tiny = false;
+#pragma unroll 1
+    for (int k0 = first * 32; k0 < p.K; k0 += step * 32) {
+        typename LA::regs_t ra;
+        typename LB::regs_t rb;
+        if (k0 + 32 <= p.K) {
+            la.load(ra, k0, wa, lane);
+            lb.load(rb, k0, wb, lane);
+        } else {
+            la.load_tail(ra, k0, wa, lane);
+            lb.load_tail(rb, k0, wb, lane);
+        }
+        tiny |= LA::has_tiny(ra, wa) || LB::has_tiny(rb, wb);
+    }
+    return tiny;
+}
 
 // Workgroup ids are remapped so that each of the 8 XCDs (ids go round-robin over them)
 // works on a contiguous range of tiles, walked 4 tile rows at a time: the A rows and B
@@ -446,32 +527,21 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
     float largest = smax[0];
 #pragma unroll
     for (int k = 1; k < NW; ++k) largest = fmaxf(largest, smax[k]);
-    const SplitRange range(largest, K);
-    bool redo = false;
+    SplitRange range;
 #pragma unroll
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
-        for (int j = 0; j < NBJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) redo |= range.outside(acc[i][j][r]);
-    if (__syncthreads_or(redo)) {
-#pragma unroll
-        for (int i = 0; i < NBI; ++i)
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-        for (int k = g; k < K + g; k += 4) {
-            float av[NBI], bv[NBJ];
-#pragma unroll
-            for (int i = 0; i < NBI; ++i)
-                av[i] = LA::element(A, p.fz.A2, p.as0, p.as1, min(m0 + (wm * NBI + i) * 16 + r16, p.M - 1), k, p.M, K);
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j)
-                bv[j] = LB::element(B, nullptr, p.bs1, p.bs0, min(n0 + (wn * NBJ + j) * 16 + r16, p.N - 1), k, p.N, K);
+        for (int j = 0; j < NBJ; ++j) range.add(acc[i][j]);
+    const int need = range.check(FLT_MAX, largest, K);
+    if (__syncthreads_or(need)) {
+        bool redo = need == SplitRange::REDO;
+        if (!__syncthreads_or(redo)) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, 0, 1, w, wb, lane);
+        if (__syncthreads_or(redo)) {
 #pragma unroll
             for (int i = 0; i < NBI; ++i)
 #pragma unroll
-                for (int j = 0; j < NBJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            multiply_fp32<LA, LB>(p, A, B, m0 + wm * NBI * 16, n0 + wn * NBJ * 16, 0, 4, lane, acc);
         }
     }
 
@@ -509,7 +579,7 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
     using LB = SplitLoader<BM, TN, 1>;
     constexpr int PA = LA::PL;
     __shared__ floatx4 red[NW][NBLK][64];
-    __shared__ float smax[NW];
+    __shared__ int need[NW];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -534,7 +604,7 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
         for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float mx = 0.f;
+    float mx = 0.f;  // largest magnitude this wave has split
     auto compute = [&](const typename LA::regs_t &ra, const typename LB::regs_t &rb) {
         bf16x8 b[NBJ][3];
 #pragma unroll
@@ -625,17 +695,38 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
             compute(ra[0], rb[0]);
         }
     }
+    // the bound on a sum holds for each wave's part of K, and eight sums of up to 2^124 add up in range
+    SplitRange range;
 #pragma unroll
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
-        for (int j = 0; j < NBJ; ++j) red[w][i * NBJ + j][lane] = acc[i][j];
-    mx = wave_max(mx);
-    if (lane == 0) smax[w] = mx;
+        for (int j = 0; j < NBJ; ++j) {
+            red[w][i * NBJ + j][lane] = acc[i][j];
+            range.add(acc[i][j]);
+        }
+    const int mine = range.check(0x1p124f, wave_max(mx), K);
+    const bool redo_w = __builtin_amdgcn_ballot_w64(mine == SplitRange::REDO), look_w = __builtin_amdgcn_ballot_w64(mine);
+    if (lane == 0) need[w] = redo_w ? SplitRange::REDO : look_w ? SplitRange::LOOK : SplitRange::OK;
     __syncthreads();
-    float largest = smax[0];
+    int any = 0;
 #pragma unroll
-    for (int k = 1; k < NW; ++k) largest = fmaxf(largest, smax[k]);
-    const SplitRange range(largest, K);
+    for (int k = 0; k < NW; ++k) any |= need[k];
+    if (any) {
+        bool redo = any & SplitRange::REDO;
+        if (!redo) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, w, NW, 0, 0, lane);
+        if (__syncthreads_or(redo)) {  // (red is read after the barrier below)
+#pragma unroll
+            for (int i = 0; i < NBI; ++i)
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            multiply_fp32<LA, LB>(p, A, B, m0, n0, 4 * w, 4 * NW, lane, acc);
+#pragma unroll
+            for (int i = 0; i < NBI; ++i)
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j) red[w][i * NBJ + j][lane] = acc[i][j];
+            __syncthreads();
+        }
+    }
     float *C = p.C + bz * p.cbs;
     const bool pairs = p.fz.mode == FZ_SWIGLU;  // gate block i with up block i + 1
     const int n_items = pairs ? NBLK / 2 : NBLK;
@@ -646,22 +737,6 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
             floatx4 v = red[0][ii * NBJ + j][lane];
 #pragma unroll
             for (int k = 1; k < NW; ++k) v += red[k][ii * NBJ + j][lane];
-            bool redo = false;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) redo |= range.outside(v[r]);
-            if (redo) {  // this lane's four sums again, in fp32
-                const int nc = min(n, p.N - 1);
-                floatx4 f = floatx4{0.f, 0.f, 0.f, 0.f};
-                for (int k = 0; k < K; ++k) {
-                    const float bk = LB::element(B, nullptr, p.bs1, p.bs0, nc, k, p.N, K);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        f[r] = __builtin_fmaf(LA::element(A, p.fz.A2, p.as0, p.as1, min(m0 + 16 * ii + 4 * g + r, p.M - 1), k,
-                                                          p.M, K),
-                                              bk, f[r]);
-                }
-                v = f;
-            }
             return v;
         };
         if (b != w) eo.load(p, bias, m, n);

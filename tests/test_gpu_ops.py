@@ -554,6 +554,35 @@ def test_gemm_split_range(jas, M, N, K):
     assert np.isinf(got[20, 30]) and got[20, 30] > 0
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (2050, 2100, 1056), (1030, 1900, 96), (96, 64, 640), (200, 90, 120)])
+def test_gemm_split_subnormal(jas, M, N, K):
+    """Operands below 2^-110, subnormal ones and ones below the smallest bf16 among them, against
+    partners large enough that their products are ordinary numbers, and next to ordinary
+    operands; sums that cancel down to those products' size."""
+    A, B = normal((M, K), 37, 0), normal((K, N), 37, 1)
+    A[3] *= np.float32(2.0 ** -136)                      # a few bits above 2^-149
+    A[5] = np.float32(2.0 ** -149)
+    A[7] *= np.float32(2.0 ** -125)
+    A[9] = 0
+    A[9, ::2], A[9, 1::2] = np.float32(2.0 ** -120 * (1 + 2.0 ** -20)), np.float32(-2.0 ** -120)
+    B[:, 2] *= np.float32(2.0 ** 100)
+    B[:, 4] = np.float32(2.0 ** 60)
+    B[:, 6] *= np.float32(2.0 ** -130)
+    A[11] *= np.float32(2.0 ** 95)
+    dA, dB, dC = jas.to_device(A), jas.to_device(B), jas.DeviceArray((M, N))
+    jas.check(jas.lib.jas_gemm(M, N, K, dA.p, K, 1, dB.p, N, 1, dC.p, N, 1, None, 0, 0, 0, 1, 0, 0, 0, 0, None))
+    got = dC.numpy()
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    mag = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    assert np.any(A[3] != 0) and abs(want[5, 2]) > 2.0 ** -60
+    fin = mag < 2.0 ** 127  # row 11 overflows against columns 2 and 4
+    assert np.sum(~fin) == 2
+    # each product's rounding and those of the running sum (2^-24, below the sum of magnitudes),
+    # and of subnormal sums (2^-149)
+    bound = (K + 2) * (2.0 ** -24 * mag[fin] + 2.0 ** -149)
+    assert np.all(np.abs(got[fin] - want[fin]) <= bound), float(np.nanmax(np.abs(got[fin] - want[fin]) / bound))
+
+
 def test_gemm_dma_k_tail_padded_rows(jas):
     """K not a multiple of 4 with 16-byte aligned, padded rows (K-contiguous operands take the
     direct-to-LDS path): the tail slab reads element by element and zero-fills past K."""
