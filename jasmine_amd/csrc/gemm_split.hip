@@ -31,7 +31,8 @@
 // looked over for operands below 2^-110 that are not zero; if it has one, or a sum that is not
 // finite, it is computed again on the fp32 matrix cores (SplitRange).  MI355X, 1024^3, 24 us: 31
 // where every tile is looked over (a row of zeros in each), 55 where every one is computed again;
-// 4096 x 4096 x 1024, 212 us: 255 and 670.
+// 4096 x 4096 x 1024, 212 us: 255 and 670.  Beside packed bf16 weights, which need no split, the
+// activations are split times 2^16, which loses nothing, and only sums that are not finite count.
 #include "gemm.hpp"
 #include "split.hpp"
 
@@ -63,9 +64,11 @@ struct SplitRange {
     }
 };
 
-// One operand X(o, k) of a workgroup: its T x 32 slabs from memory to registers to LDS.
+// One operand X(o, k) of a workgroup: its T x 32 slabs from memory to registers to LDS.  SCALED: its
+// planes are those of 2^16 X, exact for every magnitude up to 2^111 (beside bf16 weights, whose
+// magnitudes are not tracked).
 // A wave moves units of 16 rows (32 outer-contiguous ones); unit u belongs to wave u % NW.
-template <int MODE, int T, int NW>
+template <int MODE, int T, int NW, bool SCALED = false>
 struct SplitLoader {
     static constexpr int OW = MODE == SM_OC ? 32 : 16, UNITS = T / OW, UPW = (UNITS + NW - 1) / NW;
     static constexpr int NR = MODE == SM_OC ? 16 : MODE == SM_PKB ? 4 : 8;
@@ -198,9 +201,9 @@ struct SplitLoader {
             float x[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = r[q][j];
-            track_max(mx, x);
+            if constexpr (!SCALED) track_max(mx, x);
             u32x4 h, m, l;
-            split8(x, h, m, l);
+            split8<SCALED>(x, h, m, l);
             pl[0] = __builtin_bit_cast(bf16x8, h);
             pl[1] = __builtin_bit_cast(bf16x8, m);
             pl[2] = __builtin_bit_cast(bf16x8, l);
@@ -229,8 +232,8 @@ struct SplitLoader {
 #pragma unroll
                     for (int j = 0; j < 8; ++j) x[j] = r[q][R * j + e];
                     u32x4 h, m, l;
-                    track_max(mx, x);
-                    split8(x, h, m, l);
+                    if constexpr (!SCALED) track_max(mx, x);
+                    split8<SCALED>(x, h, m, l);
                     const int row = MODE == SM_OC ? 2 * (i & 7) + e : i, blk = MODE == SM_OC ? 2 * u + (i >> 3) : u;
                     u32x4 *d = lds + blk * 64 + slot_of(row, g);
                     d[0] = h;
@@ -431,7 +434,7 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
 {
     constexpr int WGN = NW / WGM, NBI = TM / WGM / 16, NBJ = TN / WGN / 16;
     using LA = SplitLoader<AM, TM, NW>;
-    using LB = SplitLoader<BM, TN, NW>;
+    using LB = SplitLoader<BM, TN, NW, AM == SM_PKB>;
     constexpr int PA = LA::PL, SA = PA * TM * 4, SB = 3 * TN * 4;  // 16-byte units per stage
     static_assert(LB::PL == 3, "B is fp32");
     __shared__ u32x4 lds[2 * (SA + SB)];
@@ -533,10 +536,12 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
 #pragma unroll
         for (int j = 0; j < NBJ; ++j) range.add(acc[i][j]);
     const int need = range.check(FLT_MAX, largest, K);
+    float unscale = AM == SM_PKB ? SPLIT_UNSCALE : 1.f;
     if (__syncthreads_or(need)) {
         bool redo = need == SplitRange::REDO;
         if (!__syncthreads_or(redo)) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, 0, 1, w, wb, lane);
         if (__syncthreads_or(redo)) {
+            unscale = 1.f;
 #pragma unroll
             for (int i = 0; i < NBI; ++i)
 #pragma unroll
@@ -545,6 +550,12 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
         }
     }
 
+    if constexpr (AM == SM_PKB) {
+#pragma unroll
+        for (int i = 0; i < NBI; ++i)
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) acc[i][j] *= unscale;
+    }
     // epilogue: block (i, j) of a lane holds rows 4 g .. 4 g + 3, column r16
     float *C = p.C + bz * p.cbs;
     const float *bias = p.bias ? p.bias + bz * p.biasbs : nullptr;
@@ -576,7 +587,7 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
 {
     constexpr int TM = 16 * NBI, TN = 16 * NBJ, NBLK = NBI * NBJ;
     using LA = SplitLoader<AM, TM, 1>;
-    using LB = SplitLoader<BM, TN, 1>;
+    using LB = SplitLoader<BM, TN, 1, AM == SM_PKB>;
     constexpr int PA = LA::PL;
     __shared__ floatx4 red[NW][NBLK][64];
     __shared__ int need[NW];
@@ -711,10 +722,12 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
     int any = 0;
 #pragma unroll
     for (int k = 0; k < NW; ++k) any |= need[k];
+    float unscale = AM == SM_PKB ? SPLIT_UNSCALE : 1.f;
     if (any) {
         bool redo = any & SplitRange::REDO;
         if (!redo) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, w, NW, 0, 0, lane);
         if (__syncthreads_or(redo)) {  // (red is read after the barrier below)
+            unscale = 1.f;
 #pragma unroll
             for (int i = 0; i < NBI; ++i)
 #pragma unroll
@@ -737,6 +750,7 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
             floatx4 v = red[0][ii * NBJ + j][lane];
 #pragma unroll
             for (int k = 1; k < NW; ++k) v += red[k][ii * NBJ + j][lane];
+            if constexpr (AM == SM_PKB) v *= unscale;
             return v;
         };
         if (b != w) eo.load(p, bias, m, n);

@@ -13,7 +13,11 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // registers: given -1.0 as an inline constant the instruction takes it as an fp32 pattern.
 // Exact for every x with 2^-110 <= |x| that does not round to infinity in bf16 (checked over
 // random bit patterns of every exponent).
-__device__ __forceinline__ void split8(const float (&x)[8], u32x4 &h, u32x4 &m, u32x4 &l)
+// SCALED: the planes of 2^16 x.  fp32 numbers end at 2^-149 and bf16 ones at 2^-133, so these are
+// exact for subnormal x too, up to 2^111, for two more instructions per pair.
+constexpr float SPLIT_SCALE = 0x1p16f, SPLIT_UNSCALE = 0x1p-16f;
+template <bool SCALED = false>
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4 &h, u32x4 &m, u32x4 &l)
 {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     unsigned c0 = 0x0000bf80u, c1 = 0xbf800000u;  // bf16 (-1, 0) and (0, -1)
@@ -22,9 +26,10 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 &h, u32x4 &m, 
     const bf16x2 m0 = __builtin_bit_cast(bf16x2, c0), m1 = __builtin_bit_cast(bf16x2, c1);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const bf16x2 a = {(__bf16)x[2 * j], (__bf16)x[2 * j + 1]};
-        const float r0 = __builtin_amdgcn_fdot2_f32_bf16(a, m0, x[2 * j], false);
-        const float r1 = __builtin_amdgcn_fdot2_f32_bf16(a, m1, x[2 * j + 1], false);
+        const float x0 = SCALED ? v[2 * j] * SPLIT_SCALE : v[2 * j], x1 = SCALED ? v[2 * j + 1] * SPLIT_SCALE : v[2 * j + 1];
+        const bf16x2 a = {(__bf16)x0, (__bf16)x1};
+        const float r0 = __builtin_amdgcn_fdot2_f32_bf16(a, m0, x0, false);
+        const float r1 = __builtin_amdgcn_fdot2_f32_bf16(a, m1, x1, false);
         const bf16x2 b = {(__bf16)r0, (__bf16)r1};
         const float q0 = __builtin_amdgcn_fdot2_f32_bf16(b, m0, r0, false);
         const float q1 = __builtin_amdgcn_fdot2_f32_bf16(b, m1, r1, false);

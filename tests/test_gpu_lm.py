@@ -136,6 +136,26 @@ def test_full_batch_16(jas, kind, bf16):
     run_parity(jas, cfg, seed=21, B=16, P=9, steps=4, prompt_seed=21)
 
 
+@pytest.mark.parametrize("B,P", [(2, 40), (16, 64)])
+def test_bf16_weights_small_activations(jas, B, P):
+    """Bf16 weights times activations far below 2^-110 (a norm's gain and bias of 2^-124, the
+    following weights 2^124 times as large): the model's logits, which a power of two moved from
+    one factor to the other leaves as they are but for the activations' own subnormal rounding
+    (2^-25 of them)."""
+    cfg = jas.LmConfig(0, 1, 256, 4, 1040, 300, 64, B, 1e-5, 10000.0, 1, 0)
+    lm, small = jas.Lm(cfg), jas.Lm(cfg)
+    lm.init_random(5, 0.2)
+    for n in LM_WEIGHT_FIELDS:
+        w = lm.weight(n)
+        if w is not None:
+            f = {"ln2_g": 2.0 ** -124, "ln2_b": 2.0 ** -124, "w_fc": 2.0 ** 124}.get(n, 1.0)
+            small.set_weight(n, w * np.float32(f))
+    prompt = randint((B, P), cfg.vocab, 7)
+    _, want = lm.prefill(prompt, want_logits=True)
+    _, got = small.prefill(prompt, want_logits=True)
+    close(got, want, atol=2e-6 * np.abs(want).max(), rtol=0)
+
+
 def test_bf16_weight_roundtrip(jas):
     # set_weight rounds to bf16 (nearest even) and get_weight widens exactly; fp32 tensors
     # (norm gains, biases, positions) are untouched
