@@ -12,7 +12,8 @@
 // and the six products of the first three groups leave out at most 2^-26 |a b| -- a quarter
 // of the rounding of one fp32 multiplication.  All six accumulate in fp32, the small ones
 // first; six MFMAs take 96 cycles where the fp32 ones take 256.  Weights stored as bf16 are
-// their own h, and three products are exact.
+// their own h, and three products are exact (small ones first as well: prompt logits of a
+// four-layer GPT-2-width model 4.8e-7 from 64 bits, 5.0e-7 with the large one first).
 //
 // The split happens once per element and workgroup, between the global load and LDS: slabs
 // of 32 k are loaded to registers a slab ahead, split, and written to LDS as three planes
@@ -488,9 +489,9 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
                 mul(0, 1);
                 mul(0, 0);
             } else {
-                mul(0, 0);
-                mul(0, 1);
                 mul(0, 2);
+                mul(0, 1);
+                mul(0, 0);
             }
         }
     };
@@ -637,9 +638,9 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
                 mul(0, 1);
                 mul(0, 0);
             } else {
-                mul(0, 0);
-                mul(0, 1);
                 mul(0, 2);
+                mul(0, 1);
+                mul(0, 0);
             }
         }
     };
