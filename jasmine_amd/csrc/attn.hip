@@ -636,9 +636,10 @@ __device__ __attribute__((noinline)) void attend_row_fp32(const float *q, const 
 // S 1024, D 64, causal: 82.7 us, 156 TFLOP/s (128.8 us on the fp32 matrix cores, whose peak
 // is 157); not causal 134 us, 192 TFLOP/s (210).  D 128, 2 x 32 heads, causal: 108 us (159).
 //
-// Operands outside the split's range (gemm_split.hip) end in a non-finite row or sum, in an
-// output below 2^-108 of its row's weight, or show as magnitudes above 2^90 in Q or K (whose
-// partners could then be small enough to have lost parts that matter); a wave that sees one
+// Range: Q, K and V are split times 2^16, so that no part of one below 2^111 is lost, subnormal
+// ones included (split.hpp).  Probabilities below 2^-110 lose low bits, 2^-134 at most: against a
+// row sum of 2^-64 or more (the base) that is 2^-70 of the row's largest |V|.  Infinities, NaN
+// and larger operands, scores or outputs end in a non-finite row or sum; a wave that sees one
 // computes its queries again in fp32.
 template <int D, int NQ, int BK>
 __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p)
@@ -648,7 +649,6 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
     constexpr int KU = (UK + NW - 1) / NW, VU = (UV + NW - 1) / NW;
     __shared__ u32x4 Kp[3][NJ * CD * 64];
     __shared__ u32x4 Vp[3][NC * NM * 64];
-    __shared__ int s_large;
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int bh, qb, split;
@@ -663,11 +663,9 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
     const float *Kb = (const float *)p.K + (long)b * p.k_sb + (long)h * p.k_sh;
     const float *Vb = (const float *)p.V + (long)b * p.k_sb + (long)h * p.k_sh;
     auto slot_of = [](int row, int grp) { return (row + 16 * grp) ^ (row >> 3); };  // as in gemm_split.hip
-    if (tid == 0) s_large = 0;
 
     // Q planes (B operand): slots j < 4 hold d = 32 c + 4 g + j, j >= 4 d = 32 c + 16 + 4 g + j - 4
     bf16x8 qf[NQ][CD][3];
-    float qmax = 0.f;
 #pragma unroll
     for (int a = 0; a < NQ; ++a) {
         const int qq = min(q0 + 16 * a + r16, p.Sq - 1);
@@ -677,8 +675,7 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
             const floatx4 x0 = *(const floatx4 *)(qr + 32 * c + 4 * g), x1 = *(const floatx4 *)(qr + 32 * c + 16 + 4 * g);
             const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
             u32x4 hh, mm, ll;
-            track_max(qmax, x);
-            split8(x, hh, mm, ll);
+            split8<true>(x, hh, mm, ll);
             qf[a][c][0] = __builtin_bit_cast(bf16x8, hh);
             qf[a][c][1] = __builtin_bit_cast(bf16x8, mm);
             qf[a][c][2] = __builtin_bit_cast(bf16x8, ll);
@@ -714,15 +711,13 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
             }
         }
     };
-    float kmax = 0.f;
     auto lstore = [&]() {
 #pragma unroll
         for (int q = 0; q < KU; ++q) {
             const int u = w + NW * q;
             if (UK % NW != 0 && u >= UK) continue;
             u32x4 hh, mm, ll;
-            track_max(kmax, kr[q]);
-            split8(kr[q], hh, mm, ll);
+            split8<true>(kr[q], hh, mm, ll);
             const int at = u * 64 + slot_of(r16, g);
             Kp[0][at] = hh, Kp[1][at] = mm, Kp[2][at] = ll;
         }
@@ -736,7 +731,7 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
 #pragma unroll
                 for (int j = 0; j < 8; ++j) x[j] = vr[q][2 * j + e];
                 u32x4 hh, mm, ll;
-                split8(x, hh, mm, ll);
+                split8<true>(x, hh, mm, ll);
                 const int blk = 2 * (u % CD) + (r16 >> 3);  // 16-row block of d
                 const int at = (blk * NM + u / CD) * 64 + slot_of(2 * (r16 & 7) + e, g);
                 Vp[0][at] = hh, Vp[1][at] = mm, Vp[2][at] = ll;
@@ -752,7 +747,7 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
 #pragma unroll
         for (int c = 0; c < NC; ++c) oacc[c][a] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    const float sl2 = p.scale_log2;
+    const float sl2 = p.scale_log2 * (SPLIT_UNSCALE * SPLIT_UNSCALE);
     const int rslot = slot_of(r16, g);
     auto frag = [&](const u32x4 *const pl, int blk) { return __builtin_bit_cast(bf16x8, pl[blk * 64 + rslot]); };
 
@@ -835,10 +830,8 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
                 for (int a = 0; a < NQ; ++a) oacc[c][a] = mfma_split(vf, pf[m][a], oacc[c][a]);
             }
     }
-    if (kmax > 0x1p90f) s_large = 1;
-    __syncthreads();
 
-    bool bad = s_large || qmax > 0x1p90f;
+    bool bad = false;
     float l[NQ];
 #pragma unroll
     for (int a = 0; a < NQ; ++a) {
@@ -848,10 +841,7 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float o = fabsf(oacc[c][a][r]);
-                bad |= !(o <= FLT_MAX) || (o < l[a] * 0x1p-108f && o != 0.f);
-            }
+            for (int r = 0; r < 4; ++r) bad |= !(fabsf(oacc[c][a][r]) <= FLT_MAX);
     }
     if (__builtin_amdgcn_ballot_w64(bad)) {
         for (int q = q0; q < min(q0 + 16 * NQ, p.Sq); ++q) {
@@ -870,14 +860,14 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(const PrefillArgs p
         if (p.nsplit > 1) {  // unnormalised partial: O, then the base (exponent units) and row sum
             float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qi) * (D + 4);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) *(floatx4 *)(row + 16 * c + 4 * g) = oacc[c][a];
+            for (int c = 0; c < NC; ++c) *(floatx4 *)(row + 16 * c + 4 * g) = oacc[c][a] * SPLIT_UNSCALE;
             if (g == 0) {
                 row[D] = l[a] > 0.f ? mb[a] : -INFINITY;
                 row[D + 1] = l[a];
             }
             continue;
         }
-        const float inv = l[a] > 0.f ? 1.0f / l[a] : 0.f;
+        const float inv = l[a] > 0.f ? SPLIT_UNSCALE / l[a] : 0.f;
         float *o = (float *)p.O + (long)b * p.o_sb + (long)h * p.o_sh + (long)qi * p.o_ss;
 #pragma unroll
         for (int c = 0; c < NC; ++c) *(floatx4 *)(o + 16 * c + 4 * g) = oacc[c][a] * inv;

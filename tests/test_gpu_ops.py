@@ -774,6 +774,24 @@ def test_attn_prefill_split_range(jas, B, H, S, D):
     assert np.all(np.abs(got[fin] - want[fin]) <= bound), np.max(np.abs(got[fin] - want[fin]) / bound)
 
 
+@pytest.mark.parametrize("B,H,S,D", [(1, 2, 70, 64), (1, 1, 300, 32), (1, 1, 80, 128), (16, 17, 66, 64)])
+def test_attn_prefill_split_subnormal(jas, B, H, S, D):
+    """Values of V below the smallest bf16 (2^-133), below 2^-110 and ordinary ones in columns of
+    their own, and Q and K whose parts lie there."""
+    Q, K, V = (normal((B, H, S, D), 44, k) for k in range(3))
+    V[..., 0::4] *= np.float32(2.0 ** -140)
+    V[..., 1::4] *= np.float32(2.0 ** -120)
+    V[..., 2::4] *= np.float32(2.0 ** 90)
+    Q *= np.float32(2.0 ** -108)
+    K *= np.float32(2.0 ** 108)
+    got = _run_attention_f32(jas, Q, K, V, 1)
+    want = _attention64(Q, K, V, 1)
+    # as in test_attn_prefill_split, for each column; the output rounds at 2^-149
+    bound = 2 * 12 * D * 2.0 ** -24 * np.abs(V).max((0, 1, 2)) + 2.0 ** -149
+    assert np.all(np.abs(want[..., 0::4]).max((0, 1, 2)) > 8 * 2.0 ** -149)
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
+
+
 @pytest.mark.parametrize("D,dt,causal", [(64, 0, 1), (64, 3, 1), (128, 3, 0), (32, 3, 1), (128, 0, 0)])
 def test_attn_prefill_growing_scores(jas, D, dt, causal):
     """Keys whose scale grows along the sequence, so the running row max keeps rising by more
