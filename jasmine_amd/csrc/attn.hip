@@ -332,8 +332,8 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int r = 0; r < 4; ++r) row[16 * c + 4 * g + r] = oacc[c][r];
-        if (g == 0) {  // the base in exponent units (-inf: no visible key)
-            row[D] = lacc[0] > 0.f ? mb : -INFINITY;
+        if (g == 0) {  // the base in exponent units (-inf: no visible key; a NaN sum is one to merge)
+            row[D] = lacc[0] != 0.f ? mb : -INFINITY;
             row[D + 1] = lacc[0];
         }
         return;
@@ -561,8 +561,8 @@ __global__ void __launch_bounds__(256, 2) flash_bf16_kernel(const PrefillArgs p)
             float *row = p.part + (((long)split * p.B * p.H + bh) * p.Sq + qi) * (D + 4);
 #pragma unroll
             for (int c = 0; c < NC; ++c) *(floatx4 *)(row + 16 * c + 4 * g) = oacc[c][a];
-            if (g == 0) {  // (-inf: no visible key)
-                row[D] = l > 0.f ? mb[a] : -INFINITY;
+            if (g == 0) {  // (-inf: no visible key; a NaN sum is one to merge)
+                row[D] = l != 0.f ? mb[a] : -INFINITY;
                 row[D + 1] = l;
             }
             continue;
@@ -614,7 +614,8 @@ __device__ __attribute__((noinline)) void attend_row_fp32(const float *q, const 
         }
         m = mx;
     }
-    if (partial && lane == 0) row[D] = m, row[D + 1] = l;
+    // (NaN scores leave m as it was: -inf then has to be a base that the merge takes in)
+    if (partial && lane == 0) row[D] = m == -INFINITY && l != 0.f ? 0.f : m, row[D + 1] = l;
     const float inv = partial ? 1.f : l != 0.f ? 1.0f / l : 0.f;
 #pragma unroll
     for (int e = 0; e < E; ++e)

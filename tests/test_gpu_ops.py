@@ -792,6 +792,32 @@ def test_attn_prefill_split_subnormal(jas, B, H, S, D):
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("dt", [0, 3])
+def test_attn_prefill_key_split_nan(jas, D, dt):
+    """NaN in launches whose keys are split over work items: a NaN key reaches every query of its
+    head through the merge, a NaN query every element of its row, a NaN value its column."""
+    import ctypes as C
+    B, H, Sq, Sk = 1, 4, 40, 600
+    x = [normal(sh, 45, k) for k, sh in enumerate(((B, H, Sq, D), (B, H, Sk, D), (B, H, Sk, D)))]
+    x[1][0, 1, 450, 2] = np.nan
+    x[0][0, 2, 5, 1] = np.nan
+    x[2][0, 3, 333, 7] = np.nan
+    if dt:  # the upper halves: bf16 numbers (truncated), NaN stays NaN
+        x = [(v.view(np.uint32) >> 16).astype(np.uint16) for v in x]
+    dq, dk, dv = (jas.to_device(v) for v in x)
+    do = jas.DeviceArray((B, H, Sq, D), np.uint16 if dt else np.float32)
+    qs, ks = (H * Sq * D, Sq * D, D), (H * Sk * D, Sk * D, D)
+    jas.check(jas.lib.jas_attn_prefill(dq.p, dk.p, dv.p, do.p, B, H, Sq, Sk, D, *qs, *ks, *qs, C.c_float(1 / math.sqrt(D)),
+                                       0, dt, None))
+    got = (do.numpy().astype(np.uint32) << 16).view(np.float32) if dt else do.numpy()
+    want = np.zeros((B, H, Sq, D), bool)
+    want[0, 1] = True
+    want[0, 2, 5] = True
+    want[0, 3, :, 7] = True
+    assert np.array_equal(np.isnan(got), want)
+
+
 @pytest.mark.parametrize("D,dt,causal", [(64, 0, 1), (64, 3, 1), (128, 3, 0), (32, 3, 1), (128, 0, 0)])
 def test_attn_prefill_growing_scores(jas, D, dt, causal):
     """Keys whose scale grows along the sequence, so the running row max keeps rising by more
