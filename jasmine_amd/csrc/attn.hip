@@ -367,14 +367,13 @@ __global__ void __launch_bounds__(64 * NW, (NW == 8 && D <= 64) ? 4 : 1) flash_p
 // identically in both operands, so that S lands in the P operand's registers and every
 // accumulator entry of a lane belongs to the lane's own query.  Two buffers of LDS: tile t + 1
 // is written while tile t is read, one barrier per tile; loads run one tile ahead of that.
-template <int D, int NQ>
+template <int NQ>
 __global__ void __launch_bounds__(256, 2) flash_bf16_kernel(const PrefillArgs p)
 {
-    constexpr int NW = 4, BK = 64, BQ = 16 * NQ * NW, CD = D / 32, NC = D / 16, NJ = BK / 16, NM = BK / 32;
-    constexpr int DW = D == 128 ? 4 : 2;           // V: adjacent d per lane and key
-    constexpr int UK = NJ * CD, UV = D / (16 * DW) * NM;  // staging units: 16 keys x 32 d, 16 DW d x 32 keys
-    constexpr int KU = (UK + NW - 1) / NW, VU = (UV + NW - 1) / NW;
-    typedef uint32_t vchunk __attribute__((ext_vector_type(DW / 2 < 2 ? 1 : 2)));
+    constexpr int D = 128, NW = 4, BK = 64, BQ = 16 * NQ * NW, CD = D / 32, NC = D / 16, NJ = BK / 16, NM = BK / 32;
+    constexpr int UK = NJ * CD, UV = D / 64 * NM;  // staging units: 16 keys x 32 d, 64 d (4 a lane) x 32 keys
+    constexpr int KU = UK / NW, VU = UV / NW;
+    static_assert(UK % NW == 0 && UV % NW == 0, "units spread evenly over the waves");
     __shared__ u32x4 Ks[2][NJ * CD * 64];
     __shared__ u32x4 Vs[2][NC * NM * 64];
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
@@ -390,9 +389,9 @@ __global__ void __launch_bounds__(256, 2) flash_bf16_kernel(const PrefillArgs p)
     const int wave_kend = min(k_end, p.causal ? min(p.Sk, min(q0 + 16 * NQ - 1, p.Sq - 1) + shift + 1) : p.Sk);
     const uint16_t *Kb = (const uint16_t *)p.K + (long)b * p.k_sb + (long)h * p.k_sh;
     const uint16_t *Vb = (const uint16_t *)p.V + (long)b * p.k_sb + (long)h * p.k_sh;
-    // slot of row `row` of V's 16-row block blk: the lanes that store together (every DW-th row
+    // slot of row `row` of V's 16-row block blk: the lanes that store together (every fourth row
     // of two or more blocks) fall on different banks
-    auto vslot = [](int row, int blk) { return DW == 4 ? row ^ (row >> 2) ^ (blk & 1) : row ^ (row >> 3); };
+    auto vslot = [](int row, int blk) { return row ^ (row >> 2) ^ (blk & 1); };
 
     // Q (B operand): lane (query r16, g) holds d = 32 c + 8 g .. + 7
     bf16x8 qf[NQ][CD];
@@ -405,26 +404,24 @@ __global__ void __launch_bounds__(256, 2) flash_bf16_kernel(const PrefillArgs p)
     }
 
     u32x4 kr[KU];
-    vchunk vr[VU][8];
+    u32x2 vr[VU][8];
     auto gload = [&](int kv0) {
         const bool whole = kv0 + BK <= p.Sk;  // rows past Sk: the last row (finite, masked below)
 #pragma unroll
         for (int q = 0; q < KU; ++q) {
             const int u = w + NW * q;
-            if (UK % NW != 0 && u >= UK) continue;
             const int key = kv0 + 16 * (u / CD) + r16;
             kr[q] = *(const u32x4 *)(Kb + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss + 32 * (u % CD) + 8 * g);
         }
 #pragma unroll
         for (int q = 0; q < VU; ++q) {
             const int u = w + NW * q;
-            if (UV % NW != 0 && u >= UV) continue;
             const int key0 = kv0 + 32 * (u % NM) + 4 * g;
-            const uint16_t *src = Vb + 16 * DW * (u / NM) + DW * r16;
+            const uint16_t *src = Vb + 64 * (u / NM) + 4 * r16;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int key = key0 + j + (j < 4 ? 0 : 12);
-                vr[q][j] = *(const vchunk *)(src + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss);
+                vr[q][j] = *(const u32x2 *)(src + (long)(whole ? key : min(key, p.Sk - 1)) * p.k_ss);
             }
         }
     };
@@ -432,21 +429,19 @@ __global__ void __launch_bounds__(256, 2) flash_bf16_kernel(const PrefillArgs p)
 #pragma unroll
         for (int q = 0; q < KU; ++q) {
             const int u = w + NW * q;
-            if (UK % NW != 0 && u >= UK) continue;
             Ks[buf][u * 64 + lane] = kr[q];
         }
 #pragma unroll
         for (int q = 0; q < VU; ++q) {
             const int u = w + NW * q;
-            if (UV % NW != 0 && u >= UV) continue;
 #pragma unroll
-            for (int e = 0; e < DW; ++e) {
+            for (int e = 0; e < 4; ++e) {
                 // element e of the eight keys: the low or high halves of word e / 2
                 u32x4 t;
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                     t[k] = __builtin_amdgcn_perm(vr[q][2 * k + 1][e / 2], vr[q][2 * k][e / 2], e % 2 ? 0x07060302u : 0x05040100u);
-                const int d = 16 * DW * (u / NM) + DW * r16 + e, blk = d >> 4;
+                const int d = 64 * (u / NM) + 4 * r16 + e, blk = d >> 4;
                 Vs[buf][(blk * NM + u % NM) * 64 + 16 * g + vslot(d & 15, blk)] = t;
             }
         }
@@ -1336,8 +1331,8 @@ static jas_status decode_scratch_ptr(void **out, unsigned **ctr)
 using namespace jas;
 
 // fold argument of a causal launch (fa_work_item): the CU count when the kernel's workgroups
-// sit exactly two to a CU and the launch has at least two per CU, else 0.  Looked up once per
-// kernel and device.
+// sit exactly two to a CU and the launch has at least two per CU, else 0.  The occupancy is
+// looked up once per kernel: the library is built for one architecture.
 static int fa_fold(const void *kernel, int threads, int total)
 {
     static std::mutex mu;
@@ -1358,6 +1353,29 @@ static int fa_fold(const void *kernel, int threads, int total)
         }
     }
     return per == 2 && ncu % 8 == 0 && total >= 2 * ncu ? ncu : 0;
+}
+
+// The kernel of a prefill launch of `items` query blocks (narrow: 64 queries each, else 128)
+template <int D>
+static void launch_prefill(PrefillArgs p, int dtype, bool narrow, int items, hipStream_t s)
+{
+    auto launch = [&](auto *kernel, int threads) {
+        const int total = items * p.nsplit;
+        p.fold = p.causal && p.nsplit == 1 ? fa_fold((const void *)kernel, threads, total) : 0;
+        hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8), dim3(threads), 0, s, p);
+    };
+    if (dtype == JAS_F32) {
+        constexpr int BK = D == 128 ? 32 : 64;
+        if (D == 128 || narrow) launch(flash_split_kernel<D, 1, BK>, 256);
+        else if constexpr (D < 128) launch(flash_split_kernel<D, 2, BK>, 256);
+    } else if constexpr (D == 128) {
+        if (narrow) launch(flash_bf16_kernel<1>, 256);
+        else if (!p.causal || items >= 1024) launch(flash_bf16_kernel<2>, 256);
+        else launch(flash_prefill_kernel<D, 64, FA_WAVES>, 64 * FA_WAVES);
+    } else {
+        if (narrow) launch(flash_prefill_kernel<D, 64, 4>, 256);
+        else launch(flash_prefill_kernel<D, 64, FA_WAVES>, 64 * FA_WAVES);
+    }
 }
 
 extern "C" {
@@ -1401,28 +1419,9 @@ jas_status jas_attn_prefill(const void *Q, const void *K, const void *V, void *O
             JAS_CHECK(p.part, JAS_ERR_OOM, "jas_attn_prefill: workspace allocation failed");
         }
     }
-#define JAS_FA_LAUNCH(KERNEL, NT)                                                                       \
-    {                                                                                                  \
-        const int total = (int)items * p.nsplit;                                                       \
-        p.fold = causal && p.nsplit == 1 ? fa_fold((const void *)KERNEL, NT, total) : 0;               \
-        hipLaunchKernelGGL(KERNEL, dim3((total + 7) / 8 * 8), dim3(NT), 0, s, p);                      \
-    }
-#define JAS_FA(DD)                                                                                     \
-    if (D == DD) {                                                                                     \
-        constexpr int BKV = DD == 128 ? 32 : 64, NQV = DD == 128 ? 1 : 2;                              \
-        if (dtype == JAS_BF16) {                                                                       \
-            if (DD == 128 && narrow) JAS_FA_LAUNCH((flash_bf16_kernel<DD, 1>), 256)                    \
-            else if (DD == 128 && (!causal || items >= 1024)) JAS_FA_LAUNCH((flash_bf16_kernel<DD, 2>), 256) \
-            else if (narrow) JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, 4>), 256)                     \
-            else JAS_FA_LAUNCH((flash_prefill_kernel<DD, 64, FA_WAVES>), 64 * FA_WAVES)                \
-        } else {                                                                                       \
-            if (narrow) JAS_FA_LAUNCH((flash_split_kernel<DD, 1, BKV>), 256)                           \
-            else JAS_FA_LAUNCH((flash_split_kernel<DD, NQV, BKV>), 256)                                \
-        }                                                                                              \
-    }
-    JAS_FA(32) JAS_FA(64) JAS_FA(128)
-#undef JAS_FA
-#undef JAS_FA_LAUNCH
+    if (D == 32) launch_prefill<32>(p, dtype, narrow, (int)items, s);
+    else if (D == 64) launch_prefill<64>(p, dtype, narrow, (int)items, s);
+    else launch_prefill<128>(p, dtype, narrow, (int)items, s);
     if (p.nsplit > 1) {
         const dim3 grid(ceil_div((long)B * H * Sq * (D / 4), 256));
         if (dtype == JAS_BF16) hipLaunchKernelGGL(flash_merge_kernel<uint16_t>, grid, dim3(256), 0, s, p, D);
