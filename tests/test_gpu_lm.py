@@ -392,7 +392,7 @@ def test_weight_set_get_roundtrip(jas):
 # (sequences are
 # independent, so a subset pins the batch); its cost is the prompt length times the weights.
 
-def run_parity_subset(jas, cfg, seed, B, P, steps, prompt_seed, check, want_splits, exact=False):
+def run_parity_subset(jas, cfg, seed, B, P, steps, prompt_seed, check, want_splits, exact=False, decode_atol=ATOL):
     lm = jas.Lm(cfg)
     lm.init_random(seed, 0.02)
     got_splits = lm.attn_splits(B)
@@ -420,8 +420,21 @@ def run_parity_subset(jas, cfg, seed, B, P, steps, prompt_seed, check, want_spli
         nxt, lg = lm.decode(feed, want_logits=True)
         gpu_logits.append(lg[check])
         feed = nxt.copy()
-    close(np.stack(gpu_logits), cpu_logits)
+    close(gpu_logits[0], cpu_logits[0])
+    close(np.stack(gpu_logits), cpu_logits, atol=decode_atol)
     return lm
+
+
+@pytest.mark.parametrize("kv_bf16", [0, 1])
+def test_bf16_weights_long_prefill(jas, kv_bf16):
+    """Bf16 weights at d 4096 over 2032 prompt tokens: every projection on 256 x 128 tiles (gate
+    and up paired in a wave's row blocks, 22048 and 2032 ragged; an FFN of 11024, whose last packed
+    slab is half full; the QKV product of either cache).  The prompt's logits, and a decode step's,
+    whose keys and values are the cache that the prefill wrote (a bf16 one to the tolerance of
+    test_llama7b_width_bf16_weights_b16).  Oracle on the first and the last sequence."""
+    cfg = jas.LmConfig(1, 1, 4096, 32, 11024, 96, 130, 16, 1e-6, 10000.0, 1, kv_bf16)
+    run_parity_subset(jas, cfg, seed=35, B=16, P=127, steps=2, prompt_seed=35, check=(0, 15), want_splits=1,
+                      decode_atol=5e-3 if kv_bf16 else ATOL)
 
 
 @pytest.mark.parametrize("kv_bf16", [0, 1])

@@ -11,6 +11,7 @@ import pytest
 
 from jasmine_amd import expr as E
 from oracle_lib import orc, fp, normal
+from split_model import ATTENTION_BOUND, attention64, error, gemm_bound
 
 pytestmark = pytest.mark.gpu
 
@@ -435,7 +436,7 @@ def test_gemm_epilogues(jas, bias_mode, act, acc, batch):
 @pytest.mark.parametrize("ta,tb,col_c", [(0, 0, 0), (1, 0, 0), (0, 1, 0), (1, 1, 1), (0, 0, 1), (1, 0, 1)])
 @pytest.mark.parametrize("bias_mode,acc,batch", [(0, 0, 1), (1, 0, 2), (2, 0, 1), (0, 1, 3)])
 def test_gemm_library_sizes(jas, ta, tb, col_c, bias_mode, acc, batch):
-    """Library-size products on the direct-to-LDS kernel (gemm_dma_kernel): every operand
+    """Products of a few hundred rows and columns (32 x 16 to 64 x 32 tiles): every operand
     layout, both bias modes, accumulation, batches; K of 200 and 129 leave a partial slab."""
     _gemm_case(jas, 300, 260, 200, ta=bool(ta), tb=bool(tb), col_c=bool(col_c), bias_mode=bias_mode, acc=bool(acc),
                batch=batch)
@@ -446,24 +447,23 @@ def test_gemm_library_sizes(jas, ta, tb, col_c, bias_mode, acc, batch):
 @pytest.mark.parametrize("ta,tb,col_c", [(0, 0, 0), (1, 1, 0), (0, 1, 1), (1, 0, 1)])
 @pytest.mark.parametrize("M,N,K", [(4096, 4096, 40), (2048, 2100, 70), (1024, 1024, 1024)])
 def test_gemm_dma_geometries(jas, ta, tb, col_c, M, N, K):
-    """The three tile geometries of the direct-to-LDS kernel (256 x 256 with 8 waves when they
-    give every CU a workgroup, 128 x 128, 64 x 64) over every operand layout, with ragged M/N
-    edges and partial K slabs."""
+    """256 x 128 tiles (512 of them: two whole rounds), 64 x 64 and 64 x 32 tiles of
+    gemm_split.hip over operand layouts, with ragged edges, partial K slabs, bias and
+    accumulation."""
     _gemm_case(jas, M, N, K, ta=bool(ta), tb=bool(tb), col_c=bool(col_c), bias_mode=1, acc=True)
 
 
 @pytest.mark.parametrize("M,N,K,act,rcol,bstride,ccol", [
     (512, 512, 512, 0, 0, 0, 0), (300, 260, 200, 1, 0, 0, 0), (257, 129, 129, 1, 1, 0, 0), (96, 70, 64, 0, 0, 3, 0),
-    # 64 x 64 tiles (256 of them): float4 row-major store, and the column-major C store
+    # 64 x 32 tiles: row-major and column-major C
     (1024, 1024, 256, 1, 0, 0, 0), (1024, 1024, 256, 0, 1, 0, 1),
-    # 256 x 256 tiles (256 of them; the 128-wide geometry needs >= 1024 of its tiles with
-    # fewer than 256 of 256, which no single product meets): both C layouts
+    # 256 x 128 tiles (512 of them): both C layouts
     (4096, 4096, 128, 0, 0, 0, 0), (4096, 4096, 128, 1, 1, 0, 1), (300, 516, 96, 1, 0, 0, 1)])
 def test_gemm_residual(jas, M, N, K, act, rcol, bstride, ccol):
     """jas_gemm_residual: act(A B + bias) + R, against jas_gemm of the same operands followed by
     the residual added in fp32 (bit for bit: the same product, then the same two roundings).
     R row- or column-major, C row- or column-major; B with a padded row stride (3 extra
-    floats) is not 16-byte addressable per row, which takes the product-then-add path."""
+    floats), whose rows are not 16-byte aligned."""
     rng = np.random.default_rng(61)
     A = rng.standard_normal((M, K), dtype=np.float32)
     ldb = N + bstride
@@ -518,6 +518,8 @@ def test_gemm_split_geometries(jas, M, N, K, batch, la, lb, lc):
     # of magnitudes), and 2^-26 of each product left out by the split
     bound = (K + 2) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
     assert np.all(np.abs(got - want) <= bound + 1e-30), float(np.max(np.abs(got - want) / (bound + 1e-30)))
+    # and the root mean square, which a lost product of two planes exceeds (test_split_model.py)
+    assert error(got, want, np.sqrt(K)) <= gemm_bound(K), (error(got, want, np.sqrt(K)), gemm_bound(K))
 
 
 @pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (1024, 4096, 1056), (2048, 1536, 96), (96, 64, 640), (200, 90, 120)])
@@ -584,8 +586,8 @@ def test_gemm_split_subnormal(jas, M, N, K):
 
 
 def test_gemm_dma_k_tail_padded_rows(jas):
-    """K not a multiple of 4 with 16-byte aligned, padded rows (K-contiguous operands take the
-    direct-to-LDS path): the tail slab reads element by element and zero-fills past K."""
+    """K not a multiple of 4 with padded, K-contiguous rows: the tail slab reads element by
+    element and zero-fills past K."""
     M, N, K, Kp = 300, 260, 147, 152
     A = np.zeros((M, Kp), np.float32)
     Bt = np.zeros((N, Kp), np.float32)
@@ -748,6 +750,10 @@ def test_attn_prefill_split(jas, B, H, Sq, Sk, D, causal):
     # of it, a probability that relative error twice (its own and its row sum's)
     bound = 2 * 12 * D * 2.0 ** -24 * np.abs(V).max()
     assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
+    # and the root mean square over all heads, which a lost product exceeds (test_split_model.py)
+    rms = np.sqrt(np.mean([error(got[b, h], *attention64(Q[b, h], K[b, h], V[b, h], causal)) ** 2
+                           for b, h in np.ndindex(B, H)]))
+    assert rms <= ATTENTION_BOUND, rms
 
 
 @pytest.mark.parametrize("B,H,S,D", [(1, 2, 70, 64), (1, 1, 300, 32), (1, 1, 80, 128), (16, 17, 66, 64)])
