@@ -429,11 +429,19 @@ __device__ __forceinline__ void split_epilogue(const SplitArgs &p, float *C, con
 // workgroup splits each element once; per slab and CU a 256 x 128 tile needs 3072 cycles of
 // matrix core, about 900 of vector ALU, 2100 of LDS.  MI355X, 4096^3: 1083 us on the fp32
 // matrix cores (127 TFLOP/s), 690 us here (199 TFLOP/s of fp32 products, 1.2 PFLOP/s of bf16
-// ones, the rate a plain bf16 product of this size reaches).
-template <int AM, int BM, int TM, int TN, int NW, int WGM>
+// ones, the rate a plain bf16 product of this size reaches).  A slab takes about 6400 cycles: the
+// waves leave its barrier together, and their phases add up rather than overlap (matrix cores busy
+// 0.49).
+//
+// SUMS (where tiles compete with waves that split K): a slab's six products add up by themselves,
+// then to the sum, so a slab rounds the long sum once and not six times: the error is that of four
+// waves' sums or less.  SUMS_FEW: and the last slab is not loaded again (see below).
+enum SlabSums : int { PLAIN = 0, SUMS = 1, SUMS_FEW = 2 };
+template <int AM, int BM, int TM, int TN, int NW, int WGM, int FORM = PLAIN>
 __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs p)
 {
     constexpr int WGN = NW / WGM, NBI = TM / WGM / 16, NBJ = TN / WGN / 16;
+    constexpr bool TWO = FORM != PLAIN;
     using LA = SplitLoader<AM, TM, NW>;
     using LB = SplitLoader<BM, TN, NW, AM == SM_PKB>;
     constexpr int PA = LA::PL, SA = PA * TM * 4, SB = 3 * TN * 4;  // 16-byte units per stage
@@ -475,11 +483,16 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
             bf16x8 a[PA];
 #pragma unroll
             for (int pl = 0; pl < PA; ++pl) a[pl] = __builtin_bit_cast(bf16x8, pa[(pl * LA::NB + i) * 64]);
+            floatx4 slab[NBJ];  // TWO
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) slab[j] = floatx4{0.f, 0.f, 0.f, 0.f};
             // small products first; the NBJ accumulators innermost
             auto mul = [&](int ia, int ib) {
 #pragma unroll
-                for (int j = 0; j < NBJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[j][ib], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NBJ; ++j) {
+                    floatx4 &d = TWO ? slab[j] : acc[i][j];
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[j][ib], d, 0, 0, 0);
+                }
             };
             if constexpr (PA == 3) {
                 mul(2, 0);
@@ -492,6 +505,10 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
                 mul(0, 2);
                 mul(0, 1);
                 mul(0, 0);
+            }
+            if constexpr (TWO) {
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j) acc[i][j] += slab[j];
             }
         }
     };
@@ -506,12 +523,13 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
     // Slab s goes to stage s % 2, which was last read two slabs ago, before the barrier of the
     // slab in between: one barrier per slab.  The loads of the next slab are issued whether or
     // not it exists (past the last one: the last again), so the wait counts do not depend on
-    // the path.
+    // the path.  Where there are few slabs, one load more is dearer than the waits (3072 x 509 x 64
+    // 8.4 us with it, 7.7 without; 1024^2 x 768 20.8 and 22.7).
     auto step = [&](int s, bool more) {
         u32x4 *sa = lds + (s & 1) * (SA + SB);
         la.store(ra, sa, w, lane, mx);
         lb.store(rb, sa + SA, wb, lane, mx);
-        if (more) fetch(min(s + 1, nk - 1) * 32);
+        if (more && (FORM != SUMS_FEW || s + 1 < nk)) fetch(min(s + 1, nk - 1) * 32);
         __syncthreads();
         compute(sa);
     };
@@ -587,6 +605,7 @@ template <int AM, int BM, int NBI, int NBJ, int NW, int PD>
 __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArgs p)
 {
     constexpr int TM = 16 * NBI, TN = 16 * NBJ, NBLK = NBI * NBJ;
+    constexpr bool TWO = NW == 2;  // (as above: two waves' sums would be longer than four's)
     using LA = SplitLoader<AM, TM, 1>;
     using LB = SplitLoader<BM, TN, 1, AM == SM_PKB>;
     constexpr int PA = LA::PL;
@@ -625,10 +644,15 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
         for (int i = 0; i < NBI; ++i) {
             bf16x8 a[PA];
             LA::planes(ra, i, mx, a);
+            floatx4 slab[NBJ];  // TWO
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) slab[j] = floatx4{0.f, 0.f, 0.f, 0.f};
             auto mul = [&](int ia, int ib) {
 #pragma unroll
-                for (int j = 0; j < NBJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[j][ib], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NBJ; ++j) {
+                    floatx4 &d = TWO ? slab[j] : acc[i][j];
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[j][ib], d, 0, 0, 0);
+                }
             };
             if constexpr (PA == 3) {
                 mul(2, 0);
@@ -641,6 +665,10 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
                 mul(0, 2);
                 mul(0, 1);
                 mul(0, 0);
+            }
+            if constexpr (TWO) {
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j) acc[i][j] += slab[j];
             }
         }
     };
@@ -760,10 +788,10 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
     }
 }
 
-template <int AM, int BM, int TM, int TN, int NW, int WGM>
+template <int AM, int BM, int TM, int TN, int NW, int WGM, int FORM = PLAIN>
 static void launch_tile(const SplitArgs &p, int batch, hipStream_t s)
 {
-    hipLaunchKernelGGL((gemm_split_kernel<AM, BM, TM, TN, NW, WGM>), dim3(ceil_div(p.N, TN), ceil_div(p.M, TM), batch),
+    hipLaunchKernelGGL((gemm_split_kernel<AM, BM, TM, TN, NW, WGM, FORM>), dim3(ceil_div(p.N, TN), ceil_div(p.M, TM), batch),
                        dim3(NW * 64), 0, s, p);
 }
 template <int AM, int BM, int NBI, int NBJ, int NW, int PD>
@@ -773,6 +801,97 @@ static void launch_wave_split(const SplitArgs &p, int batch, hipStream_t s)
     constexpr int AD = AM == SM_OC ? (int)SM_GEN : AM, BD = BM == SM_OC ? (int)SM_GEN : BM;
     hipLaunchKernelGGL((gemm_split_k_kernel<AD, BD, NBI, NBJ, NW, PD>),
                        dim3(ceil_div(p.N, 16 * NBJ), ceil_div(p.M, 16 * NBI), batch), dim3(NW * 64), 0, s, p);
+}
+
+// Unpacked operands, each K-contiguous (KC below), outer-contiguous (OC) or of general strides:
+// the products that launch_split's geometries, chosen for weights and a long K, serve badly; false:
+// none of them.  Waves that split K read KC rows 16 apart in memory and OC rows element by element,
+// and four of them have little to do for a K of a few slabs: tiles in LDS are ahead from the size at
+// which they fill the chip.  t64, t32: tiles of 64 x 64 (three workgroups per CU: 768 at a time) and
+// 32 x 32.  MI355X, us per product (M x N x K, operands A x B; launch_split's form -> here; the
+// former fp32-MFMA kernels):
+//   128 x 64, eight waves, past one round of 64 x 64: 2048^2 x 64 OC x KC 18.8 -> 11.7 (14.7),
+//     2048^2 x 128 KC x KC 26.1 -> 15.2 (19.4).  Four waves where both are OC (pieces of 32 rows: half
+//     of eight waves would stage nothing): 2048^2 x 64 19.3 -> 14.9 (13.9; eight waves 17.6); from
+//     K = 96 on four waves that split K are ahead.  Four waves too from K = 256 on for KC x KC:
+//     2048^2 x 512 47.2 -> 36.4 (46.1)
+//   64 x 64, four waves, from 448 of them on: 1500^2 x 128 OC x OC 18.5 -> 13.7 (15.7), 1500^2 x 200
+//     OC x KC 23.3 -> 19.9 (22.6); past K = 320 with OC in A, splitting K is ahead again.  KC x KC at
+//     every K and from 224 of them on: 1500^2 x 1024 71.7 -> 50.4 (63.8), 1024^2 x 768 26.5 -> 20.8
+//     (20.3).  Eight waves hide more where there is little K: KC x KC 768 x 4096 x 64 17.8 -> 11.8
+//     (12.9; in plain sums 10.2, by four waves 10.6), OC x KC 753 x 2592 x 110 13.5 -> 11.8 (11.9;
+//     by four 12.2)
+//   64 x 32, four waves, OC x OC under 448: 3072 x 509 x 64 12.8 -> 7.7 (9.6)
+//   32 x 32 by two waves, a few slabs: 1024^2 x 64 OC x KC 7.5 -> 6.2 (6.6), OC x OC 9.1 -> 6.5 (6.3);
+//     four waves: 1024 x 512 x 192 KC x OC 8.4 -> 6.8 (6.2), 1024^2 x 256 KC x OC 13.4 -> 10.9 (10.2)
+//   64 x 32, four waves, one slab ahead: 1024 x 512 x 384 KC x KC 11.3 -> 10.1 (8.5)
+//   general strides, each operand in its own mode: 1000^3 with every second element of B's K
+//     105.7 -> 41.1 (33.8), 2048^2 x 512 with both such 80.1 -> 60.0 (81.0); still behind by up to a
+//     third: 1000^2 x 64 one such 13.1 -> 9.0 (6.4), 2000 x 1500 x 100 28.3 -> 23.2 (14.6)
+// Errors against 64 bits over 11 sizes, 10 K from 32 to 2048 and four layouts: nowhere above those
+// of launch_split's forms, and below the fp32 kernels'.
+template <int AM, int BM>
+static bool launch_unpacked(const SplitArgs &p, long t64, long t32, int batch, hipStream_t s)
+{
+    const int K = p.K;
+    constexpr bool kk = AM == SM_KC && BM == SM_KC, oo = AM == SM_OC && BM == SM_OC, ko = AM == SM_KC && BM == SM_OC;
+    constexpr bool ok = AM == SM_OC && BM == SM_KC;
+    if constexpr (AM > SM_GEN || BM > SM_GEN) {
+        return false;
+    } else if constexpr (AM == SM_GEN || BM == SM_GEN) {
+        if constexpr (AM == SM_OC || BM == SM_OC)
+            if (t64 > 192 && t64 <= 512 && K >= 512) {
+                launch_wave_split<AM, BM, 4, 2, 4, 0>(p, batch, s);
+                return true;
+            }
+        if (t64 > 512) launch_tile<AM, BM, 128, 64, 4, 2, SUMS>(p, batch, s);
+        else if (t64 > 192) launch_tile<AM, BM, 64, 64, 4, 2, SUMS>(p, batch, s);
+        else if (K <= 128 || t32 > 256) launch_wave_split<AM, BM, 2, 2, 4, 0>(p, batch, s);
+        else if (t32 > 128) launch_wave_split<AM, BM, 2, 2, 8, 0>(p, batch, s);
+        else launch_wave_split<AM, BM, 2, 1, 8, 0>(p, batch, s);
+        return true;
+    } else if (t64 > 768) {
+        if constexpr (oo) {
+            if (K >= 96) return false;
+            launch_tile<AM, BM, 128, 64, 4, 2, SUMS_FEW>(p, batch, s);
+            return true;
+        }
+        if (K >= (kk ? 1024 : 256)) return false;
+        if constexpr (!oo)
+            if (K < 256) launch_tile<AM, BM, 128, 64, 8, 4, SUMS_FEW>(p, batch, s);
+        if constexpr (kk)
+            if (K >= 256) launch_tile<AM, BM, 128, 64, 4, 2, SUMS>(p, batch, s);
+        return true;
+    } else if (t64 >= 448 || (kk && t64 >= 224)) {
+        if (!kk && K > (ko ? 1000 : 320)) return false;
+        if constexpr (kk || ok)
+            if (kk ? K < (t64 >= 448 ? 96 : 129) : t64 <= 512 && K <= 128) {
+                launch_tile<AM, BM, 64, 64, 8, 4, SUMS_FEW>(p, batch, s);
+                return true;
+            }
+        launch_tile<AM, BM, 64, 64, 4, 2, kk || ko ? SUMS : SUMS_FEW>(p, batch, s);
+        return true;
+    } else {
+        if constexpr (oo)
+            if (t64 > 300) {
+                if (K > 160) return false;
+                launch_tile<AM, BM, 64, 32, 4, 2, SUMS_FEW>(p, batch, s);
+                return true;
+            }
+        if constexpr (!kk)
+            if (K <= (oo ? 256 : 160) && (t64 >= 224 || (oo && t32 > 512))) {
+                launch_wave_split<AM, BM, 2, 2, 2, 0>(p, batch, s);
+                return true;
+            }
+        if (K <= 128 || t32 < 400 || (ko ? K >= 1024 : t64 >= 224 || (K > 256 && !kk))) return false;
+        if constexpr (kk)
+            if (K > 256) {
+                launch_wave_split<AM, BM, 4, 2, 4, 0>(p, batch, s);
+                return true;
+            }
+        launch_wave_split<AM, BM, 2, 2, 4, 0>(p, batch, s);
+        return true;
+    }
 }
 
 // Geometry by the number of tiles (256 CUs) and K; MI355X, us per product (M x N x K):
@@ -794,16 +913,22 @@ template <int AM, int BM>
 static void launch_split(const SplitArgs &p, int batch, hipStream_t s)
 {
     auto tiles = [&](int a, int b) { return (long)ceil_div(p.M, a) * ceil_div(p.N, b) * batch; };
-    const long big = tiles(256, 128);
-    if (big >= 256 && big * 5 >= (big + 255) / 256 * 256 * 4) launch_tile<AM, BM, 256, 128, 8, 4>(p, batch, s);
-    else if (tiles(128, 64) >= 512 && p.K >= 1024) launch_tile<AM, BM, 128, 64, 4, 2>(p, batch, s);
-    else if (tiles(64, 64) >= 768) launch_wave_split<AM, BM, 4, 4, 4, 1>(p, batch, s);
-    else if (p.K <= 128) launch_wave_split<AM, BM, 2, 2, 4, 0>(p, batch, s);
-    else if (tiles(64, 32) >= 256) launch_wave_split<AM, BM, 4, 2, 4, 2>(p, batch, s);
-    else if (tiles(32, 32) > 256) launch_wave_split<AM, BM, 4, 2, 8, 0>(p, batch, s);
-    else if (tiles(32, 32) > 128) launch_wave_split<AM, BM, 2, 2, 8, 0>(p, batch, s);
-    else launch_wave_split<AM, BM, 2, 1, 8, 0>(p, batch, s);
+    if (launch_unpacked<AM, BM>(p, tiles(64, 64), tiles(32, 32), batch, s)) return;
+    if constexpr (AM != SM_GEN && BM != SM_GEN) {
+        const long big = tiles(256, 128);
+        if (big >= 256 && big * 5 >= (big + 255) / 256 * 256 * 4) launch_tile<AM, BM, 256, 128, 8, 4>(p, batch, s);
+        else if (tiles(128, 64) >= 512 && p.K >= 1024) launch_tile<AM, BM, 128, 64, 4, 2>(p, batch, s);
+        else if (tiles(64, 64) >= 768) launch_wave_split<AM, BM, 4, 4, 4, 1>(p, batch, s);
+        else if (p.K <= 128) launch_wave_split<AM, BM, 2, 2, 4, 0>(p, batch, s);
+        else if (tiles(64, 32) >= 256) launch_wave_split<AM, BM, 4, 2, 4, 2>(p, batch, s);
+        else if (tiles(32, 32) > 256) launch_wave_split<AM, BM, 4, 2, 8, 0>(p, batch, s);
+        else if (tiles(32, 32) > 128) launch_wave_split<AM, BM, 2, 2, 8, 0>(p, batch, s);
+        else launch_wave_split<AM, BM, 2, 1, 8, 0>(p, batch, s);
+    }
 }
+
+template <int MODE>
+using mode_c = std::integral_constant<int, MODE>;
 
 // staging mode of operand X(o, k) = X[o * so + k * sk]
 static int split_mode(long so, long sk) { return sk == 1 ? SM_KC : so == 1 ? SM_OC : SM_GEN; }
@@ -829,14 +954,16 @@ jas_status gemm_split(SplitArgs p, bool a_packed, bool a_bf16, int batch, hipStr
         JAS_CHECK(bm == SM_KC, JAS_ERR_INVALID, "gemm: packed weights take K-contiguous activations");
         if (a_bf16) launch_split<SM_PKB, SM_KC>(p, batch, s);
         else launch_split<SM_PK, SM_KC>(p, batch, s);
-    } else if (am == SM_GEN || bm == SM_GEN) {
-        launch_split<SM_GEN, SM_GEN>(p, batch, s);
-    } else if (am == SM_KC) {
-        if (bm == SM_KC) launch_split<SM_KC, SM_KC>(p, batch, s);
-        else launch_split<SM_KC, SM_OC>(p, batch, s);
     } else {
-        if (bm == SM_KC) launch_split<SM_OC, SM_KC>(p, batch, s);
-        else launch_split<SM_OC, SM_OC>(p, batch, s);
+        auto go = [&](auto a, auto b) { launch_split<decltype(a)::value, decltype(b)::value>(p, batch, s); };
+        auto with_b = [&](auto a) {
+            if (bm == SM_KC) go(a, mode_c<SM_KC>());
+            else if (bm == SM_OC) go(a, mode_c<SM_OC>());
+            else go(a, mode_c<SM_GEN>());
+        };
+        if (am == SM_KC) with_b(mode_c<SM_KC>());
+        else if (am == SM_OC) with_b(mode_c<SM_OC>());
+        else with_b(mode_c<SM_GEN>());
     }
     JAS_LAUNCH_CHECK();
     return JAS_OK;

@@ -436,7 +436,7 @@ def test_gemm_epilogues(jas, bias_mode, act, acc, batch):
 @pytest.mark.parametrize("ta,tb,col_c", [(0, 0, 0), (1, 0, 0), (0, 1, 0), (1, 1, 1), (0, 0, 1), (1, 0, 1)])
 @pytest.mark.parametrize("bias_mode,acc,batch", [(0, 0, 1), (1, 0, 2), (2, 0, 1), (0, 1, 3)])
 def test_gemm_library_sizes(jas, ta, tb, col_c, bias_mode, acc, batch):
-    """Products of a few hundred rows and columns (32 x 16 to 64 x 32 tiles): every operand
+    """Products of a few hundred rows and columns, single and batched: every operand
     layout, both bias modes, accumulation, batches; K of 200 and 129 leave a partial slab."""
     _gemm_case(jas, 300, 260, 200, ta=bool(ta), tb=bool(tb), col_c=bool(col_c), bias_mode=bias_mode, acc=bool(acc),
                batch=batch)
@@ -447,17 +447,16 @@ def test_gemm_library_sizes(jas, ta, tb, col_c, bias_mode, acc, batch):
 @pytest.mark.parametrize("ta,tb,col_c", [(0, 0, 0), (1, 1, 0), (0, 1, 1), (1, 0, 1)])
 @pytest.mark.parametrize("M,N,K", [(4096, 4096, 40), (2048, 2100, 70), (1024, 1024, 1024)])
 def test_gemm_dma_geometries(jas, ta, tb, col_c, M, N, K):
-    """256 x 128 tiles (512 of them: two whole rounds), 64 x 64 and 64 x 32 tiles of
-    gemm_split.hip over operand layouts, with ragged edges, partial K slabs, bias and
-    accumulation."""
+    """Large and middle-sized products over operand layouts, with ragged edges, partial K slabs,
+    bias and accumulation."""
     _gemm_case(jas, M, N, K, ta=bool(ta), tb=bool(tb), col_c=bool(col_c), bias_mode=1, acc=True)
 
 
 @pytest.mark.parametrize("M,N,K,act,rcol,bstride,ccol", [
     (512, 512, 512, 0, 0, 0, 0), (300, 260, 200, 1, 0, 0, 0), (257, 129, 129, 1, 1, 0, 0), (96, 70, 64, 0, 0, 3, 0),
-    # 64 x 32 tiles: row-major and column-major C
+    # 32 x 32 tiles by two waves: row-major and column-major C
     (1024, 1024, 256, 1, 0, 0, 0), (1024, 1024, 256, 0, 1, 0, 1),
-    # 256 x 128 tiles (512 of them): both C layouts
+    # 128 x 64 tiles: both C layouts
     (4096, 4096, 128, 0, 0, 0, 0), (4096, 4096, 128, 1, 1, 0, 1), (300, 516, 96, 1, 0, 0, 1)])
 def test_gemm_residual(jas, M, N, K, act, rcol, bstride, ccol):
     """jas_gemm_residual: act(A B + bias) + R, against jas_gemm of the same operands followed by
@@ -484,13 +483,16 @@ def test_gemm_residual(jas, M, N, K, act, rcol, bstride, ccol):
     assert np.array_equal(g_, w + R)
 
 
-# every geometry of launch_split (gemm_split.hip) at its edges: partial tiles in both
+# every geometry of launch_split and launch_unpacked (gemm_split.hip) at its edges: partial tiles in both
 # dimensions, K tails, K of less than a slab, rows that are not 16-byte aligned (odd leading
 # dimensions), general strides (a step of 2 in both dimensions), both orders of C, batches
 @pytest.mark.parametrize("M,N,K,batch", [
     (4100, 2050, 70, 1),    # 256 x 128, whole rounds
     (4097, 1023, 1057, 1),  # 128 x 64, long K
-    (1537, 2049, 90, 1),    # 64 x 64
+    (1537, 2049, 90, 1), (2100, 2050, 70, 1), (2100, 2050, 260, 1),  # 128 x 64, few slabs (64 x 64 split four ways)
+    (1300, 1500, 90, 1), (350, 400, 140, 14),  # 64 x 64 in LDS, eight and four waves
+    (1000, 1000, 100, 1), (1000, 1400, 170, 1), (1100, 1200, 100, 1),  # 64 x 64, 64 x 32 and, by two and four waves, 32 x 32
+    (700, 900, 200, 1), (700, 900, 300, 1),  # 32 x 32 by four or two waves, 64 x 32
     (65, 33, 65, 40), (65, 33, 128, 1),  # K <= 128: 32 x 32, four waves
     (1023, 515, 333, 1),    # 64 x 32, four waves
     (600, 501, 257, 1),     # 64 x 32, eight waves
@@ -522,7 +524,8 @@ def test_gemm_split_geometries(jas, M, N, K, batch, la, lb, lc):
     assert error(got, want, np.sqrt(K)) <= gemm_bound(K), (error(got, want, np.sqrt(K)), gemm_bound(K))
 
 
-@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (1024, 4096, 1056), (2048, 1536, 96), (96, 64, 640), (200, 90, 120)])
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (1024, 4096, 1056), (2048, 1536, 96), (1000, 1000, 100),
+                                   (96, 64, 640), (200, 90, 120)])
 def test_gemm_split_range(jas, M, N, K):
     """Values outside the bf16 split's range: infinities, NaN, magnitudes that round to infinity
     in bf16, products that overflow, and operands so small that their parts underflow -- each
@@ -556,7 +559,8 @@ def test_gemm_split_range(jas, M, N, K):
     assert np.isinf(got[20, 30]) and got[20, 30] > 0
 
 
-@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (2050, 2100, 1056), (1030, 1900, 96), (96, 64, 640), (200, 90, 120)])
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (2050, 2100, 1056), (1030, 1900, 96), (1000, 1000, 100),
+                                   (96, 64, 640), (200, 90, 120)])
 def test_gemm_split_subnormal(jas, M, N, K):
     """Operands below 2^-110, subnormal ones and ones below the smallest bf16 among them, against
     partners large enough that their products are ordinary numbers, and next to ordinary
