@@ -28,11 +28,12 @@
 // in bf16 make the six-product sum non-finite.  Magnitudes below 2^-110 lose the bits of m and
 // l under bf16's smallest step, below 2^-134 all of h too: at most 2^-134 per element, so an
 // error of at most K 2^-134 (max|A| + max|B|) in a sum -- more than 2^-24 of it only if the sum
-// is below K 2^-110 (max|A| + max|B|), which a sum of zero always is.  A tile with such a sum is
-// looked over for operands below 2^-110 that are not zero; if it has one, or a sum that is not
-// finite, it is computed again on the fp32 matrix cores (SplitRange).  MI355X, 1024^3, 24 us: 31
-// where every tile is looked over (a row of zeros in each), 55 where every one is computed again;
-// 4096 x 4096 x 1024, 212 us: 255 and 670.  Beside packed bf16 weights, which need no split, the
+// is below K 2^-110 (max|A| + max|B|), which a sum of zero always is.  The rows and columns of a few
+// such sums, or a tile with many, are looked over for operands below 2^-110 that are not zero; a tile
+// that has one, or a sum that is not finite, is computed again on the fp32 matrix cores (SplitRange).
+// MI355X: 1024^3, 22 us, 32 where every tile is looked over (zeros in each), 55 where every one is
+// computed again; 4096 x 4096 x 1024, 205 us: 211 with a row of zeros in each tile, 670 computed again;
+// 4096^3, 667 us: 700 with one sum that cancels to zero.  Beside packed bf16 weights, which need no split, the
 // activations are split times 2^16, which loses nothing, and only sums that are not finite count.
 #include "gemm.hpp"
 #include "split.hpp"
@@ -58,12 +59,21 @@ struct SplitRange {
         }
     }
     enum : int { OK = 0, LOOK = 1, REDO = 2 };
-    // limit: the largest number, or less where further sums follow; largest: operand magnitude
+    // sums below this, of operands up to `largest`, may have lost too much
+    __device__ __forceinline__ static float bound(float largest, int K) { return 2.f * (float)K * 0x1p-110f * largest; }
+    // limit: the largest number, or less where further sums follow
     __device__ __forceinline__ int check(float limit, float largest, int K) const
     {
-        return !(hi <= limit) ? REDO : lo < 2.f * (float)K * 0x1p-110f * largest ? LOOK : OK;
+        return !(hi <= limit) ? REDO : lo < bound(largest, K) ? LOOK : OK;
     }
 };
+
+// the largest of lanes r16, r16 + 16, r16 + 32 and r16 + 48
+__device__ __forceinline__ float max_over_g(float v)
+{
+    v = fmaxf(v, __shfl_xor(v, 16, WAVE));
+    return fmaxf(v, __shfl_xor(v, 32, WAVE));
+}
 
 // One operand X(o, k) of a workgroup: its T x 32 slabs from memory to registers to LDS.  SCALED: its
 // planes are those of 2^16 X, exact for every magnitude up to 2^111 (beside bf16 weights, whose
@@ -75,6 +85,8 @@ struct SplitLoader {
     static constexpr int NR = MODE == SM_OC ? 16 : MODE == SM_PKB ? 4 : 8;
     static constexpr int PL = MODE == SM_PKB ? 1 : 3, NB = T / 16;  // planes, 16-row blocks
     typedef float regs_t[UPW][NR];
+    static constexpr int R = MODE == SM_OC ? 2 : 1;  // rows per lane and unit
+    typedef float max_t[UPW * R];                    // largest magnitude in each of them
 
     const float *X;
     long so, sk;
@@ -216,7 +228,7 @@ struct SplitLoader {
     // of outer-contiguous units (two rows per lane, every other slot) off each other's banks.
     __device__ __forceinline__ static int slot_of(int r16, int g) { return (r16 + 16 * g) ^ (r16 >> 3); }
 
-    __device__ __forceinline__ void store(const regs_t &r, u32x4 *lds, int w, int lane, float &mx) const
+    __device__ __forceinline__ void store(const regs_t &r, u32x4 *lds, int w, int lane, max_t &mx) const
     {
         const int i = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -226,14 +238,13 @@ struct SplitLoader {
             if constexpr (MODE == SM_PKB) {
                 lds[u * 64 + slot_of(i, g)] = __builtin_bit_cast(u32x4, floatx4{r[q][0], r[q][1], r[q][2], r[q][3]});
             } else {
-                constexpr int R = MODE == SM_OC ? 2 : 1;  // rows per lane
 #pragma unroll
                 for (int e = 0; e < R; ++e) {
                     float x[8];
 #pragma unroll
                     for (int j = 0; j < 8; ++j) x[j] = r[q][R * j + e];
                     u32x4 h, m, l;
-                    if constexpr (!SCALED) track_max(mx, x);
+                    if constexpr (!SCALED) track_max(mx[q * R + e], x);
                     split8<SCALED>(x, h, m, l);
                     const int row = MODE == SM_OC ? 2 * (i & 7) + e : i, blk = MODE == SM_OC ? 2 * u + (i >> 3) : u;
                     u32x4 *d = lds + blk * 64 + slot_of(row, g);
@@ -241,6 +252,27 @@ struct SplitLoader {
                     d[NB * 64] = m;
                     d[2 * NB * 64] = l;
                 }
+            }
+        }
+    }
+
+    // over all slabs a wave has moved: one value for all its lanes' rows, and each row's into out[row]
+    __device__ __forceinline__ static float largest(const max_t &mx)
+    {
+        float v = 0.f;
+#pragma unroll
+        for (int q = 0; q < UPW * R; ++q) v = fmaxf(v, mx[q]);
+        return v;
+    }
+    __device__ __forceinline__ static void store_max(const max_t &mx, float *out, int w, int lane)
+    {
+#pragma unroll
+        for (int q = 0; q < UPW; ++q) {
+            if (!mine(w, q)) continue;
+#pragma unroll
+            for (int e = 0; e < R; ++e) {
+                const float v = max_over_g(mx[q * R + e]);
+                if (lane < 16) out[(w + q * NW) * OW + R * lane + e] = v;
             }
         }
     }
@@ -330,6 +362,47 @@ __device__ __forceinline__ bool tiny_operand(const SplitArgs &p, const float *A,
             lb.load_tail(rb, k0, wb, lane);
         }
         tiny |= LA::has_tiny(ra, wa) || LB::has_tiny(rb, wb);
+    }
+    return tiny;
+}
+
+// The same for the rows and columns of a wave's sums below `bound` alone, if there are at most eight
+// (`many`: there are more); blocks of 16 rows from m on and 16 columns from n on.  Sums of ordinary
+// numbers cancel to zero now and then (one of 10^8 at K = 4096), and one tile looked over as a whole is
+// 95 us of a 4096^3 product's 667 (its row and column 30).  Sums of a row or column of zeros (rm, cm:
+// the largest magnitudes) are zero rightly: 4096^3 with a zero row in every tile 890 us when those were
+// looked over, 667 without.
+template <typename LA, typename LB, int NBI, int NBJ, typename RM, typename CM>
+__device__ __forceinline__ bool tiny_lines(const SplitArgs &p, const float *A, const float *B, int m, int n, int first, int step,
+                                           int lane, const floatx4 (&acc)[NBI][NBJ], RM rm, CM cm, float bound, bool &many)
+{
+    asm volatile("" : "+v"(lane));  // (as above)
+    static_assert(NBI * NBJ <= 16, "a bit per sum");
+    uint64_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < NBI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (fabsf(acc[i][j][r]) < bound && rm(i, r) > 0.f && cm(j) > 0.f) bits |= 1ull << (4 * (i * NBJ + j) + r);
+    many = wave_sum((float)__popcll(bits)) > 8.f;
+    if (many) return false;
+    bool tiny = false;
+    for (uint64_t lanes = __builtin_amdgcn_ballot_w64(bits != 0); lanes; lanes = __builtin_amdgcn_ballot_w64(bits != 0)) {
+        const int l = __builtin_ctzll(lanes);
+        const uint64_t b = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(bits >> 32), l) << 32 |
+                           (unsigned)__builtin_amdgcn_readlane((int)bits, l);
+        const int at = __builtin_ctzll(b), blk = at / 4;
+        const int row = min(m + 16 * (blk / NBJ) + 4 * (l >> 4) + at % 4, p.M - 1), col = min(n + 16 * (blk % NBJ) + (l & 15), p.N - 1);
+        if (lane == l) bits &= bits - 1;
+#pragma unroll 8
+        for (int k0 = first * 32; k0 < p.K; k0 += step * 32) {  // a slab of the row in lanes 0..31, of the column above
+            const int k = k0 + (lane & 31);
+            const float v = lane < 32 ? LA::element(A, p.fz.A2, p.as0, p.as1, row, k, p.M, p.K)
+                                      : LB::element(B, nullptr, p.bs1, p.bs0, col, k, p.N, p.K);
+            tiny |= 2 * __float_as_uint(v) - 1 < 2 * __float_as_uint(0x1p-110f) - 1;
+        }
     }
     return tiny;
 }
@@ -431,7 +504,7 @@ __device__ __forceinline__ void split_epilogue(const SplitArgs &p, float *C, con
 // matrix cores (127 TFLOP/s), 690 us here (199 TFLOP/s of fp32 products, 1.2 PFLOP/s of bf16
 // ones, the rate a plain bf16 product of this size reaches).  A slab takes about 6400 cycles: the
 // waves leave its barrier together, and their phases add up rather than overlap (matrix cores busy
-// 0.49).
+// 0.48).
 //
 // SUMS (where tiles compete with waves that split K): a slab's six products add up by themselves,
 // then to the sum, so a slab rounds the long sum once and not six times: the error is that of four
@@ -513,7 +586,8 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
         }
     };
 
-    float mx = 0.f;  // largest magnitude this thread has staged
+    typename LA::max_t mxa = {};
+    typename LB::max_t mxb = {};
     typename LA::regs_t ra;
     typename LB::regs_t rb;
     auto fetch = [&](int k0) {
@@ -527,8 +601,8 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
     // 8.4 us with it, 7.7 without; 1024^2 x 768 20.8 and 22.7).
     auto step = [&](int s, bool more) {
         u32x4 *sa = lds + (s & 1) * (SA + SB);
-        la.store(ra, sa, w, lane, mx);
-        lb.store(rb, sa + SA, wb, lane, mx);
+        la.store(ra, sa, w, lane, mxa);
+        lb.store(rb, sa + SA, wb, lane, mxb);
         if (more && (FORM != SUMS_FEW || s + 1 < nk)) fetch(min(s + 1, nk - 1) * 32);
         __syncthreads();
         compute(sa);
@@ -543,7 +617,7 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
 
     // a sum outside the split's range anywhere in the tile: compute the tile again in fp32
     __shared__ float smax[NW];
-    mx = wave_max(mx);
+    const float mx = wave_max(fmaxf(LA::largest(mxa), LB::largest(mxb)));
     if (lane == 0) smax[w] = mx;
     __syncthreads();
     float largest = smax[0];
@@ -558,7 +632,17 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_kernel(const SplitArgs 
     float unscale = AM == SM_PKB ? SPLIT_UNSCALE : 1.f;
     if (__syncthreads_or(need)) {
         bool redo = need == SplitRange::REDO;
-        if (!__syncthreads_or(redo)) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, 0, 1, w, wb, lane);
+        float *lines = (float *)lds;  // (every wave has read its last operands)
+        LA::store_max(mxa, lines, w, lane);
+        LB::store_max(mxb, lines + TM, wb, lane);
+        if (!__syncthreads_or(redo)) {
+            bool many;
+            auto rm = [&](int i, int r) { return lines[(wm * NBI + i) * 16 + 4 * g + r]; };
+            auto cm = [&](int j) { return lines[TM + (wn * NBJ + j) * 16 + r16]; };
+            redo = tiny_lines<LA, LB>(p, A, B, m0 + wm * NBI * 16, n0 + wn * NBJ * 16, 0, 1, lane, acc, rm, cm,
+                                      SplitRange::bound(largest, K), many);
+            if (__syncthreads_or(many)) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, 0, 1, w, wb, lane);
+        }
         if (__syncthreads_or(redo)) {
             unscale = 1.f;
 #pragma unroll
@@ -744,7 +828,8 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
             red[w][i * NBJ + j][lane] = acc[i][j];
             range.add(acc[i][j]);
         }
-    const int mine = range.check(0x1p124f, wave_max(mx), K);
+    mx = wave_max(mx);
+    const int mine = range.check(0x1p124f, mx, K);
     const bool redo_w = __builtin_amdgcn_ballot_w64(mine == SplitRange::REDO), look_w = __builtin_amdgcn_ballot_w64(mine);
     if (lane == 0) need[w] = redo_w ? SplitRange::REDO : look_w ? SplitRange::LOOK : SplitRange::OK;
     __syncthreads();
@@ -754,7 +839,13 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_split_k_kernel(const SplitArg
     float unscale = AM == SM_PKB ? SPLIT_UNSCALE : 1.f;
     if (any) {
         bool redo = any & SplitRange::REDO;
-        if (!redo) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, w, NW, 0, 0, lane);
+        if (!redo && need[w]) {
+            bool many;
+            // (the magnitude of each row and column would cost the loop registers, and a wave per SIMD)
+            auto unknown = [](auto...) { return 1.f; };
+            redo = tiny_lines<LA, LB>(p, A, B, m0, n0, w, NW, lane, acc, unknown, unknown, SplitRange::bound(mx, K), many);
+            if (many) redo = tiny_operand<LA, LB>(p, A, B, m0, n0, w, NW, 0, 0, lane);
+        }
         if (__syncthreads_or(redo)) {  // (red is read after the barrier below)
             unscale = 1.f;
 #pragma unroll
@@ -841,7 +932,7 @@ static bool launch_unpacked(const SplitArgs &p, long t64, long t32, int batch, h
     } else if constexpr (AM == SM_GEN || BM == SM_GEN) {
         if constexpr (AM == SM_OC || BM == SM_OC)
             if (t64 > 192 && t64 <= 512 && K >= 512) {
-                launch_wave_split<AM, BM, 4, 2, 4, 0>(p, batch, s);
+                launch_wave_split<AM, BM, 4, 2, 4, 2>(p, batch, s);
                 return true;
             }
         if (t64 > 512) launch_tile<AM, BM, 128, 64, 4, 2, SUMS>(p, batch, s);

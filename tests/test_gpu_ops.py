@@ -589,6 +589,25 @@ def test_gemm_split_subnormal(jas, M, N, K):
     assert np.all(np.abs(got[fin] - want[fin]) <= bound), float(np.nanmax(np.abs(got[fin] - want[fin]) / bound))
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 2048, 64), (2050, 2100, 1056), (1030, 1900, 96), (1000, 1000, 100),
+                                   (96, 64, 640), (200, 90, 120)])
+def test_gemm_split_one_lost_sum(jas, M, N, K):
+    """A single product below the split's range in a tile of ordinary sums: column n is zero but for
+    one element of 2^100, which row m alone meets with a number that has no bf16 part.  Rows and
+    columns of zeros, whose sums are zero rightly, beside it."""
+    A, B = normal((M, K), 38, 0), normal((K, N), 38, 1)
+    m, n, k = M - 3, N // 2 + 1, K - 2
+    A[::16], B[:, ::24] = 0, 0
+    B[:, n], B[k, n], A[m, k] = 0, np.float32(2.0 ** 100), np.float32(1.25 * 2.0 ** -136)
+    dA, dB, dC = jas.to_device(A), jas.to_device(B), jas.DeviceArray((M, N))
+    jas.check(jas.lib.jas_gemm(M, N, K, dA.p, K, 1, dB.p, N, 1, dC.p, N, 1, None, 0, 0, 0, 1, 0, 0, 0, 0, None))
+    got = dC.numpy()
+    assert got[m, n] == np.float32(A[m, k]) * np.float32(B[k, n])
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))  # as above
+    assert np.all(np.abs(got - want) <= bound)
+
+
 def test_gemm_dma_k_tail_padded_rows(jas):
     """K not a multiple of 4 with padded, K-contiguous rows: the tail slab reads element by
     element and zero-fills past K."""
