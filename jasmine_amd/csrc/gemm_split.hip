@@ -985,7 +985,8 @@ static bool launch_unpacked(const SplitArgs &p, long t64, long t32, int batch, h
     }
 }
 
-// Geometry by the number of tiles (256 CUs) and K; MI355X, us per product (M x N x K):
+// Geometry by the number of tiles (256 CUs) and K, for packed weights and what launch_unpacked leaves;
+// MI355X, us per product (M x N x K):
 //   256 x 128 tiles when their rounds over the CUs are at least four fifths full: 12288 x 2048
 //     x 4096 1075 (128 x 64: 1320, 64 x 64: 1250); but 2304 x 4096 x 768, 288 tiles, 166 (123)
 //   128 x 64 for a long K with two tiles per CU: 2048^3 109 (64 x 64: 153, 256 x 128: 175)
